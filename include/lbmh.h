@@ -396,12 +396,15 @@ int lbmh_device_synchronize(int device);
  * fewer waves in flight keep fewer DRAM rows open for the 2*Q concurrent
  * population streams.  xcd_group G > 0 hands each XCD runs of G consecutive
  * 256-cell chunks inside a window of 8*G chunks, so a cache line two chunks
- * share is fetched into one L2 instead of two.  Defaults: lds_bytes 40960
- * (4 workgroups per CU) and xcd_group 4 for FP32 storage, lds_bytes 49152
- * and xcd_group 8 for FP64, lds_bytes 0 and xcd_group 8 for FP16 storage;
- * FP64/FP32 lattices with local velocity /
- * pressure boundaries switch to lds_bytes 0 (their whole-lattice pass also
- * collides the flat faces, whose divergent waves need the occupancy).  A
+ * share is fetched into one L2 instead of two.  Successive steps go through
+ * the chunks in opposite directions, each chunk on the same XCD.  Defaults
+ * follow the storage type and the size of the block: blocks up to 64 MB of
+ * populations lds_bytes 0 and one eighth of the chunks per XCD (up to 64),
+ * larger ones lds_bytes 40960 and xcd_group 32 (4 above 512 MB) in FP32,
+ * 49152 and 16 in FP64, 0 and 32 in FP16; lattices with local velocity /
+ * pressure boundaries take lds_bytes 0 and xcd_group 4 (FP16: 8), as their
+ * whole-lattice pass also collides the flat faces, whose divergent waves need
+ * the occupancy.  A
  * shape set here or chosen by lbmh_autotune is kept. */
 typedef struct lbmh_launch_config {
   int lds_bytes;    /* 0 .. 65536                                             */

@@ -65,6 +65,7 @@ __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args
   a.div_y = e.div_y;
   a.periodic = e.periodic;
   a.xcd_group = 0;
+  a.reverse = 0;
   a.walls = walls + uint64_t(lat) * kEnsembleWalls * 4;
   a.info = info ? info + uint64_t(lat) * kEnsembleWalls : nullptr;
   a.force = nullptr;  // members take the uniform force
@@ -101,8 +102,7 @@ __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEnt
                                                                const uint32_t* __restrict__ info, uint32_t xcd_group,
                                                                EnsembleLimits limits)
 {
-  uint32_t b = blockIdx.x;
-  if (xcd_group) b = remap_xcd(b, gridDim.x, xcd_group);
+  const uint32_t b = chunk_of_block(blockIdx.x, gridDim.x, xcd_group, 0);
   const uint32_t lat = chunk_lattice[b];
   if (lat >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lat];

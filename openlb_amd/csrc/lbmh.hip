@@ -75,6 +75,7 @@ struct lbmh_lattice {
   uint64_t stride = 0;
   uint32_t ncore = 0;
   int64_t steps = 0;
+  uint32_t passes = 0;         // whole-block passes so far: odd ones run from the block's end to its start
   int64_t shift[27] = {};
   int64_t dist[27] = {};
   void* d_pop = nullptr;
@@ -132,19 +133,36 @@ struct lbmh_lattice {
   size_t remote_batch_bytes = 0;
 };
 
-// Library default launch shape, from sweeps of (LDS reservation, XCD group)
-// on the porous channel, the turbulent channel and a Taylor-Green box.  FP32:
-// a 40 KB LDS reservation caps the resident workgroups at 4 per CU (fewer
-// concurrent DRAM streams), XCD groups of 4.  FP64: 48 KB (3 per CU), groups
-// of 8, 1-2% ahead of the FP32 shape.  FP16: no cap, groups of 8.  With
-// local boundaries the whole-lattice pass collides the flat faces too, and
+// Library default launch shape of a block, from sweeps of (LDS reservation,
+// XCD group) on porous channels, turbulent channels, cavities and Taylor-Green
+// boxes of 1 MB to 3 GB of populations.
+// Up to 64 MB the lines stay in the caches from step to step: each XCD takes one
+// contiguous eighth of the chunks, so that its L2 holds the lines it used in the
+// last step (FP32 D3Q27 48^3: group 8 9.5 us, 54 7.4 us), as far as the group
+// limit of 64 allows, and a cap on the resident workgroups only costs latency
+// (FP32 D3Q19 67x83x91 with 40 KB of LDS 14.8 us, without 14.2 us).
+// Beyond that: FP32 a 40 KB reservation, 4 workgroups per CU (fewer concurrent
+// DRAM streams: 256^3 470 us against 488 us uncapped), FP64 48 KB (3 per CU),
+// FP16 no cap (D3Q27 384x192x192 341 us against 380 us).  Wide XCD groups keep the
+// lines that neighbouring chunks share in one L2 (FP64 D3Q27 384x192x192, group 8
+// -> 16: 1285 -> 1189 us; FP16 the same block, 8 -> 32: 346 -> 341 us; FP32
+// 128^3, 4 -> 32: 54.3 -> 52.8 us); an FP32 block above 512 MB is faster with
+// groups of 4 (256^3 466 us against 470 us).
+// With local boundaries the whole-lattice pass collides the flat faces too, and
 // its divergent waves need the occupancy: no cap (201^3 cavity, FP32: 298 us
 // against 324 us).
-static lbmh_launch_config default_launch(int storage, bool local)
+static lbmh_launch_config default_launch(const lbmh_lattice* L, bool local)
 {
-  if (storage == LBMH_F16) return lbmh_launch_config{0, 8};
-  if (local) return lbmh_launch_config{0, 4};
-  return storage == LBMH_F64 ? lbmh_launch_config{49152, 8} : lbmh_launch_config{40960, 4};
+  constexpr uint64_t kMB = 1000000;
+  const uint64_t bytes = L->stride * uint64_t(L->q) * storage_size(L->storage);
+  if (local) return lbmh_launch_config{0, L->storage == LBMH_F16 ? 8 : 4};
+  if (bytes < 64 * kMB) {
+    const uint32_t eighth = L->ncore / (8 * kBlock);
+    return lbmh_launch_config{0, int(std::min(std::max(eighth, 1u), 64u))};
+  }
+  if (L->storage == LBMH_F16) return lbmh_launch_config{0, 32};
+  if (L->storage == LBMH_F64) return lbmh_launch_config{49152, 16};
+  return lbmh_launch_config{40960, bytes < 512 * kMB ? 32 : 4};
 }
 
 struct lbmh_halo {
@@ -566,6 +584,7 @@ StepArgs<Q, V> step_args(const lbmh_lattice* L)
   a.div_y = FastDiv(uint32_t(L->n[1]));
   a.periodic = uint32_t(L->periodic[0] | (L->periodic[1] << 1) | (L->periodic[2] << 2));
   a.xcd_group = uint32_t(L->launch.xcd_group);
+  a.reverse = L->passes & 1u;
   a.walls = L->d_walls;
   a.info = L->d_info;
   a.force = static_cast<const V*>(L->d_force);
@@ -609,6 +628,7 @@ int launch_kind(lbmh_lattice* L, hipStream_t stream, int phase)
     hipLaunchKernelGGL((collide_stream_kernel<Q, S, KIND, true>), dim3(grid), dim3(kBlock), lds, stream, a);
   }
   LBMH_HIP(hipGetLastError());
+  L->passes += 1;
   }
   if (!(phase & kPhaseStream)) return LBMH_OK;
   advance_shifts(L);
@@ -725,9 +745,7 @@ int lbmh_lattice_create(const lbmh_lattice_desc* desc, lbmh_lattice** out)
                             : neighbor_distance<27>(i, int64_t(sy * sz), int64_t(sz));
   }
   L->params.omega = 1.0;
-  // measured best shapes on MI355X for the 256^3 D3Q19 step: FP16 columns
-  // want full occupancy, FP32/FP64 three to four workgroups per CU
-  L->launch = default_launch(L->storage, false);
+  L->launch = default_launch(L, false);
   for (int w = 0; w < kMaxWalls; ++w) {
     L->walls[w][0] = 1.0;
     L->material_of[w] = uint8_t(w);
@@ -801,7 +819,7 @@ int lbmh_set_dynamics_ids(lbmh_lattice* L, const uint8_t* ids)
   // a new id map drops the local boundaries defined on the previous one
   L->h_ids.assign(ids, ids + L->ncore);
   L->has_local = false;
-  if (!L->launch_chosen) L->launch = default_launch(L->storage, false);
+  if (!L->launch_chosen) L->launch = default_launch(L, false);
   L->h_edges.clear();
   L->h_corners.clear();
   L->h_local.clear();
@@ -1047,7 +1065,7 @@ int lbmh_set_local_boundary(lbmh_lattice* L, int id, int kind, double rho, const
   if (rc != LBMH_OK) return rc;
   L->has_local = true;
   L->uniform_bulk = false;
-  if (!L->launch_chosen) L->launch = default_launch(L->storage, true);
+  if (!L->launch_chosen) L->launch = default_launch(L, true);
   return LBMH_OK;
 }
 
@@ -1301,6 +1319,7 @@ int lbmh_pattern_ceiling(lbmh_lattice* L, int64_t n_steps, void* stream)
       return LBMH_OK;
     });
     if (rc != LBMH_OK) return rc;
+    L->passes += 1;
     advance_shifts(L);
     L->steps += 1;
   }

@@ -350,6 +350,32 @@ def test_local_boundary_lattices_default_to_full_occupancy(gpu_available):
     np.testing.assert_array_equal(runs[0], runs[1])
 
 
+@pytest.mark.parametrize("shape,periodic_walls", [((1, 1, 1), False), ((8, 16, 16), True), ((7, 37, 64), False),
+                                                  ((9, 32, 65), True), ((13, 41, 33), False)])
+def test_alternating_passes_match_the_oracle(gpu_available, shape, periodic_walls):
+    """Successive passes run through the chunks in opposite directions, on
+    whole windows of 8 XCDs x group chunks, with the rest in dispatch order:
+    one cell, exactly one window, windows and a rest, for groups around an
+    eighth of the chunks and the default.  Every population after an odd and an
+    even number of steps, FP64, to the step's bound of 1e-14 per 7 steps."""
+    case = W.couette_channel(shape) if periodic_walls else W.random_periodic(shape, seed=5)
+    f0 = O.initial_populations(case, "f64")
+    ref = O.OracleLattice(case, "f64")
+    ref.upload(f0)
+    ref.step(7, threads=4)
+    fluid = case.ids == 1
+    eighth = max(1, case.ids.size // 2048)
+    for group in (None, 1, eighth, eighth + 1):
+        with BlockLattice.from_case(case, "f64") as lat:
+            lat.upload_populations(f0, "f64")
+            if group is not None:
+                lat.set_launch_config(0, group)
+            lat.collide_and_stream(3)
+            lat.collide_and_stream(4)
+            got = lat.download_populations("f64")
+        assert np.abs(got[:, fluid] - ref.download()[:, fluid]).max() <= 1e-14
+
+
 def test_launch_configs_give_identical_results(gpu_available):
     """Launch shape is scheduling only: every configuration must give bit-identical
     populations. The autotuner must leave the lattice's own state untouched."""
