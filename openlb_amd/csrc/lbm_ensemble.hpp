@@ -5,10 +5,16 @@
 // The launch covers the concatenated 256-cell chunks of every active lattice.
 // A chunk finds its lattice through `chunk_lattice` and reads that lattice's
 // entry from the table with uniform (scalar) loads, then runs exactly the
-// cell body of the single-block kernel.  The shifts and step counters live in
-// the table and are advanced on the device by a one-thread-per-lattice kernel,
-// so a sequence of steps needs no host involvement and can be captured in a
-// HIP graph.
+// cell body of the single-block kernel.  The shifts and step counters live on
+// the device in two copies: a step reads one and the first workgroup of each
+// lattice writes the other, advanced by one step, so a sequence of steps needs
+// no host involvement, can be captured in a HIP graph, and takes one launch per
+// step.  A call starts and ends on the first copy (an odd number of steps is
+// followed by a copy), so that a call a program captures can be replayed.
+// (An advance kernel of its own, one thread per lattice, took 5-9 us
+// per step behind the step kernel: 96 FP16 cavities 148 + 8.9 us, the solve
+// server's two ensembles 26 + 16 + 2 x 5.2 us.)  The copy a step reads also
+// gives the pass its direction (chunk_of_block).
 #pragma once
 
 #include "lbm_kernels.hpp"
@@ -26,13 +32,18 @@ struct EnsembleEntry {
   FastDiv div_z, div_y;
   uint32_t periodic;
   uint32_t chunk_begin;     // first chunk of this lattice in the launch
+  BulkParams<double> bp;
+  uint32_t dmod[Q];         // (c_i . projection) mod n_padded
+};
+
+// What a step changes of a lattice besides its populations.
+template <int Q>
+struct MemberState {
   int64_t steps_left;       // 0: idle, < 0: unbounded
   int64_t steps_done;
-  uint32_t stepped;         // 1 if the last advance moved this lattice (its post-processors run)
+  uint32_t stepped;         // 1 if the last step moved this lattice (its post-processors run)
   uint32_t pad_;
-  BulkParams<double> bp;
   uint32_t shift[Q];        // PS shifts, in [0, n_padded)
-  uint32_t dmod[Q];         // (c_i . projection) mod n_padded
 };
 
 // Sizes of the arenas, so that a workgroup can refuse an entry that does not fit.
@@ -45,7 +56,7 @@ struct EnsembleLimits {
 // Whole-member arguments of the single-block cell body, from a table entry.
 template <int Q, typename S>
 __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args(
-    const EnsembleEntry<Q>& e, uint32_t lat, S* arena, const uint8_t* ids, const double* walls, const uint32_t* info)
+    const EnsembleEntry<Q>& e, const MemberState<Q>& st, uint32_t lat, S* arena, const uint8_t* ids, const double* walls, const uint32_t* info)
 {
   using V = typename StorageTraits<S>::V;
   StepArgs<Q, V> a;
@@ -53,7 +64,7 @@ __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args
   a.stride = e.stride;
   a.n_padded = e.n_padded;
 #pragma unroll
-  for (int i = 0; i < Q; ++i) a.shift[i] = e.shift[i];
+  for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
   a.ids = ids + e.ids_offset;
   a.ncore = e.ncore;
   a.nx = e.nx;
@@ -92,23 +103,53 @@ __device__ __forceinline__ bool entry_fits(const EnsembleEntry<Q>& e, const Ense
            e.ids_offset + e.ncore > limits.id_bytes);
 }
 
+// Streaming of a lattice, by the threads of its first workgroup: rotate its
+// columns and count the step if it stepped, into the copy the next step reads.
+template <int Q>
+__device__ __forceinline__ void advance_member(const EnsembleEntry<Q>& e, const MemberState<Q>& st, MemberState<Q>& next)
+{
+  const uint32_t i = threadIdx.x;
+  const bool step = st.steps_left != 0;
+  if (i < uint32_t(Q)) {
+    const uint32_t s = st.shift[i], d = e.dmod[i];
+    next.shift[i] = !step ? s : (s >= d ? s - d : s + (e.n_padded - d));
+  }
+  if (i == 0) {
+    next.stepped = step ? 1u : 0u;
+    next.steps_left = st.steps_left > 0 ? st.steps_left - 1 : st.steps_left;
+    next.steps_done = st.steps_done + (step ? 1 : 0);
+  }
+}
+
+// The states of all members from one copy to the other, `words` 32-bit words.
+static __global__ __launch_bounds__(kBlock) void ensemble_settle_kernel(uint32_t* __restrict__ to,
+                                                                        const uint32_t* __restrict__ from, uint32_t words)
+{
+  const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+  if (k < words) to[k] = from[k];
+}
+
 // LOCAL = kLocalSkip when some member has local boundaries: their cells are
 // left to ensemble_local_kernel.
 template <int Q, typename S, int KIND, int LOCAL = kLocalNone>
 __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEntry<Q>* __restrict__ table,
+                                                               const MemberState<Q>* __restrict__ state,
+                                                               MemberState<Q>* __restrict__ next, uint32_t reverse,
                                                                const uint32_t* __restrict__ chunk_lattice,
                                                                S* __restrict__ arena, const uint8_t* __restrict__ ids,
                                                                const double* __restrict__ walls,
                                                                const uint32_t* __restrict__ info, uint32_t xcd_group,
                                                                EnsembleLimits limits)
 {
-  const uint32_t b = chunk_of_block(blockIdx.x, gridDim.x, xcd_group, 0);
+  const uint32_t b = chunk_of_block(blockIdx.x, gridDim.x, xcd_group, reverse);
   const uint32_t lat = chunk_lattice[b];
   if (lat >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lat];
-  if (e.steps_left == 0) return;
+  const MemberState<Q>& st = state[lat];
+  if (b == e.chunk_begin) advance_member(e, st, next[lat]);
+  if (st.steps_left == 0) return;
   if (!entry_fits(e, limits)) return;
-  const auto a = member_args<Q, S>(e, lat, arena, ids, walls, LOCAL == kLocalNone ? nullptr : info);
+  const auto a = member_args<Q, S>(e, st, lat, arena, ids, walls, LOCAL == kLocalNone ? nullptr : info);
   collide_stream_cell<Q, S, KIND, true, LOCAL>(a, (b - e.chunk_begin) * kBlock + threadIdx.x);
 }
 
@@ -116,6 +157,7 @@ __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEnt
 // (member, core cell) pairs.
 template <int Q, typename S, int KIND>
 __global__ __launch_bounds__(64) void ensemble_local_kernel(const EnsembleEntry<Q>* __restrict__ table,
+                                                            const MemberState<Q>* __restrict__ state,
                                                             const uint2* __restrict__ cells, uint32_t count,
                                                             S* __restrict__ arena, const uint8_t* __restrict__ ids,
                                                             const double* __restrict__ walls,
@@ -126,8 +168,9 @@ __global__ __launch_bounds__(64) void ensemble_local_kernel(const EnsembleEntry<
   const uint2 lc = cells[k];
   if (lc.x >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lc.x];
-  if (e.steps_left == 0 || !entry_fits(e, limits) || lc.y >= e.ncore) return;
-  const auto a = member_args<Q, S>(e, lc.x, arena, ids, walls, info);
+  const MemberState<Q>& st = state[lc.x];
+  if (st.steps_left == 0 || !entry_fits(e, limits) || lc.y >= e.ncore) return;
+  const auto a = member_args<Q, S>(e, st, lc.x, arena, ids, walls, info);
   collide_stream_cell<Q, S, KIND, true, kLocalCollide>(a, lc.y);
 }
 
@@ -142,6 +185,7 @@ __global__ __launch_bounds__(64) void ensemble_local_kernel(const EnsembleEntry<
 // compiles the reconstruction exactly as the lattice does.
 template <int Q, typename S, int KIND, bool SCRATCH = false>
 __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q>* __restrict__ table,
+                                                           const MemberState<Q>* __restrict__ state,
                                                            const uint2* __restrict__ cells, uint32_t count,
                                                            S* __restrict__ arena, const uint8_t* __restrict__ ids,
                                                            const double* __restrict__ walls,
@@ -162,13 +206,14 @@ __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q
   }
   if (valid) {
     const EnsembleEntry<Q>& e = table[lc.x];
-    valid = (only >= 0 ? int(lc.x) == only : e.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore;
+    const MemberState<Q>& st = state[lc.x];
+    valid = (only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore;
     if (valid) {
       a.pop = arena + e.pop_offset;
       a.stride = e.stride;
       a.n_padded = e.n_padded;
 #pragma unroll
-      for (int i = 0; i < Q; ++i) a.shift[i] = e.shift[i];
+      for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
       a.ids = ids + e.ids_offset;
       a.walls = walls + uint64_t(lc.x) * kEnsembleWalls * 4;
       a.info = info + uint64_t(lc.x) * kEnsembleWalls;
@@ -206,6 +251,7 @@ __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q
 // Second half of a two-phase plane pass: entry k's populations from scratch.
 template <int Q, typename S>
 __global__ __launch_bounds__(64) void ensemble_plane_store_kernel(const EnsembleEntry<Q>* __restrict__ table,
+                                                                  const MemberState<Q>* __restrict__ state,
                                                                   const uint2* __restrict__ cells, uint32_t count,
                                                                   S* __restrict__ arena,
                                                                   const typename StorageTraits<S>::V* scratch,
@@ -217,33 +263,16 @@ __global__ __launch_bounds__(64) void ensemble_plane_store_kernel(const Ensemble
   const uint2 lc = cells[k];
   if (lc.x >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lc.x];
-  if (!((only >= 0 ? int(lc.x) == only : e.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore)) return;
+  const MemberState<Q>& st = state[lc.x];
+  if (!((only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore)) return;
   int x, y, z;
   core_coords(e.div_z, e.div_y, int(e.ny), int(e.nz), lc.y, x, y, z);
   const uint32_t n = uint32_t(x + 1) * e.sx + uint32_t(y + 1) * e.sy + uint32_t(z + 1);
   S* pop = arena + e.pop_offset;
 #pragma unroll
   for (int i = 0; i < Q; ++i)
-    store_pop<S, V>(column_at(pop + uint64_t(i) * e.stride, wrap_index(n, e.shift[i], e.n_padded)),
+    store_pop<S, V>(column_at(pop + uint64_t(i) * e.stride, wrap_index(n, st.shift[i], e.n_padded)),
                     scratch[uint64_t(k) * Q + i]);
-}
-
-// Streaming of every lattice that stepped: rotate its columns, count the step.
-// One thread owns one lattice, so the read of steps_left and its update cannot race.
-template <int Q>
-__global__ void ensemble_advance_kernel(EnsembleEntry<Q>* table, uint32_t nslots)
-{
-  const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
-  if (l >= nslots) return;
-  EnsembleEntry<Q>& e = table[l];
-  e.stepped = e.steps_left != 0 ? 1u : 0u;
-  if (e.steps_left == 0) return;
-  for (int i = 0; i < Q; ++i) {
-    const uint32_t s = e.shift[i], d = e.dmod[i];
-    e.shift[i] = s >= d ? s - d : s + (e.n_padded - d);
-  }
-  if (e.steps_left > 0) e.steps_left -= 1;
-  e.steps_done += 1;
 }
 
 }  // namespace lbmh

@@ -109,8 +109,14 @@ struct lbmh_ensemble {
   Arena pop_arena, id_arena;
   std::vector<Member> members;
   std::vector<unsigned char> h_table;   // host mirror of the member table
-  lbmh_launch_config launch{0, 4};
-  bool launch_chosen = false;     // set by lbmh_ensemble_set_launch_config: keep it
+  // steps left and done and PS shifts of every member: two copies of
+  // max_members records on the device, the first current between calls (each
+  // step reads one and writes the other), and a host mirror of it
+  void* d_state = nullptr;
+  size_t state_bytes = 0;               // one record
+  std::vector<unsigned char> h_state;
+  lbmh_launch_config launch{0, 4};  // used once launch_chosen, else step_launch()
+  bool launch_chosen = false;     // set by lbmh_ensemble_set_launch_config / _autotune: keep it
   uint64_t version = 1;
   hipStream_t capture_stream = nullptr;
   hipGraphExec_t graph = nullptr;
@@ -139,6 +145,18 @@ EnsembleEntry<Q>& entry(lbmh_ensemble* E, int m)
   return *reinterpret_cast<EnsembleEntry<Q>*>(E->h_table.data() + size_t(m) * E->entry_bytes);
 }
 
+template <int Q>
+MemberState<Q>& state(lbmh_ensemble* E, int m)
+{
+  return *reinterpret_cast<MemberState<Q>*>(E->h_state.data() + size_t(m) * E->state_bytes);
+}
+
+// The device's copy k of member m's state.
+char* device_state(lbmh_ensemble* E, uint32_t k, int m = 0)
+{
+  return static_cast<char*>(E->d_state) + (size_t(k) * size_t(E->max_members) + size_t(m)) * E->state_bytes;
+}
+
 template <typename F>
 int with_q(const lbmh_ensemble* E, F&& f)
 {
@@ -158,10 +176,11 @@ int with_types(const lbmh_ensemble* E, F&& f)
   return f(std::integral_constant<int, 27>(), _Float16());
 }
 
-int pull_table(lbmh_ensemble* E)
+// The members' states as the device holds them; the table only changes here on the host.
+int pull_state(lbmh_ensemble* E)
 {
   LBMH_HIP(hipDeviceSynchronize());
-  LBMH_HIP(hipMemcpy(E->h_table.data(), E->d_table, E->h_table.size(), hipMemcpyDeviceToHost));
+  LBMH_HIP(hipMemcpy(E->h_state.data(), device_state(E, 0), E->h_state.size(), hipMemcpyDeviceToHost));
   return LBMH_OK;
 }
 
@@ -176,7 +195,7 @@ int push_table(lbmh_ensemble* E)
       EnsembleEntry<Q>& e = entry<Q>(E, m);
       if (!E->members[m].active) {
         e.chunk_begin = 0;
-        e.steps_left = 0;
+        std::memset(&state<Q>(E, m), 0, sizeof(MemberState<Q>));
         continue;
       }
       e.chunk_begin = uint32_t(map.size());
@@ -189,6 +208,9 @@ int push_table(lbmh_ensemble* E)
   if (map.size() > E->chunk_capacity) return fail(LBMH_E_MEMORY, "chunk map capacity exceeded");
   E->total_chunks = uint32_t(map.size());
   LBMH_HIP(hipMemcpy(E->d_table, E->h_table.data(), E->h_table.size(), hipMemcpyHostToDevice));
+  // both copies: a slot without a member has no workgroup to carry its state over
+  for (uint32_t k = 0; k < 2; ++k)
+    LBMH_HIP(hipMemcpy(device_state(E, k), E->h_state.data(), E->h_state.size(), hipMemcpyHostToDevice));
   if (!map.empty()) LBMH_HIP(hipMemcpy(E->d_chunk, map.data(), map.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
   E->version += 1;
   return LBMH_OK;
@@ -246,23 +268,23 @@ CoreGeom geom_of(const EnsembleEntry<Q>& e)
 }
 
 template <int Q>
-Shifts<Q> shifts_of(const EnsembleEntry<Q>& e)
+Shifts<Q> shifts_of(const MemberState<Q>& st)
 {
   Shifts<Q> s;
-  for (int i = 0; i < Q; ++i) s.s[i] = e.shift[i];
+  for (int i = 0; i < Q; ++i) s.s[i] = st.shift[i];
   return s;
 }
 
 // PostStream stage of the local boundaries: edges, then corners, of the
 // members that stepped (only < 0) or of member `only`.
 template <int Q, typename S>
-int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, S* arena, const EnsembleLimits& limits,
+int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, const MemberState<Q>* st, S* arena, const EnsembleLimits& limits,
                 hipStream_t stream, int only)
 {
   const int forced = (E->kind == LBMH_FORCED_BGK || E->kind == LBMH_FORCED_TRT) ? 1 : 0;
   if (E->n_planes) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostPlane>), dim3(grid_for(E->n_planes, 64 / kPostLanes)), dim3(64),
-                       0, stream, table, E->d_planes, E->n_planes, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
+                       0, stream, table, st, E->d_planes, E->n_planes, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
                        forced);
     LBMH_HIP(hipGetLastError());
   }
@@ -271,38 +293,52 @@ int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, S* arena, const
     using V = typename StorageTraits<S>::V;
     V* scratch = static_cast<V*>(E->d_plane_scratch);
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostPlane, true>), dim3(grid_for(E->n_pplanes, 64 / kPostLanes)),
-                       dim3(64), 0, stream, table, E->d_pplanes, E->n_pplanes, arena, E->d_ids, E->d_walls, E->d_info,
+                       dim3(64), 0, stream, table, st, E->d_pplanes, E->n_pplanes, arena, E->d_ids, E->d_walls, E->d_info,
                        limits, only, forced, scratch);
     LBMH_HIP(hipGetLastError());
     hipLaunchKernelGGL((ensemble_plane_store_kernel<Q, S>), dim3(grid_for(E->n_pplanes, 64)), dim3(64), 0, stream,
-                       table, E->d_pplanes, E->n_pplanes, arena, static_cast<const V*>(scratch), limits, only);
+                       table, st, E->d_pplanes, E->n_pplanes, arena, static_cast<const V*>(scratch), limits, only);
     LBMH_HIP(hipGetLastError());
   }
   if (E->n_edges) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostEdge>), dim3(grid_for(E->n_edges, 64 / kPostLanes)), dim3(64), 0,
-                       stream, table,
-                       E->d_edges, E->n_edges, arena, E->d_ids, E->d_walls, E->d_info, limits, only, forced);
+                       stream, table, st, E->d_edges, E->n_edges, arena, E->d_ids, E->d_walls, E->d_info, limits, only, forced);
     LBMH_HIP(hipGetLastError());
   }
   if (E->n_corners) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostCorner>), dim3(grid_for(E->n_corners, 64 / kPostLanes)), dim3(64), 0,
-                       stream, table, E->d_corners, E->n_corners, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
+                       stream, table, st, E->d_corners, E->n_corners, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
                        forced);
     LBMH_HIP(hipGetLastError());
   }
   return LBMH_OK;
 }
 
+// Launch shape of a step: the chosen one, else by what the members hold.
+// LDS reservation as for a single block: 40 KB in FP32 and 48 KB in FP64, none
+// in FP16 and while the members fit the caches (up to 64 MB; 12 FP32 cavities,
+// 38 MB, 15.6 us capped, 15.0 us not).  With local-boundary members the step
+// kernel collides their flat faces too, in divergent waves that need more
+// occupancy: 24 KB (FP32, 96 local-velocity cavities 458 us per step against
+// 509 us; velocity-inlet ducts 266 against 269 us).  XCD groups of 32 keep a
+// small member's chunks, and the lines they share, on one XCD (group 8 -> 32:
+// 12 FP16 cavities 11.4 -> 11.2 us, 16 FP32 ducts 60.6 -> 59.7 us, 40 FP64
+// cavities 142.1 -> 140.7 us, 96 FP32 cavities 236 -> 237 us).
+lbmh_launch_config step_launch(const lbmh_ensemble* E)
+{
+  if (E->launch_chosen) return E->launch;
+  lbmh_launch_config c{0, 32};
+  if (E->storage == LBMH_F16) return c;
+  if (E->has_local) c.lds_bytes = 24576;
+  else if (E->pop_arena.used() >= 64000000u) c.lds_bytes = E->storage == LBMH_F64 ? 49152 : 40960;
+  return c;
+}
+
 int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
 {
-  // With local-boundary members the step kernel collides their flat faces
-  // too, in divergent waves that need more occupancy than the FP64/FP32 cap
-  // gives: 24 KB instead (FP32, 96 local-velocity cavities: 458 us per step
-  // against 509 us; velocity-inlet ducts 266 against 269 us).  FP16 has no cap.
-  const bool relax = E->has_local && !E->launch_chosen && E->storage != LBMH_F16;
-  const unsigned lds = relax ? 24576u : unsigned(E->launch.lds_bytes);
-  const uint32_t group = uint32_t(E->launch.xcd_group);
-  const uint32_t adv_grid = grid_for(uint32_t(E->max_members), 256);
+  const lbmh_launch_config launch = step_launch(E);
+  const unsigned lds = unsigned(launch.lds_bytes);
+  const uint32_t group = uint32_t(launch.xcd_group);
   return with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
@@ -312,13 +348,16 @@ int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
                                 uint32_t(E->max_members)};
     const bool local = E->has_local;
     for (int64_t k = 0; k < n; ++k) {
+      const uint32_t cur = uint32_t(k & 1);
+      const auto* st = reinterpret_cast<const MemberState<Q>*>(device_state(E, cur));
+      auto* next = reinterpret_cast<MemberState<Q>*>(device_state(E, cur ^ 1u));
       if (E->total_chunks) {
 #define LBMH_ENSEMBLE_STEP(KIND_)                                                                               \
-  hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_>), dim3(E->total_chunks), dim3(kBlock), lds, stream, table, \
-                     E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
+  hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_>), dim3(E->total_chunks), dim3(kBlock), lds, stream, table, st, \
+                     next, cur, E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
 #define LBMH_ENSEMBLE_STEP_LOCAL(KIND_)                                                                         \
   hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_, kLocalFlat>), dim3(E->total_chunks), dim3(kBlock), lds,    \
-                     stream, table, E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
+                     stream, table, st, next, cur, E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
         if (local) {
           // the boundary cells collide with their BGK mixin whatever the bulk kind
           switch (E->kind) {
@@ -344,7 +383,7 @@ int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
       if (local && E->n_local) {
 #define LBMH_ENSEMBLE_LOCAL(KIND_)                                                                              \
   hipLaunchKernelGGL((ensemble_local_kernel<Q, S, KIND_>), dim3(grid_for(E->n_local, 64)), dim3(64), 0, stream,      \
-                     table, E->d_local, E->n_local, arena, E->d_ids, E->d_walls, E->d_info, limits)
+                     table, st, E->d_local, E->n_local, arena, E->d_ids, E->d_walls, E->d_info, limits)
         switch (E->kind) {
         case LBMH_BGK: LBMH_ENSEMBLE_LOCAL(kBGK); break;
         case LBMH_FORCED_BGK: LBMH_ENSEMBLE_LOCAL(kForcedBGK); break;
@@ -355,11 +394,15 @@ int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
 #undef LBMH_ENSEMBLE_LOCAL
         LBMH_HIP(hipGetLastError());
       }
-      hipLaunchKernelGGL((ensemble_advance_kernel<Q>), dim3(adv_grid), dim3(256), 0, stream, table,
-                         uint32_t(E->max_members));
-      LBMH_HIP(hipGetLastError());
-      const int rc = launch_post(E, table, arena, limits, stream, -1);
+      const int rc = launch_post(E, table, static_cast<const MemberState<Q>*>(next), arena, limits, stream, -1);
       if (rc != LBMH_OK) return rc;
+    }
+    if (n & 1) {
+      const uint32_t words = uint32_t(E->h_state.size() / sizeof(uint32_t));
+      hipLaunchKernelGGL(ensemble_settle_kernel, dim3(grid_for(words, kBlock)), dim3(kBlock), 0, stream,
+                         reinterpret_cast<uint32_t*>(device_state(E, 0)),
+                         reinterpret_cast<const uint32_t*>(device_state(E, 1)), words);
+      LBMH_HIP(hipGetLastError());
     }
     return LBMH_OK;
   });
@@ -389,18 +432,18 @@ int lbmh_ensemble_create(const lbmh_ensemble_desc* d, lbmh_ensemble** out)
   E->entry_bytes = E->q == 19 ? sizeof(EnsembleEntry<19>) : sizeof(EnsembleEntry<27>);
   E->members.resize(size_t(E->max_members));
   E->h_table.assign(E->entry_bytes * size_t(E->max_members), 0);
+  E->state_bytes = E->q == 19 ? sizeof(MemberState<19>) : sizeof(MemberState<27>);
+  E->h_state.assign(E->state_bytes * size_t(E->max_members), 0);
   E->pop_arena = Arena(align_up(d->population_bytes));
   E->id_arena = Arena(align_up(d->cell_capacity) + kAlign * size_t(E->max_members));
   E->chunk_capacity = uint32_t(d->cell_capacity / kBlock + size_t(E->max_members) + 1);
-  // the single-lattice defaults (an ensemble sweep of 256 cavities agrees within 1%)
-  E->launch = d->storage == LBMH_F16   ? lbmh_launch_config{0, 8}
-              : d->storage == LBMH_F64 ? lbmh_launch_config{49152, 8}
-                                       : lbmh_launch_config{40960, 4};
   DeviceGuard guard(E->device);
   hipError_t e = hipMalloc(&E->d_pop, E->pop_arena.capacity());
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_ids, E->id_arena.capacity());
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_walls, sizeof(double) * 4 * kEnsembleWalls * E->max_members);
   if (e == hipSuccess) e = hipMalloc(&E->d_table, E->h_table.size());
+  if (e == hipSuccess) e = hipMalloc(&E->d_state, 2 * E->h_state.size());
+  if (e == hipSuccess) e = hipMemset(E->d_state, 0, 2 * E->h_state.size());
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_chunk, sizeof(uint32_t) * E->chunk_capacity);
   E->boundary_capacity = d->boundary_capacity ? d->boundary_capacity : d->cell_capacity / 4 + 64;
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_info, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
@@ -429,6 +472,7 @@ int lbmh_ensemble_destroy(lbmh_ensemble* E)
   if (E->d_ids) (void)hipFree(E->d_ids);
   if (E->d_walls) (void)hipFree(E->d_walls);
   if (E->d_table) (void)hipFree(E->d_table);
+  if (E->d_state) (void)hipFree(E->d_state);
   if (E->d_chunk) (void)hipFree(E->d_chunk);
   if (E->d_info) (void)hipFree(E->d_info);
   if (E->d_local) (void)hipFree(E->d_local);
@@ -500,7 +544,7 @@ int lbmh_ensemble_add(lbmh_ensemble* E, const int extent[3], const int periodic[
     E->id_arena.release(mem.ids_off, mem.ids_bytes);
     return rc;
   };
-  int rc = pull_table(E);
+  int rc = pull_state(E);
   if (rc != LBMH_OK) return undo(rc);
   hipError_t e = hipMemset(static_cast<char*>(E->d_pop) + mem.pop_off, 0, pop_bytes);
   if (e == hipSuccess) e = hipMemcpy(E->d_ids + mem.ids_off, ids, ncore, hipMemcpyHostToDevice);
@@ -532,15 +576,15 @@ int lbmh_ensemble_add(lbmh_ensemble* E, const int extent[3], const int periodic[
     en.div_z = FastDiv(uint32_t(extent[2]));
     en.div_y = FastDiv(uint32_t(extent[1]));
     en.periodic = uint32_t(mem.periodic[0] | (mem.periodic[1] << 1) | (mem.periodic[2] << 2));
-    en.steps_left = steps;
-    en.steps_done = 0;
+    MemberState<Q>& st = state<Q>(E, slot);
+    std::memset(&st, 0, sizeof(st));
+    st.steps_left = steps;
     en.bp = derive_bulk_params<double>(E->q, *params);
     for (int i = 0; i < Q; ++i) {
       const int64_t dist = neighbor_distance<Q>(i, int64_t(sy * sz), int64_t(sz));
       int64_t dm = dist % int64_t(npad);
       if (dm < 0) dm += int64_t(npad);
       en.dmod[i] = uint32_t(dm);
-      en.shift[i] = 0;
     }
     return LBMH_OK;
   });
@@ -559,7 +603,7 @@ int lbmh_ensemble_remove(lbmh_ensemble* E, int m)
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   Member& mem = E->members[m];
   E->pop_arena.release(mem.pop_off, mem.pop_bytes);
@@ -688,8 +732,9 @@ int lbmh_ensemble_initialize(lbmh_ensemble* E, int m)
     using S = decltype(s);
     const EnsembleLimits limits{E->pop_arena.capacity() / sizeof(S), E->id_arena.capacity(),
                                 uint32_t(E->max_members)};
-    return launch_post<Q, S>(E, static_cast<EnsembleEntry<Q>*>(E->d_table), static_cast<S*>(E->d_pop), limits,
-                             nullptr, m);
+    return launch_post<Q, S>(E, static_cast<EnsembleEntry<Q>*>(E->d_table),
+                             reinterpret_cast<const MemberState<Q>*>(device_state(E, 0)), static_cast<S*>(E->d_pop),
+                             limits, nullptr, m);
   });
   if (rc != LBMH_OK) return rc;
   LBMH_HIP(hipDeviceSynchronize());
@@ -701,14 +746,14 @@ int lbmh_ensemble_set_steps(lbmh_ensemble* E, int m, int64_t steps)
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
-    EnsembleEntry<Q>& en = entry<Q>(E, m);
-    en.steps_left = steps;
-    char* dst = static_cast<char*>(E->d_table) + size_t(m) * E->entry_bytes + offsetof(EnsembleEntry<Q>, steps_left);
-    LBMH_HIP(hipMemcpy(dst, &en.steps_left, sizeof(int64_t), hipMemcpyHostToDevice));
+    MemberState<Q>& st = state<Q>(E, m);
+    st.steps_left = steps;
+    char* dst = device_state(E, 0, m) + offsetof(MemberState<Q>, steps_left);
+    LBMH_HIP(hipMemcpy(dst, &st.steps_left, sizeof(int64_t), hipMemcpyHostToDevice));
     return LBMH_OK;
   });
 }
@@ -718,13 +763,13 @@ int lbmh_ensemble_status(lbmh_ensemble* E, int m, int64_t* done, int64_t* left)
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
-    const EnsembleEntry<Q>& en = entry<Q>(E, m);
-    if (done) *done = en.steps_done;
-    if (left) *left = en.steps_left;
+    const MemberState<Q>& st = state<Q>(E, m);
+    if (done) *done = st.steps_done;
+    if (left) *left = st.steps_left;
     return LBMH_OK;
   });
 }
@@ -733,15 +778,15 @@ int lbmh_ensemble_status_all(lbmh_ensemble* E, int64_t* done, int64_t* left)
 {
   if (!E || !done || !left) return fail(LBMH_E_INVALID, "null argument");
   DeviceGuard guard(E->device);
-  const int rc = pull_table(E);
+  const int rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
     for (int m = 0; m < E->max_members; ++m) {
-      const EnsembleEntry<Q>& en = entry<Q>(E, m);
+      const MemberState<Q>& st = state<Q>(E, m);
       const bool on = E->members[m].active;
-      done[m] = on ? en.steps_done : 0;
-      left[m] = on ? en.steps_left : 0;
+      done[m] = on ? st.steps_done : 0;
+      left[m] = on ? st.steps_left : 0;
     }
     return LBMH_OK;
   });
@@ -753,7 +798,7 @@ int lbmh_ensemble_ini_equilibrium(lbmh_ensemble* E, int m, const double* rho_u)
   if (rc != LBMH_OK) return rc;
   if (!rho_u) return fail(LBMH_E_INVALID, "null moments");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer staging;
@@ -765,9 +810,10 @@ int lbmh_ensemble_ini_equilibrium(lbmh_ensemble* E, int m, const double* rho_u)
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     S* pop = static_cast<S*>(E->d_pop) + en.pop_offset;
     hipLaunchKernelGGL((ini_equilibrium_kernel<Q, S>), dim3(grid_for(mem.ncore, 256)), dim3(256), 0, 0,
-                       (const double*)staging.p, E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(en),
+                       (const double*)staging.p, E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(st),
                        mem.params.force[0] * 0.5, mem.params.force[1] * 0.5, mem.params.force[2] * 0.5, forced,
                        nullptr);
     LBMH_HIP(hipGetLastError());
@@ -784,7 +830,7 @@ int lbmh_ensemble_upload(lbmh_ensemble* E, int m, const void* host, int dtype)
   if (rc != LBMH_OK) return rc;
   if (!host || dtype < LBMH_F64 || dtype > LBMH_F16) return fail(LBMH_E_INVALID, "bad host buffer or dtype");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer staging;
@@ -795,14 +841,15 @@ int lbmh_ensemble_upload(lbmh_ensemble* E, int m, const void* host, int dtype)
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     S* pop = static_cast<S*>(E->d_pop) + en.pop_offset;
     const dim3 grid(grid_for(mem.ncore, 256));
     if (dtype == LBMH_F64)
-      hipLaunchKernelGGL((scatter_populations<Q, double, S>), grid, dim3(256), 0, 0, (const double*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((scatter_populations<Q, double, S>), grid, dim3(256), 0, 0, (const double*)staging.p, pop, geom_of(en), shifts_of(st));
     else if (dtype == LBMH_F32)
-      hipLaunchKernelGGL((scatter_populations<Q, float, S>), grid, dim3(256), 0, 0, (const float*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((scatter_populations<Q, float, S>), grid, dim3(256), 0, 0, (const float*)staging.p, pop, geom_of(en), shifts_of(st));
     else
-      hipLaunchKernelGGL((scatter_populations<Q, _Float16, S>), grid, dim3(256), 0, 0, (const _Float16*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((scatter_populations<Q, _Float16, S>), grid, dim3(256), 0, 0, (const _Float16*)staging.p, pop, geom_of(en), shifts_of(st));
     LBMH_HIP(hipGetLastError());
     return LBMH_OK;
   });
@@ -817,7 +864,7 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
   if (rc != LBMH_OK) return rc;
   if (!host || dtype < LBMH_F64 || dtype > LBMH_F16) return fail(LBMH_E_INVALID, "bad host buffer or dtype");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer staging;
@@ -827,14 +874,15 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     const S* pop = static_cast<const S*>(E->d_pop) + en.pop_offset;
     const dim3 grid(grid_for(mem.ncore, 256));
     if (dtype == LBMH_F64)
-      hipLaunchKernelGGL((gather_populations<Q, double, S>), grid, dim3(256), 0, 0, (double*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((gather_populations<Q, double, S>), grid, dim3(256), 0, 0, (double*)staging.p, pop, geom_of(en), shifts_of(st));
     else if (dtype == LBMH_F32)
-      hipLaunchKernelGGL((gather_populations<Q, float, S>), grid, dim3(256), 0, 0, (float*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((gather_populations<Q, float, S>), grid, dim3(256), 0, 0, (float*)staging.p, pop, geom_of(en), shifts_of(st));
     else
-      hipLaunchKernelGGL((gather_populations<Q, _Float16, S>), grid, dim3(256), 0, 0, (_Float16*)staging.p, pop, geom_of(en), shifts_of(en));
+      hipLaunchKernelGGL((gather_populations<Q, _Float16, S>), grid, dim3(256), 0, 0, (_Float16*)staging.p, pop, geom_of(en), shifts_of(st));
     LBMH_HIP(hipGetLastError());
     return LBMH_OK;
   });
@@ -868,11 +916,12 @@ int member_block(lbmh_ensemble* E, int m, CheckpointBlock& b, std::vector<double
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     b.n_padded = en.n_padded;
     b.stride = en.stride;
     b.d_pop = static_cast<char*>(E->d_pop) + en.pop_offset * storage_size(E->storage);
     for (int i = 0; i < Q; ++i) {
-      b.shift[i] = en.shift[i];
+      b.shift[i] = st.shift[i];
       b.dist[i] = neighbor_distance<Q>(i, int64_t(en.sx), int64_t(en.sy));
     }
     return LBMH_OK;
@@ -888,7 +937,7 @@ int lbmh_ensemble_checkpoint_size(lbmh_ensemble* E, int m, int real, size_t* byt
   if (!bytes) return fail(LBMH_E_INVALID, "null argument");
   if (real != LBMH_F64 && real != LBMH_F32) return fail(LBMH_E_INVALID, "checkpoint value type must be F64 or F32");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   CheckpointBlock b;
   std::vector<double> walls;
@@ -903,7 +952,7 @@ int lbmh_ensemble_checkpoint_save(lbmh_ensemble* E, int m, int real, void* buffe
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   CheckpointBlock b;
   std::vector<double> walls;
@@ -917,7 +966,7 @@ int lbmh_ensemble_checkpoint_load(lbmh_ensemble* E, int m, int real, const void*
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   CheckpointBlock b;
   std::vector<double> walls;
@@ -929,10 +978,10 @@ int lbmh_ensemble_checkpoint_load(lbmh_ensemble* E, int m, int real, const void*
   // only the member's shifts change in the table
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
-    EnsembleEntry<Q>& en = entry<Q>(E, m);
-    for (int i = 0; i < Q; ++i) en.shift[i] = uint32_t(shift[i]);
-    char* dst = static_cast<char*>(E->d_table) + size_t(m) * E->entry_bytes + offsetof(EnsembleEntry<Q>, shift);
-    LBMH_HIP(hipMemcpy(dst, en.shift, sizeof(en.shift), hipMemcpyHostToDevice));
+    MemberState<Q>& st = state<Q>(E, m);
+    for (int i = 0; i < Q; ++i) st.shift[i] = uint32_t(shift[i]);
+    char* dst = device_state(E, 0, m) + offsetof(MemberState<Q>, shift);
+    LBMH_HIP(hipMemcpy(dst, st.shift, sizeof(st.shift), hipMemcpyHostToDevice));
     return LBMH_OK;
   });
 }
@@ -956,7 +1005,7 @@ int lbmh_ensemble_field_export(lbmh_ensemble* E, int m, int field, int overlap, 
   if (points > 0xffffffffull || !field_export_grid_fits(field_export_blocks(mem.n[0], mem.n[1], mem.n[2], overlap)))
     return fail(LBMH_E_INVALID, "member too large for one export (its 32z x 8x tiles exceed 2^32 work-items)");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   DeviceBuffer out;
   LBMH_HIP(hipMalloc(&out.p, want * sizeof(float)));
@@ -968,11 +1017,12 @@ int lbmh_ensemble_field_export(lbmh_ensemble* E, int m, int field, int overlap, 
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     PostArgs<Q> a;
     a.pop = static_cast<S*>(E->d_pop) + en.pop_offset;
     a.stride = en.stride;
     a.n_padded = en.n_padded;
-    for (int i = 0; i < Q; ++i) a.shift[i] = en.shift[i];
+    for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
     a.ids = E->d_ids + en.ids_offset;
     a.walls = E->d_walls + size_t(m) * kEnsembleWalls * 4;
     a.info = E->d_info + size_t(m) * kEnsembleWalls;
@@ -1008,7 +1058,7 @@ int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
   if (rc != LBMH_OK) return rc;
   if (!rho_u) return fail(LBMH_E_INVALID, "null output");
   DeviceGuard guard(E->device);
-  rc = pull_table(E);
+  rc = pull_state(E);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer out;
@@ -1019,9 +1069,10 @@ int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
+    const MemberState<Q>& st = state<Q>(E, m);
     const S* pop = static_cast<const S*>(E->d_pop) + en.pop_offset;
     hipLaunchKernelGGL((moments_kernel<Q, S>), dim3(grid_for(mem.ncore, 256)), dim3(256), 0, 0, (double*)out.p,
-                       E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(en), mem.params.force[0] * 0.5,
+                       E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(st), mem.params.force[0] * 0.5,
                        mem.params.force[1] * 0.5, mem.params.force[2] * 0.5, forced, nullptr);
     LBMH_HIP(hipGetLastError());
     return LBMH_OK;
@@ -1089,8 +1140,8 @@ int lbmh_ensemble_autotune(lbmh_ensemble* E, int trial_steps, lbmh_launch_config
   if (!E) return fail(LBMH_E_INVALID, "null ensemble");
   if (trial_steps < 1) return fail(LBMH_E_INVALID, "trial_steps must be >= 1");
   DeviceGuard guard(E->device);
-  // The trials run real steps: the members' populations and the device table
-  // (shifts, step counters) are copied aside first and put back after each
+  // The trials run real steps: the members' populations and their
+  // states (shifts, step counters) are copied aside first and put back after each
   // candidate, so every candidate times the same members and the ensemble
   // ends as it began.
   uint64_t end = 0;
@@ -1098,35 +1149,35 @@ int lbmh_ensemble_autotune(lbmh_ensemble* E, int trial_steps, lbmh_launch_config
     if (m.active) end = std::max(end, m.pop_off + m.pop_bytes);
   struct Scratch {
     void* pop = nullptr;
-    void* table = nullptr;
+    void* state = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     ~Scratch()
     {
       if (pop) (void)hipFree(pop);
-      if (table) (void)hipFree(table);
+      if (state) (void)hipFree(state);
       if (e0) (void)hipEventDestroy(e0);
       if (e1) (void)hipEventDestroy(e1);
     }
   } sc;
-  const size_t table_bytes = E->h_table.size();
+  const size_t state_bytes = E->h_state.size();
   LBMH_HIP(hipDeviceSynchronize());
   if (end) {
     const hipError_t e = hipMalloc(&sc.pop, end);
     if (e != hipSuccess) return fail(LBMH_E_MEMORY, "autotune needs device memory for a copy of the members' populations");
     LBMH_HIP(hipMemcpy(sc.pop, E->d_pop, end, hipMemcpyDeviceToDevice));
   }
-  LBMH_HIP(hipMalloc(&sc.table, table_bytes));
-  LBMH_HIP(hipMemcpy(sc.table, E->d_table, table_bytes, hipMemcpyDeviceToDevice));
+  LBMH_HIP(hipMalloc(&sc.state, state_bytes));
+  LBMH_HIP(hipMemcpy(sc.state, E->d_state, state_bytes, hipMemcpyDeviceToDevice));
   LBMH_HIP(hipEventCreate(&sc.e0));
   LBMH_HIP(hipEventCreate(&sc.e1));
   auto restore = [&]() -> int {
     LBMH_HIP(hipDeviceSynchronize());
     if (end) LBMH_HIP(hipMemcpy(E->d_pop, sc.pop, end, hipMemcpyDeviceToDevice));
-    LBMH_HIP(hipMemcpy(E->d_table, sc.table, table_bytes, hipMemcpyDeviceToDevice));
+    LBMH_HIP(hipMemcpy(E->d_state, sc.state, state_bytes, hipMemcpyDeviceToDevice));
     return LBMH_OK;
   };
   static const int kLds[] = {0, 16384, 24576, 32768, 40960, 49152};
-  static const int kGroup[] = {4, 8};
+  static const int kGroup[] = {8, 32};
   const lbmh_launch_config before = E->launch;
   const bool before_chosen = E->launch_chosen;
   lbmh_launch_config best = before;

@@ -311,3 +311,31 @@ def test_guarded_ensemble_members_match_plain_ensembles(gpu_available):
             one.ini_equilibrium(k, c.rho_u)
             one.step(25)
             np.testing.assert_array_equal(got[m], one.download(k))
+
+
+@pytest.mark.parametrize("calls", [((1, False),), ((2, False), (1, False)), ((33, True), (3, False)),
+                                   ((65, True), (32, True), (1, False), (2, True))])
+def test_step_state_over_odd_and_even_calls(gpu_available, calls):
+    """Each step reads one copy of the members' shifts and counters and writes
+    the other, odd calls copy back: members that run on, stop within the calls
+    and never start, in slots with a removed one between them, are bit-identical
+    to the same lattices stepped alone, through graph replays and plain steps."""
+    total = sum(n for n, _ in calls)
+    budgets = [-1, 2, 0, 34]
+    cases = [W.lid_driven_cavity((5 + k, 7, 9), tau=0.6 + 0.05 * k, lid_u=0.05) for k in range(4)]
+    cases[3] = W.random_periodic((8, 6, 11), seed=4)
+    with Ensemble(19, "f32", "bgk", max_members=6, population_bytes=1 << 22, cell_capacity=1 << 14) as ens:
+        gap = ens.add(cases[0])
+        members = [ens.add(c, steps=b) for c, b in zip(cases, budgets)]
+        ens.remove(gap)
+        for m, c in zip(members, cases):
+            ens.ini_equilibrium(m, c.rho_u)
+        for n, graph in calls:
+            ens.step(n, graph=graph)
+        for m, c, b in zip(members, cases, budgets):
+            ran = total if b < 0 else min(b, total)
+            assert ens.status(m) == (ran, b if b < 0 else b - ran)
+            with BlockLattice.from_case(c, "f32") as lat:
+                lat.ini_equilibrium(c.rho_u)
+                lat.collide_and_stream(ran)
+                np.testing.assert_array_equal(ens.download(m, "f32"), lat.download_populations("f32"))
