@@ -1177,7 +1177,7 @@ int lbmh_ensemble_autotune(lbmh_ensemble* E, int trial_steps, lbmh_launch_config
     return LBMH_OK;
   };
   static const int kLds[] = {0, 16384, 24576, 32768, 40960, 49152};
-  static const int kGroup[] = {8, 32};
+  static const int kGroup[] = {4, 8};
   const lbmh_launch_config before = E->launch;
   const bool before_chosen = E->launch_chosen;
   lbmh_launch_config best = before;
