@@ -179,6 +179,18 @@ int lbmh_halo_copy(lbmh_halo* halo, void* stream);
  * stream. */
 int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream);
 
+/* n_steps time steps of all blocks of a split lattice: per step the collision
+ * of every block, the copies of every halo, and the streaming with the
+ * post-processors stage by stage across the blocks (SuperLattice::
+ * collideAndStream, src/core/superLattice.hh:601-663): lbmh_collide of every
+ * block, lbmh_halo_copy_many and lbmh_stream of every block, bit for bit.
+ * Blocks that share device, q, storage, bulk kind and step count, listed
+ * together with every block their halos join them to, run each phase in one
+ * launch; others one launch per block.  The tables of the call are kept by
+ * the first block, so calls led by one block must run on one stream. */
+int lbmh_split_step(lbmh_lattice* const* lattices, size_t n_lattices, lbmh_halo* const* halos, size_t n_halos,
+                    int64_t n_steps, void* stream);
+
 /* Number of completed time steps and the PS shift of every column, in the
  * convention of CyclicColumn::_shift, normalised to [0, n_padded_cells)
  * (src/core/platform/cpu/sisd/column.h:193-204). */

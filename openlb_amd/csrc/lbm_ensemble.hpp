@@ -25,9 +25,12 @@ constexpr int kEnsembleWalls = 64;  // wall-table entries per lattice (ids 0..63
 
 template <int Q>
 struct EnsembleEntry {
-  uint64_t pop_offset;      // element offset of column 0 inside the population arena
+  void* pop;                // column 0
   uint64_t stride;          // elements between columns
-  uint64_t ids_offset;      // byte offset of the lattice's ids inside the id arena
+  const uint8_t* ids;       // per core cell dynamics id
+  const double* walls;      // [id][4] rho, ux, uy, uz
+  const uint32_t* info;     // [id] packed LocalInfo
+  const void* force;        // per-cell FORCE [3][ncore] in the arithmetic type, or null (bp.force)
   uint32_t n_padded, ncore, nx, ny, nz, sx, sy;
   FastDiv div_z, div_y;
   uint32_t periodic;
@@ -46,26 +49,26 @@ struct MemberState {
   uint32_t shift[Q];        // PS shifts, in [0, n_padded)
 };
 
-// Sizes of the arenas, so that a workgroup can refuse an entry that does not fit.
+// Address ranges of the arenas, so that a workgroup can refuse an entry that does not fit.
 struct EnsembleLimits {
-  uint64_t pop_elements;    // elements in the population arena
-  uint64_t id_bytes;        // bytes in the id arena
+  uint64_t pop_begin, pop_end;
+  uint64_t ids_begin, ids_end;
   uint32_t members;         // table slots
 };
 
 // Whole-member arguments of the single-block cell body, from a table entry.
 template <int Q, typename S>
 __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args(
-    const EnsembleEntry<Q>& e, const MemberState<Q>& st, uint32_t lat, S* arena, const uint8_t* ids, const double* walls, const uint32_t* info)
+    const EnsembleEntry<Q>& e, const MemberState<Q>& st, bool local)
 {
   using V = typename StorageTraits<S>::V;
   StepArgs<Q, V> a;
-  a.pop = arena + e.pop_offset;
+  a.pop = e.pop;
   a.stride = e.stride;
   a.n_padded = e.n_padded;
 #pragma unroll
   for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
-  a.ids = ids + e.ids_offset;
+  a.ids = e.ids;
   a.ncore = e.ncore;
   a.nx = e.nx;
   a.ny = e.ny;
@@ -77,9 +80,9 @@ __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args
   a.periodic = e.periodic;
   a.xcd_group = 0;
   a.reverse = 0;
-  a.walls = walls + uint64_t(lat) * kEnsembleWalls * 4;
-  a.info = info ? info + uint64_t(lat) * kEnsembleWalls : nullptr;
-  a.force = nullptr;  // members take the uniform force
+  a.walls = e.walls;
+  a.info = local ? e.info : nullptr;
+  a.force = static_cast<const V*>(e.force);
   a.bp.omega = V(e.bp.omega);
   a.bp.omega2 = V(e.bp.omega2);
   a.bp.guo = V(e.bp.guo);
@@ -96,11 +99,12 @@ __device__ __forceinline__ StepArgs<Q, typename StorageTraits<S>::V> member_args
 }
 
 // uniform guard: every column and the id range of the entry inside the arenas
-template <int Q>
+template <int Q, typename S>
 __device__ __forceinline__ bool entry_fits(const EnsembleEntry<Q>& e, const EnsembleLimits& limits)
 {
-  return !(e.stride < e.n_padded || e.pop_offset + uint64_t(Q) * e.stride > limits.pop_elements ||
-           e.ids_offset + e.ncore > limits.id_bytes);
+  const uint64_t pop = reinterpret_cast<uint64_t>(e.pop), ids = reinterpret_cast<uint64_t>(e.ids);
+  return !(e.stride < e.n_padded || pop < limits.pop_begin || pop + uint64_t(Q) * e.stride * sizeof(S) > limits.pop_end ||
+           ids < limits.ids_begin || ids + e.ncore > limits.ids_end);
 }
 
 // Streaming of a lattice, by the threads of its first workgroup: rotate its
@@ -136,10 +140,7 @@ __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEnt
                                                                const MemberState<Q>* __restrict__ state,
                                                                MemberState<Q>* __restrict__ next, uint32_t reverse,
                                                                const uint32_t* __restrict__ chunk_lattice,
-                                                               S* __restrict__ arena, const uint8_t* __restrict__ ids,
-                                                               const double* __restrict__ walls,
-                                                               const uint32_t* __restrict__ info, uint32_t xcd_group,
-                                                               EnsembleLimits limits)
+                                                               uint32_t xcd_group, EnsembleLimits limits)
 {
   const uint32_t b = chunk_of_block(blockIdx.x, gridDim.x, xcd_group, reverse);
   const uint32_t lat = chunk_lattice[b];
@@ -148,8 +149,8 @@ __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEnt
   const MemberState<Q>& st = state[lat];
   if (b == e.chunk_begin) advance_member(e, st, next[lat]);
   if (st.steps_left == 0) return;
-  if (!entry_fits(e, limits)) return;
-  const auto a = member_args<Q, S>(e, st, lat, arena, ids, walls, LOCAL == kLocalNone ? nullptr : info);
+  if (!entry_fits<Q, S>(e, limits)) return;
+  const auto a = member_args<Q, S>(e, st, LOCAL != kLocalNone);
   collide_stream_cell<Q, S, KIND, true, LOCAL>(a, (b - e.chunk_begin) * kBlock + threadIdx.x);
 }
 
@@ -159,9 +160,7 @@ template <int Q, typename S, int KIND>
 __global__ __launch_bounds__(64) void ensemble_local_kernel(const EnsembleEntry<Q>* __restrict__ table,
                                                             const MemberState<Q>* __restrict__ state,
                                                             const uint2* __restrict__ cells, uint32_t count,
-                                                            S* __restrict__ arena, const uint8_t* __restrict__ ids,
-                                                            const double* __restrict__ walls,
-                                                            const uint32_t* __restrict__ info, EnsembleLimits limits)
+                                                            EnsembleLimits limits)
 {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= count) return;
@@ -169,8 +168,8 @@ __global__ __launch_bounds__(64) void ensemble_local_kernel(const EnsembleEntry<
   if (lc.x >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lc.x];
   const MemberState<Q>& st = state[lc.x];
-  if (st.steps_left == 0 || !entry_fits(e, limits) || lc.y >= e.ncore) return;
-  const auto a = member_args<Q, S>(e, st, lc.x, arena, ids, walls, info);
+  if (st.steps_left == 0 || !entry_fits<Q, S>(e, limits) || lc.y >= e.ncore) return;
+  const auto a = member_args<Q, S>(e, st, true);
   collide_stream_cell<Q, S, KIND, true, kLocalCollide>(a, lc.y);
 }
 
@@ -187,9 +186,7 @@ template <int Q, typename S, int KIND, bool SCRATCH = false>
 __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q>* __restrict__ table,
                                                            const MemberState<Q>* __restrict__ state,
                                                            const uint2* __restrict__ cells, uint32_t count,
-                                                           S* __restrict__ arena, const uint8_t* __restrict__ ids,
-                                                           const double* __restrict__ walls,
-                                                           const uint32_t* __restrict__ info, EnsembleLimits limits,
+                                                            EnsembleLimits limits,
                                                            int only, int forced,
                                                            typename StorageTraits<S>::V* scratch = nullptr)
 {
@@ -207,16 +204,16 @@ __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q
   if (valid) {
     const EnsembleEntry<Q>& e = table[lc.x];
     const MemberState<Q>& st = state[lc.x];
-    valid = (only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore;
+    valid = (only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits<Q, S>(e, limits) && lc.y < e.ncore;
     if (valid) {
-      a.pop = arena + e.pop_offset;
+      a.pop = e.pop;
       a.stride = e.stride;
       a.n_padded = e.n_padded;
 #pragma unroll
       for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
-      a.ids = ids + e.ids_offset;
-      a.walls = walls + uint64_t(lc.x) * kEnsembleWalls * 4;
-      a.info = info + uint64_t(lc.x) * kEnsembleWalls;
+      a.ids = e.ids;
+      a.walls = e.walls;
+      a.info = e.info;
       a.cells = nullptr;
       a.recs = nullptr;
       a.remote = nullptr;
@@ -253,7 +250,6 @@ template <int Q, typename S>
 __global__ __launch_bounds__(64) void ensemble_plane_store_kernel(const EnsembleEntry<Q>* __restrict__ table,
                                                                   const MemberState<Q>* __restrict__ state,
                                                                   const uint2* __restrict__ cells, uint32_t count,
-                                                                  S* __restrict__ arena,
                                                                   const typename StorageTraits<S>::V* scratch,
                                                                   EnsembleLimits limits, int only)
 {
@@ -264,11 +260,11 @@ __global__ __launch_bounds__(64) void ensemble_plane_store_kernel(const Ensemble
   if (lc.x >= limits.members) return;
   const EnsembleEntry<Q>& e = table[lc.x];
   const MemberState<Q>& st = state[lc.x];
-  if (!((only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits(e, limits) && lc.y < e.ncore)) return;
+  if (!((only >= 0 ? int(lc.x) == only : st.stepped != 0) && entry_fits<Q, S>(e, limits) && lc.y < e.ncore)) return;
   int x, y, z;
   core_coords(e.div_z, e.div_y, int(e.ny), int(e.nz), lc.y, x, y, z);
   const uint32_t n = uint32_t(x + 1) * e.sx + uint32_t(y + 1) * e.sy + uint32_t(z + 1);
-  S* pop = arena + e.pop_offset;
+  S* pop = static_cast<S*>(e.pop);
 #pragma unroll
   for (int i = 0; i < Q; ++i)
     store_pop<S, V>(column_at(pop + uint64_t(i) * e.stride, wrap_index(n, st.shift[i], e.n_padded)),

@@ -791,17 +791,24 @@ __global__ __launch_bounds__(64) void plane_store_kernel(PostArgs<Q> a, const ty
                     scratch[uint64_t(k) * Q + i]);
 }
 
+// Eight cells of the list from entry `first` on, by one workgroup of 64 lanes.
 template <int Q, typename S, int KIND>
-__global__ __launch_bounds__(64) void outer_post_kernel(PostArgs<Q> a)
+__device__ __forceinline__ void outer_post_cells(const PostArgs<Q>& a, uint32_t first)
 {
   using V = typename StorageTraits<S>::V;
   __shared__ V nb[64 / kPostLanes][kPostSlots][4];
   const int slot = int(threadIdx.x % kPostLanes), j = int(threadIdx.x / kPostLanes);
-  const uint32_t k = blockIdx.x * (64 / kPostLanes) + uint32_t(j);
+  const uint32_t k = first + uint32_t(j);
   const bool valid = k < a.count;
   if (valid && slot < kPostSlots) post_gather_rec<Q, S>(a, a.recs + k, slot, nb[j][slot]);
   __syncthreads();
   if (valid && slot == 0) post_finish<Q, S, KIND>(a, a.recs[k].c, int(a.recs[k].id), nb[j]);
+}
+
+template <int Q, typename S, int KIND>
+__global__ __launch_bounds__(64) void outer_post_kernel(PostArgs<Q> a)
+{
+  outer_post_cells<Q, S, KIND>(a, blockIdx.x * (64 / kPostLanes));
 }
 
 // Neighbours of post-processed cells that lie in another block: entry `slot`
@@ -812,6 +819,21 @@ struct RemotePair {
   uint32_t src_core;
   uint32_t slot;
 };
+
+// rho and u of one such neighbour, from its block's arguments `a` into the
+// consuming block's remote buffer.
+template <int Q, typename S>
+__device__ __forceinline__ void remote_moments(const PostArgs<Q>& a, const RemotePair& p, void* out)
+{
+  using V = typename StorageTraits<S>::V;
+  V rho, u[3];
+  rho_u_at<Q, S, V>(a, p.src_padded, int(a.ids[p.src_core]), rho, u);
+  V* o = static_cast<V*>(out) + uint64_t(p.slot) * 4;
+  o[0] = rho;
+  o[1] = u[0];
+  o[2] = u[1];
+  o[3] = u[2];
+}
 
 // The PostStream exchange of the post-processors' neighbourhood
 // (superLattice.hh:639-640, the overlap cells boundary::set requests through
@@ -831,7 +853,6 @@ template <int Q, typename S>
 __global__ __launch_bounds__(64) void remote_moments_many_kernel(const RemoteBatchDesc<Q>* __restrict__ descs,
                                                                  uint32_t halos, uint32_t total)
 {
-  using V = typename StorageTraits<S>::V;
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= total) return;
   uint32_t lo = 0, hi = halos;
@@ -843,14 +864,7 @@ __global__ __launch_bounds__(64) void remote_moments_many_kernel(const RemoteBat
   const RemoteBatchDesc<Q>& d = descs[lo];
   const uint32_t j = k - d.first;
   if (j >= d.count) return;
-  const RemotePair p = d.pairs[j];
-  V rho, u[3];
-  rho_u_at<Q, S, V>(d.a, p.src_padded, int(d.a.ids[p.src_core]), rho, u);
-  V* o = static_cast<V*>(d.out) + uint64_t(p.slot) * 4;
-  o[0] = rho;
-  o[1] = u[0];
-  o[2] = u[1];
-  o[3] = u[2];
+  remote_moments<Q, S>(d.a, d.pairs[j], d.out);
 }
 
 }  // namespace lbmh

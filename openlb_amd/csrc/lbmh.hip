@@ -23,6 +23,7 @@
 #include "checkpoint.hpp"
 #include "lbm_fields.hpp"
 #include "lbm_kernels.hpp"
+#include "lbm_split.hpp"
 #include "lbmh.h"
 #include "lbmh_common.hpp"
 
@@ -131,6 +132,9 @@ struct lbmh_lattice {
   size_t halo_batch_bytes = 0;
   void* d_remote_batch = nullptr;
   size_t remote_batch_bytes = 0;
+  // tables of lbmh_split_step calls this block leads
+  void* d_split = nullptr;
+  size_t split_bytes = 0;
 };
 
 // Library default launch shape of a block, from sweeps of (LDS reservation,
@@ -604,6 +608,32 @@ void advance_shifts(lbmh_lattice* L)
   }
 }
 
+// The local-boundary cells that the whole-lattice pass leaves out.
+template <int Q, typename S, int KIND>
+int launch_local_list(const lbmh_lattice* L, const StepArgs<Q, typename StorageTraits<S>::V>& a, hipStream_t stream)
+{
+  const uint32_t count = L->has_local ? uint32_t(L->h_local.size()) : 0;
+  if (!count) return LBMH_OK;
+  hipLaunchKernelGGL((local_boundary_kernel<Q, S, KIND>), dim3(grid_for(count, 64)), dim3(64), 0, stream, a,
+                     static_cast<const uint32_t*>(L->d_local), count);
+  LBMH_HIP(hipGetLastError());
+  return LBMH_OK;
+}
+
+template <int Q, typename S>
+int launch_local_list(const lbmh_lattice* L, hipStream_t stream)
+{
+  if (!L->has_local || L->h_local.empty()) return LBMH_OK;
+  const auto a = step_args<Q, typename StorageTraits<S>::V>(L);
+  switch (L->kind) {
+  case LBMH_BGK: return launch_local_list<Q, S, kBGK>(L, a, stream);
+  case LBMH_FORCED_BGK: return launch_local_list<Q, S, kForcedBGK>(L, a, stream);
+  case LBMH_TRT: return launch_local_list<Q, S, kTRT>(L, a, stream);
+  case LBMH_FORCED_TRT: return launch_local_list<Q, S, kForcedTRT>(L, a, stream);
+  default: return launch_local_list<Q, S, kSmagorinsky>(L, a, stream);
+  }
+}
+
 template <int Q, typename S, int KIND>
 int launch_kind(lbmh_lattice* L, hipStream_t stream, int phase)
 {
@@ -617,11 +647,8 @@ int launch_kind(lbmh_lattice* L, hipStream_t stream, int phase)
     // the boundary cells collide with their BGK mixin (OMEGA) whatever the bulk kind
     hipLaunchKernelGGL((collide_stream_kernel<Q, S, KIND, true, kLocalFlat>), dim3(grid), dim3(kBlock), lds, stream, a);
     LBMH_HIP(hipGetLastError());
-    const uint32_t count = uint32_t(L->h_local.size());
-    if (count) {
-      hipLaunchKernelGGL((local_boundary_kernel<Q, S, KIND>), dim3(grid_for(count, 64)), dim3(64), 0, stream, a,
-                         static_cast<const uint32_t*>(L->d_local), count);
-    }
+    const int rc = launch_local_list<Q, S, KIND>(L, a, stream);
+    if (rc != LBMH_OK) return rc;
   } else if (L->uniform_bulk) {
     hipLaunchKernelGGL((collide_stream_kernel<Q, S, KIND, false>), dim3(grid), dim3(kBlock), lds, stream, a);
   } else {
@@ -658,6 +685,210 @@ int step_q(lbmh_lattice* L, hipStream_t stream, int phase = kPhaseBoth)
   case LBMH_F32: return launch_step<Q, float>(L, stream, phase);
   default: return launch_step<Q, _Float16>(L, stream, phase);
   }
+}
+
+// Tables of one lbmh_split_step call, laid out one after the other in host
+// memory and sent to the device in one copy.
+class SplitTables {
+ public:
+  template <typename T>
+  size_t add(const std::vector<T>& v)
+  {
+    const size_t at = (bytes_.size() + 255) / 256 * 256;
+    bytes_.resize(at + sizeof(T) * v.size());
+    if (!v.empty()) std::memcpy(bytes_.data() + at, v.data(), sizeof(T) * v.size());
+    return at;
+  }
+  const std::vector<unsigned char>& bytes() const { return bytes_; }
+
+ private:
+  std::vector<unsigned char> bytes_;
+};
+
+// One job per `run` entries of item `item`.
+void add_jobs(std::vector<SplitJob>& jobs, uint32_t item, uint32_t count, uint32_t run)
+{
+  for (uint32_t k = 0; k < count; k += run) jobs.push_back(SplitJob{item, k});
+}
+
+// n_steps steps of the blocks of a split lattice, from tables: the blocks share
+// q, storage, kind and step count and are closed under their halos.
+template <int Q, typename S>
+int split_steps(const std::vector<lbmh_lattice*>& blocks, const std::vector<lbmh_halo*>& halos, int64_t n_steps,
+                hipStream_t stream)
+{
+  using V = typename StorageTraits<S>::V;
+  lbmh_lattice* lead = blocks[0];
+  bool local = false;
+  std::unordered_map<const lbmh_lattice*, uint32_t> index;
+  std::vector<lbmh_lattice*> group;  // blocks with post-processors
+  for (uint32_t b = 0; b < blocks.size(); ++b) {
+    lbmh_lattice* X = blocks[b];
+    index[X] = b;
+    local = local || X->has_local;
+    if (!has_post(X)) continue;
+    group.push_back(X);
+    if (X->remote_pos.empty()) continue;
+    const int rc = resolve_remote(X);
+    if (rc != LBMH_OK) return rc;
+  }
+  std::vector<EnsembleEntry<Q>> table(blocks.size());
+  std::vector<MemberState<Q>> state(blocks.size());
+  std::vector<uint32_t> chunk_block;
+  std::vector<SplitPost<Q>> posts(blocks.size());
+  for (uint32_t b = 0; b < blocks.size(); ++b) {
+    const lbmh_lattice* X = blocks[b];
+    const CoreGeom g = core_geom(X);
+    EnsembleEntry<Q>& e = table[b];
+    e.pop = X->d_pop;
+    e.stride = X->stride;
+    e.ids = X->d_ids;
+    e.walls = X->d_walls;
+    e.info = X->d_info;
+    e.force = X->d_force;
+    e.n_padded = g.n_padded;
+    e.ncore = g.ncore;
+    e.nx = g.nx;
+    e.ny = g.ny;
+    e.nz = g.nz;
+    e.sx = g.sx;
+    e.sy = g.sy;
+    e.div_z = g.div_z;
+    e.div_y = g.div_y;
+    e.periodic = uint32_t(X->periodic[0] | (X->periodic[1] << 1) | (X->periodic[2] << 2));
+    e.chunk_begin = uint32_t(chunk_block.size());
+    e.bp = derive_bulk_params<double>(Q, X->params);
+    chunk_block.insert(chunk_block.end(), grid_for(g.ncore, kBlock), b);
+    MemberState<Q>& st = state[b];
+    st.steps_left = -1;
+    st.steps_done = X->steps;
+    for (int i = 0; i < Q; ++i) {
+      int64_t d = X->dist[i] % int64_t(X->n_padded);
+      if (d < 0) d += X->n_padded;
+      e.dmod[i] = uint32_t(d);
+      st.shift[i] = uint32_t(X->shift[i]);
+    }
+    posts[b].a = post_args<Q>(X);
+    post_forcing<Q>(X, posts[b].a);
+    posts[b].block = b;
+  }
+
+  std::vector<SplitHalo> copies;
+  std::vector<SplitJob> copy_jobs;
+  std::vector<SplitRemote<Q>> remotes[kPostStages];
+  std::vector<SplitJob> remote_jobs[kPostStages], post_jobs[kPostStages];
+  std::vector<SplitPost<Q>> stage_posts[kPostStages];
+  for (lbmh_halo* H : halos) {
+    if (!H->count) continue;
+    add_jobs(copy_jobs, uint32_t(copies.size()), H->count, 256);
+    copies.push_back(SplitHalo{H->dst->d_pop, H->src->d_pop, H->d_pairs, H->dst->stride, H->src->stride,
+                               H->dst->n_padded, H->src->n_padded, index[H->dst], index[H->src], H->count});
+  }
+  bool planes = false;
+  for (lbmh_lattice* X : group) {
+    planes = planes || !X->h_planes.empty();
+    for (int stage : {int(kStageEdges), int(kStageCorners)}) {
+      for (lbmh_halo* H : X->halos_in) {
+        if (H->remote[stage].empty()) continue;
+        const uint32_t count = uint32_t(H->remote[stage].size());
+        add_jobs(remote_jobs[stage], uint32_t(remotes[stage].size()), count, 64);
+        remotes[stage].push_back(SplitRemote<Q>{posts[index[H->src]], H->d_remote[stage], X->d_remote, count});
+      }
+      const auto& cells = stage == kStageEdges ? X->h_edges : X->h_corners;
+      if (cells.empty()) continue;
+      SplitPost<Q> p = posts[index[X]];
+      p.a.recs = stage == kStageEdges ? X->d_edge_recs : X->d_corner_recs;
+      p.a.count = uint32_t(cells.size());
+      add_jobs(post_jobs[stage], uint32_t(stage_posts[stage].size()), p.a.count, 64 / kPostLanes);
+      stage_posts[stage].push_back(p);
+    }
+  }
+
+  SplitTables t;
+  const size_t at_state[2] = {t.add(state), t.add(state)};
+  const size_t at_table = t.add(table), at_chunks = t.add(chunk_block);
+  const size_t at_copies = t.add(copies), at_copy_jobs = t.add(copy_jobs);
+  size_t at_remotes[kPostStages], at_remote_jobs[kPostStages], at_posts[kPostStages], at_post_jobs[kPostStages];
+  for (int stage = 0; stage < kPostStages; ++stage) {
+    at_remotes[stage] = t.add(remotes[stage]);
+    at_remote_jobs[stage] = t.add(remote_jobs[stage]);
+    at_posts[stage] = t.add(stage_posts[stage]);
+    at_post_jobs[stage] = t.add(post_jobs[stage]);
+  }
+  const size_t bytes = t.bytes().size();
+  if (lead->split_bytes < bytes) {
+    if (lead->d_split) LBMH_HIP(hipFree(lead->d_split));
+    lead->d_split = nullptr;
+    lead->split_bytes = 0;
+    LBMH_HIP(hipMalloc(&lead->d_split, bytes));
+    lead->split_bytes = bytes;
+  }
+  LBMH_HIP(hipMemcpyAsync(lead->d_split, t.bytes().data(), bytes, hipMemcpyHostToDevice, stream));
+  char* base = static_cast<char*>(lead->d_split);
+
+  BlockTableStep step{};
+  step.q = Q;
+  step.storage = lead->storage;
+  step.kind = lead->kind;
+  step.local = local;
+  step.table = base + at_table;
+  step.chunk_block = reinterpret_cast<const uint32_t*>(base + at_chunks);
+  step.chunks = uint32_t(chunk_block.size());
+  step.blocks = uint32_t(blocks.size());
+  // XCD groups as in an ensemble, unless a shape was chosen for the lead block
+  step.launch = lead->launch;
+  if (!lead->launch_chosen) step.launch.xcd_group = 32;
+
+  for (int64_t k = 0; k < n_steps; ++k) {
+    const uint32_t cur = uint32_t(k & 1);
+    const auto* before = reinterpret_cast<const MemberState<Q>*>(base + at_state[cur]);
+    const auto* after = reinterpret_cast<const MemberState<Q>*>(base + at_state[cur ^ 1u]);
+    step.state = before;
+    step.next = base + at_state[cur ^ 1u];
+    step.reverse = lead->passes & 1u;
+    const int rc = launch_block_table_step(step, stream);
+    if (rc != LBMH_OK) return rc;
+    for (lbmh_lattice* X : blocks) {
+      const int rl = launch_local_list<Q, S>(X, stream);
+      if (rl != LBMH_OK) return rl;
+    }
+    if (!copy_jobs.empty()) {
+      hipLaunchKernelGGL((split_halo_kernel<Q, S>), dim3(uint32_t(copy_jobs.size()), Q), dim3(256), 0, stream,
+                         reinterpret_cast<const SplitHalo*>(base + at_copies), before,
+                         reinterpret_cast<const SplitJob*>(base + at_copy_jobs));
+      LBMH_HIP(hipGetLastError());
+    }
+    for (lbmh_lattice* X : blocks) {
+      X->passes += 1;
+      advance_shifts(X);
+      X->steps += 1;
+    }
+    // the stages of run_post, every block reaching each stage together
+    if (planes) {
+      int rp = launch_remote_stage<Q, S>(lead, group, kStagePlanes, stream);
+      for (size_t x = 0; rp == LBMH_OK && x < group.size(); ++x)
+        rp = launch_post_stage<Q, S>(group[x], kStagePlanes, stream);
+      if (rp != LBMH_OK) return rp;
+    }
+    for (int stage : {int(kStageEdges), int(kStageCorners)}) {
+      if (!remote_jobs[stage].empty()) {
+        hipLaunchKernelGGL((split_remote_kernel<Q, S>), dim3(uint32_t(remote_jobs[stage].size())), dim3(64), 0, stream,
+                           reinterpret_cast<const SplitRemote<Q>*>(base + at_remotes[stage]), after,
+                           reinterpret_cast<const SplitJob*>(base + at_remote_jobs[stage]));
+        LBMH_HIP(hipGetLastError());
+      }
+      if (post_jobs[stage].empty()) continue;
+      const dim3 grid(uint32_t(post_jobs[stage].size()));
+      const auto* sp = reinterpret_cast<const SplitPost<Q>*>(base + at_posts[stage]);
+      const auto* jobs = reinterpret_cast<const SplitJob*>(base + at_post_jobs[stage]);
+      if (stage == kStageEdges)
+        hipLaunchKernelGGL((split_post_kernel<Q, S, kPostEdge>), grid, dim3(64), 0, stream, sp, after, jobs);
+      else
+        hipLaunchKernelGGL((split_post_kernel<Q, S, kPostCorner>), grid, dim3(64), 0, stream, sp, after, jobs);
+      LBMH_HIP(hipGetLastError());
+    }
+  }
+  return LBMH_OK;
 }
 
 // Dispatch of a functor over (Q, storage type).
@@ -785,6 +1016,7 @@ int lbmh_lattice_destroy(lbmh_lattice* L)
   if (L->d_remote) (void)hipFree(L->d_remote);
   if (L->d_halo_batch) (void)hipFree(L->d_halo_batch);
   if (L->d_remote_batch) (void)hipFree(L->d_remote_batch);
+  if (L->d_split) (void)hipFree(L->d_split);
   if (L->d_pop) (void)hipFree(L->d_pop);
   if (L->d_force) (void)hipFree(L->d_force);
   if (L->d_ids) (void)hipFree(L->d_ids);
@@ -1484,6 +1716,56 @@ int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream)
     LBMH_HIP(hipGetLastError());
     return LBMH_OK;
   });
+}
+
+int lbmh_split_step(lbmh_lattice* const* lattices, size_t n_lattices, lbmh_halo* const* halos, size_t n_halos,
+                    int64_t n_steps, void* stream)
+{
+  if (!lattices || !n_lattices || (n_halos && !halos)) return fail(LBMH_E_INVALID, "null argument");
+  if (n_steps < 0) return fail(LBMH_E_INVALID, "negative step count");
+  if (n_halos > 0xffffu) return fail(LBMH_E_INVALID, "too many halos in one batch");
+  const std::vector<lbmh_lattice*> blocks(lattices, lattices + n_lattices);
+  const std::vector<lbmh_halo*> joins(halos, halos + n_halos);
+  // the tables take blocks of one kind and step count that are closed under
+  // their halos, as many as fit one launch (HIP's 2^32 - 1 work-items)
+  bool tables = true;
+  uint64_t chunks = 0;
+  for (const lbmh_lattice* X : blocks) {
+    if (!X) return fail(LBMH_E_INVALID, "null lattice");
+    const lbmh_lattice* L = blocks[0];
+    tables = tables && X->device == L->device && X->q == L->q && X->storage == L->storage && X->kind == L->kind &&
+             X->steps == L->steps && std::count(blocks.begin(), blocks.end(), X) == 1;
+    chunks += grid_for(X->ncore, kBlock);
+  }
+  tables = tables && chunks * kBlock <= 0xffffffffull;
+  auto known = [&](const lbmh_lattice* X) { return X && std::find(blocks.begin(), blocks.end(), X) != blocks.end(); };
+  uint64_t cells = 0;
+  for (const lbmh_halo* H : joins) {
+    if (!H) return fail(LBMH_E_INVALID, "null halo");
+    tables = tables && known(H->dst) && known(H->src);
+    cells += H->count;
+  }
+  tables = tables && cells <= 0xffffffffull;
+  for (const lbmh_lattice* X : blocks) {
+    if (!has_post(X)) continue;
+    for (const lbmh_halo* H : X->halos_in) tables = tables && known(H->src);
+    for (const lbmh_halo* H : X->halos_out) tables = tables && (!H->dst || !has_post(H->dst) || known(H->dst));
+  }
+  if (tables) {
+    if (n_steps == 0) return LBMH_OK;
+    DeviceGuard guard(blocks[0]->device);
+    return with_types(blocks[0], [&](auto qc, auto t) -> int {
+      return split_steps<decltype(qc)::value, decltype(t)>(blocks, joins, n_steps, static_cast<hipStream_t>(stream));
+    });
+  }
+  for (int64_t k = 0; k < n_steps; ++k) {
+    int rc = LBMH_OK;
+    for (size_t b = 0; rc == LBMH_OK && b < n_lattices; ++b) rc = lbmh_collide(lattices[b], stream);
+    if (rc == LBMH_OK && n_halos) rc = lbmh_halo_copy_many(halos, n_halos, stream);
+    for (size_t b = 0; rc == LBMH_OK && b < n_lattices; ++b) rc = lbmh_stream(lattices[b], stream);
+    if (rc != LBMH_OK) return rc;
+  }
+  return LBMH_OK;
 }
 
 int lbmh_get_step_count(const lbmh_lattice* L, int64_t* steps)

@@ -101,4 +101,21 @@ BulkParams<V> derive_bulk_params(int q, const lbmh_bulk_params& p)
   return b;
 }
 
+// Collision of every block of a table in one launch, the ensemble's step
+// kernel: EnsembleEntry<q> table, MemberState<q> copies to read and to write,
+// chunk_block the block of each 256-cell chunk.  `local`: some block has local
+// boundaries (their flat faces are collided in this pass).
+struct BlockTableStep {
+  int q, storage, kind;
+  bool local;
+  const void* table;
+  const void* state;
+  void* next;
+  uint32_t reverse;
+  const uint32_t* chunk_block;
+  uint32_t chunks, blocks;
+  lbmh_launch_config launch;
+};
+int launch_block_table_step(const BlockTableStep& t, hipStream_t stream);
+
 }  // namespace lbmh

@@ -157,6 +157,12 @@ char* device_state(lbmh_ensemble* E, uint32_t k, int m = 0)
   return static_cast<char*>(E->d_state) + (size_t(k) * size_t(E->max_members) + size_t(m)) * E->state_bytes;
 }
 
+EnsembleLimits limits_of(const lbmh_ensemble* E)
+{
+  const uint64_t pop = reinterpret_cast<uint64_t>(E->d_pop), ids = reinterpret_cast<uint64_t>(E->d_ids);
+  return EnsembleLimits{pop, pop + E->pop_arena.capacity(), ids, ids + E->id_arena.capacity(), uint32_t(E->max_members)};
+}
+
 template <typename F>
 int with_q(const lbmh_ensemble* E, F&& f)
 {
@@ -164,16 +170,22 @@ int with_q(const lbmh_ensemble* E, F&& f)
 }
 
 template <typename F>
-int with_types(const lbmh_ensemble* E, F&& f)
+int with_types(int q, int storage, F&& f)
 {
-  if (E->q == 19) {
-    if (E->storage == LBMH_F64) return f(std::integral_constant<int, 19>(), double());
-    if (E->storage == LBMH_F32) return f(std::integral_constant<int, 19>(), float());
+  if (q == 19) {
+    if (storage == LBMH_F64) return f(std::integral_constant<int, 19>(), double());
+    if (storage == LBMH_F32) return f(std::integral_constant<int, 19>(), float());
     return f(std::integral_constant<int, 19>(), _Float16());
   }
-  if (E->storage == LBMH_F64) return f(std::integral_constant<int, 27>(), double());
-  if (E->storage == LBMH_F32) return f(std::integral_constant<int, 27>(), float());
+  if (storage == LBMH_F64) return f(std::integral_constant<int, 27>(), double());
+  if (storage == LBMH_F32) return f(std::integral_constant<int, 27>(), float());
   return f(std::integral_constant<int, 27>(), _Float16());
+}
+
+template <typename F>
+int with_types(const lbmh_ensemble* E, F&& f)
+{
+  return with_types(E->q, E->storage, std::forward<F>(f));
 }
 
 // The members' states as the device holds them; the table only changes here on the host.
@@ -278,13 +290,13 @@ Shifts<Q> shifts_of(const MemberState<Q>& st)
 // PostStream stage of the local boundaries: edges, then corners, of the
 // members that stepped (only < 0) or of member `only`.
 template <int Q, typename S>
-int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, const MemberState<Q>* st, S* arena, const EnsembleLimits& limits,
+int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, const MemberState<Q>* st, const EnsembleLimits& limits,
                 hipStream_t stream, int only)
 {
   const int forced = (E->kind == LBMH_FORCED_BGK || E->kind == LBMH_FORCED_TRT) ? 1 : 0;
   if (E->n_planes) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostPlane>), dim3(grid_for(E->n_planes, 64 / kPostLanes)), dim3(64),
-                       0, stream, table, st, E->d_planes, E->n_planes, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
+                       0, stream, table, st, E->d_planes, E->n_planes, limits, only,
                        forced);
     LBMH_HIP(hipGetLastError());
   }
@@ -293,21 +305,21 @@ int launch_post(lbmh_ensemble* E, const EnsembleEntry<Q>* table, const MemberSta
     using V = typename StorageTraits<S>::V;
     V* scratch = static_cast<V*>(E->d_plane_scratch);
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostPlane, true>), dim3(grid_for(E->n_pplanes, 64 / kPostLanes)),
-                       dim3(64), 0, stream, table, st, E->d_pplanes, E->n_pplanes, arena, E->d_ids, E->d_walls, E->d_info,
+                       dim3(64), 0, stream, table, st, E->d_pplanes, E->n_pplanes,
                        limits, only, forced, scratch);
     LBMH_HIP(hipGetLastError());
     hipLaunchKernelGGL((ensemble_plane_store_kernel<Q, S>), dim3(grid_for(E->n_pplanes, 64)), dim3(64), 0, stream,
-                       table, st, E->d_pplanes, E->n_pplanes, arena, static_cast<const V*>(scratch), limits, only);
+                       table, st, E->d_pplanes, E->n_pplanes, static_cast<const V*>(scratch), limits, only);
     LBMH_HIP(hipGetLastError());
   }
   if (E->n_edges) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostEdge>), dim3(grid_for(E->n_edges, 64 / kPostLanes)), dim3(64), 0,
-                       stream, table, st, E->d_edges, E->n_edges, arena, E->d_ids, E->d_walls, E->d_info, limits, only, forced);
+                       stream, table, st, E->d_edges, E->n_edges, limits, only, forced);
     LBMH_HIP(hipGetLastError());
   }
   if (E->n_corners) {
     hipLaunchKernelGGL((ensemble_post_kernel<Q, S, kPostCorner>), dim3(grid_for(E->n_corners, 64 / kPostLanes)), dim3(64), 0,
-                       stream, table, st, E->d_corners, E->n_corners, arena, E->d_ids, E->d_walls, E->d_info, limits, only,
+                       stream, table, st, E->d_corners, E->n_corners, limits, only,
                        forced);
     LBMH_HIP(hipGetLastError());
   }
@@ -334,56 +346,62 @@ lbmh_launch_config step_launch(const lbmh_ensemble* E)
   return c;
 }
 
+template <int Q, typename S, int LOCAL>
+int launch_step_kernel(int kind, const EnsembleEntry<Q>* table, const MemberState<Q>* st, MemberState<Q>* next,
+                       uint32_t reverse, const uint32_t* chunk_member, uint32_t chunks, const lbmh_launch_config& launch,
+                       const EnsembleLimits& limits, hipStream_t stream)
+{
+  const unsigned lds = unsigned(launch.lds_bytes);
+  const uint32_t group = uint32_t(launch.xcd_group);
+#define LBMH_ENSEMBLE_STEP(KIND_)                                                                               \
+  hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_, LOCAL>), dim3(chunks), dim3(kBlock), lds, stream, table, st, \
+                     next, reverse, chunk_member, group, limits)
+  switch (kind) {
+  case LBMH_BGK: LBMH_ENSEMBLE_STEP(kBGK); break;
+  case LBMH_FORCED_BGK: LBMH_ENSEMBLE_STEP(kForcedBGK); break;
+  case LBMH_TRT: LBMH_ENSEMBLE_STEP(kTRT); break;
+  case LBMH_FORCED_TRT: LBMH_ENSEMBLE_STEP(kForcedTRT); break;
+  default: LBMH_ENSEMBLE_STEP(kSmagorinsky); break;
+  }
+#undef LBMH_ENSEMBLE_STEP
+  LBMH_HIP(hipGetLastError());
+  return LBMH_OK;
+}
+
+// The boundary cells of a `local` step collide with their BGK mixin whatever the bulk kind.
+template <int Q, typename S>
+int launch_step_kernel(int kind, bool local, const EnsembleEntry<Q>* table, const MemberState<Q>* st,
+                       MemberState<Q>* next, uint32_t reverse, const uint32_t* chunk_member, uint32_t chunks,
+                       const lbmh_launch_config& launch, const EnsembleLimits& limits, hipStream_t stream)
+{
+  return local ? launch_step_kernel<Q, S, kLocalFlat>(kind, table, st, next, reverse, chunk_member, chunks, launch,
+                                                      limits, stream)
+               : launch_step_kernel<Q, S, kLocalNone>(kind, table, st, next, reverse, chunk_member, chunks, launch,
+                                                      limits, stream);
+}
+
 int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
 {
   const lbmh_launch_config launch = step_launch(E);
-  const unsigned lds = unsigned(launch.lds_bytes);
-  const uint32_t group = uint32_t(launch.xcd_group);
   return with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
     auto* table = static_cast<EnsembleEntry<Q>*>(E->d_table);
-    S* arena = static_cast<S*>(E->d_pop);
-    const EnsembleLimits limits{E->pop_arena.capacity() / sizeof(S), E->id_arena.capacity(),
-                                uint32_t(E->max_members)};
+    const EnsembleLimits limits = limits_of(E);
     const bool local = E->has_local;
     for (int64_t k = 0; k < n; ++k) {
       const uint32_t cur = uint32_t(k & 1);
       const auto* st = reinterpret_cast<const MemberState<Q>*>(device_state(E, cur));
       auto* next = reinterpret_cast<MemberState<Q>*>(device_state(E, cur ^ 1u));
       if (E->total_chunks) {
-#define LBMH_ENSEMBLE_STEP(KIND_)                                                                               \
-  hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_>), dim3(E->total_chunks), dim3(kBlock), lds, stream, table, st, \
-                     next, cur, E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
-#define LBMH_ENSEMBLE_STEP_LOCAL(KIND_)                                                                         \
-  hipLaunchKernelGGL((ensemble_step_kernel<Q, S, KIND_, kLocalFlat>), dim3(E->total_chunks), dim3(kBlock), lds,    \
-                     stream, table, st, next, cur, E->d_chunk, arena, E->d_ids, E->d_walls, E->d_info, group, limits)
-        if (local) {
-          // the boundary cells collide with their BGK mixin whatever the bulk kind
-          switch (E->kind) {
-          case LBMH_BGK: LBMH_ENSEMBLE_STEP_LOCAL(kBGK); break;
-          case LBMH_FORCED_BGK: LBMH_ENSEMBLE_STEP_LOCAL(kForcedBGK); break;
-          case LBMH_TRT: LBMH_ENSEMBLE_STEP_LOCAL(kTRT); break;
-          case LBMH_FORCED_TRT: LBMH_ENSEMBLE_STEP_LOCAL(kForcedTRT); break;
-          default: LBMH_ENSEMBLE_STEP_LOCAL(kSmagorinsky); break;
-          }
-        } else {
-          switch (E->kind) {
-          case LBMH_BGK: LBMH_ENSEMBLE_STEP(kBGK); break;
-          case LBMH_FORCED_BGK: LBMH_ENSEMBLE_STEP(kForcedBGK); break;
-          case LBMH_TRT: LBMH_ENSEMBLE_STEP(kTRT); break;
-          case LBMH_FORCED_TRT: LBMH_ENSEMBLE_STEP(kForcedTRT); break;
-          default: LBMH_ENSEMBLE_STEP(kSmagorinsky); break;
-          }
-        }
-#undef LBMH_ENSEMBLE_STEP_LOCAL
-#undef LBMH_ENSEMBLE_STEP
-        LBMH_HIP(hipGetLastError());
+        const int rc = launch_step_kernel<Q, S>(E->kind, local, table, st, next, cur, E->d_chunk, E->total_chunks,
+                                                launch, limits, stream);
+        if (rc != LBMH_OK) return rc;
       }
       if (local && E->n_local) {
 #define LBMH_ENSEMBLE_LOCAL(KIND_)                                                                              \
   hipLaunchKernelGGL((ensemble_local_kernel<Q, S, KIND_>), dim3(grid_for(E->n_local, 64)), dim3(64), 0, stream,      \
-                     table, st, E->d_local, E->n_local, arena, E->d_ids, E->d_walls, E->d_info, limits)
+                     table, st, E->d_local, E->n_local, limits)
         switch (E->kind) {
         case LBMH_BGK: LBMH_ENSEMBLE_LOCAL(kBGK); break;
         case LBMH_FORCED_BGK: LBMH_ENSEMBLE_LOCAL(kForcedBGK); break;
@@ -394,7 +412,7 @@ int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
 #undef LBMH_ENSEMBLE_LOCAL
         LBMH_HIP(hipGetLastError());
       }
-      const int rc = launch_post(E, table, static_cast<const MemberState<Q>*>(next), arena, limits, stream, -1);
+      const int rc = launch_post<Q, S>(E, table, static_cast<const MemberState<Q>*>(next), limits, stream, -1);
       if (rc != LBMH_OK) return rc;
     }
     if (n & 1) {
@@ -409,6 +427,19 @@ int launch_steps(lbmh_ensemble* E, int64_t n, hipStream_t stream)
 }
 
 }  // namespace
+
+int lbmh::launch_block_table_step(const BlockTableStep& t, hipStream_t stream)
+{
+  return with_types(t.q, t.storage, [&](auto qc, auto s) -> int {
+    constexpr int Q = decltype(qc)::value;
+    using S = decltype(s);
+    // the blocks are the caller's own allocations, not ranges of an arena
+    const EnsembleLimits limits{0, ~uint64_t(0), 0, ~uint64_t(0), t.blocks};
+    return launch_step_kernel<Q, S>(t.kind, t.local, static_cast<const EnsembleEntry<Q>*>(t.table),
+                                    static_cast<const MemberState<Q>*>(t.state), static_cast<MemberState<Q>*>(t.next),
+                                    t.reverse, t.chunk_block, t.chunks, t.launch, limits, stream);
+  });
+}
 
 extern "C" {
 
@@ -563,9 +594,11 @@ int lbmh_ensemble_add(lbmh_ensemble* E, const int extent[3], const int periodic[
     constexpr int Q = decltype(qc)::value;
     EnsembleEntry<Q>& en = entry<Q>(E, slot);
     std::memset(&en, 0, sizeof(en));
-    en.pop_offset = mem.pop_off / elem;
+    en.pop = static_cast<char*>(E->d_pop) + mem.pop_off;
     en.stride = align_up(npad * elem) / elem;
-    en.ids_offset = mem.ids_off;
+    en.ids = E->d_ids + mem.ids_off;
+    en.walls = E->d_walls + size_t(slot) * 4 * kEnsembleWalls;
+    en.info = E->d_info + size_t(slot) * kEnsembleWalls;
     en.n_padded = uint32_t(npad);
     en.ncore = ncore;
     en.nx = uint32_t(extent[0]);
@@ -730,11 +763,9 @@ int lbmh_ensemble_initialize(lbmh_ensemble* E, int m)
   rc = with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
-    const EnsembleLimits limits{E->pop_arena.capacity() / sizeof(S), E->id_arena.capacity(),
-                                uint32_t(E->max_members)};
+    const EnsembleLimits limits = limits_of(E);
     return launch_post<Q, S>(E, static_cast<EnsembleEntry<Q>*>(E->d_table),
-                             reinterpret_cast<const MemberState<Q>*>(device_state(E, 0)), static_cast<S*>(E->d_pop),
-                             limits, nullptr, m);
+                             reinterpret_cast<const MemberState<Q>*>(device_state(E, 0)), limits, nullptr, m);
   });
   if (rc != LBMH_OK) return rc;
   LBMH_HIP(hipDeviceSynchronize());
@@ -811,7 +842,7 @@ int lbmh_ensemble_ini_equilibrium(lbmh_ensemble* E, int m, const double* rho_u)
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
     const MemberState<Q>& st = state<Q>(E, m);
-    S* pop = static_cast<S*>(E->d_pop) + en.pop_offset;
+    S* pop = static_cast<S*>(en.pop);
     hipLaunchKernelGGL((ini_equilibrium_kernel<Q, S>), dim3(grid_for(mem.ncore, 256)), dim3(256), 0, 0,
                        (const double*)staging.p, E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(st),
                        mem.params.force[0] * 0.5, mem.params.force[1] * 0.5, mem.params.force[2] * 0.5, forced,
@@ -842,7 +873,7 @@ int lbmh_ensemble_upload(lbmh_ensemble* E, int m, const void* host, int dtype)
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
     const MemberState<Q>& st = state<Q>(E, m);
-    S* pop = static_cast<S*>(E->d_pop) + en.pop_offset;
+    S* pop = static_cast<S*>(en.pop);
     const dim3 grid(grid_for(mem.ncore, 256));
     if (dtype == LBMH_F64)
       hipLaunchKernelGGL((scatter_populations<Q, double, S>), grid, dim3(256), 0, 0, (const double*)staging.p, pop, geom_of(en), shifts_of(st));
@@ -875,7 +906,7 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
     const MemberState<Q>& st = state<Q>(E, m);
-    const S* pop = static_cast<const S*>(E->d_pop) + en.pop_offset;
+    const S* pop = static_cast<const S*>(en.pop);
     const dim3 grid(grid_for(mem.ncore, 256));
     if (dtype == LBMH_F64)
       hipLaunchKernelGGL((gather_populations<Q, double, S>), grid, dim3(256), 0, 0, (double*)staging.p, pop, geom_of(en), shifts_of(st));
@@ -919,7 +950,7 @@ int member_block(lbmh_ensemble* E, int m, CheckpointBlock& b, std::vector<double
     const MemberState<Q>& st = state<Q>(E, m);
     b.n_padded = en.n_padded;
     b.stride = en.stride;
-    b.d_pop = static_cast<char*>(E->d_pop) + en.pop_offset * storage_size(E->storage);
+    b.d_pop = en.pop;
     for (int i = 0; i < Q; ++i) {
       b.shift[i] = st.shift[i];
       b.dist[i] = neighbor_distance<Q>(i, int64_t(en.sx), int64_t(en.sy));
@@ -1019,11 +1050,11 @@ int lbmh_ensemble_field_export(lbmh_ensemble* E, int m, int field, int overlap, 
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
     const MemberState<Q>& st = state<Q>(E, m);
     PostArgs<Q> a;
-    a.pop = static_cast<S*>(E->d_pop) + en.pop_offset;
+    a.pop = static_cast<S*>(en.pop);
     a.stride = en.stride;
     a.n_padded = en.n_padded;
     for (int i = 0; i < Q; ++i) a.shift[i] = st.shift[i];
-    a.ids = E->d_ids + en.ids_offset;
+    a.ids = en.ids;
     a.walls = E->d_walls + size_t(m) * kEnsembleWalls * 4;
     a.info = E->d_info + size_t(m) * kEnsembleWalls;
     a.cells = nullptr;
@@ -1070,7 +1101,7 @@ int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
     using S = decltype(s);
     const EnsembleEntry<Q>& en = entry<Q>(E, m);
     const MemberState<Q>& st = state<Q>(E, m);
-    const S* pop = static_cast<const S*>(E->d_pop) + en.pop_offset;
+    const S* pop = static_cast<const S*>(en.pop);
     hipLaunchKernelGGL((moments_kernel<Q, S>), dim3(grid_for(mem.ncore, 256)), dim3(256), 0, 0, (double*)out.p,
                        E->d_ids + mem.ids_off, pop, geom_of(en), shifts_of(st), mem.params.force[0] * 0.5,
                        mem.params.force[1] * 0.5, mem.params.force[2] * 0.5, forced, nullptr);

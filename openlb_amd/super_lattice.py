@@ -81,6 +81,7 @@ class SuperLattice:
             self.blocks[key] = BlockLattice.from_case(sub, storage, device, overlap_ids=ring)
             self.origin[key] = lo
         self._build_halos(self_periodic)
+        self._block_table = (ctypes.c_void_p * len(self.blocks))(*[lat.handle.value for lat in self.blocks.values()])
         self._halo_table = (ctypes.c_void_p * max(1, len(self.halos)))(*[h.value for h in self.halos])
 
     # -- decomposition ---------------------------------------------------------
@@ -142,15 +143,10 @@ class SuperLattice:
     # -- time step -------------------------------------------------------------
 
     def collide_and_stream(self, steps: int = 1):
-        lib = abi.load()
-        for _ in range(int(steps)):
-            for lat in self.blocks.values():
-                abi.check(lib.lbmh_collide(lat.handle, None))
-            if self.halos:
-                # every block's overlap copies in one launch
-                abi.check(lib.lbmh_halo_copy_many(self._halo_table, len(self.halos), None))
-            for lat in self.blocks.values():
-                abi.check(lib.lbmh_stream(lat.handle, None))
+        if steps < 1 or not self.blocks:
+            return
+        abi.check(abi.load().lbmh_split_step(self._block_table, len(self.blocks), self._halo_table, len(self.halos),
+                                             int(steps), None))
 
     def initialize(self):
         """SuperLattice::initialize(): every block's post-processors once on the

@@ -17,6 +17,7 @@ import pytest
 
 import golden_cases as G
 from oracle import oracle as O
+from openlb_amd import abi
 from openlb_amd import workloads as W
 from openlb_amd.lattice import BlockLattice
 from openlb_amd.super_lattice import SuperLattice
@@ -346,3 +347,39 @@ def test_split_local_checkpoint_resumes_bit_identically(gpu_available, label, ma
         got = sup.download_populations("f64")
     mask = G.flow_mask(case)
     np.testing.assert_array_equal(got[mask], ref[mask])
+
+
+@pytest.mark.parametrize("blocks", [(2, 1, 1), (2, 2, 2), (1, 3, 2)])
+@pytest.mark.parametrize("name", ["cavity_local", "duct", "step", "interpolated", "forced", "periodic"])
+def test_split_step_matches_the_single_phases(gpu_available, name, blocks):
+    """lbmh_split_step runs each phase of all blocks from tables in one launch:
+    bit-identical to lbmh_collide, lbmh_halo_copy_many and lbmh_stream of every
+    block on every stored value, overlap included, over odd and even calls, with
+    edge, corner and plane post-processors, list cells, a FORCE field, and no
+    post-processors at all."""
+    case = {"cavity_local": lambda: W.local_velocity_cavity((12, 13, 14), tau=0.7, lid_u=0.06),
+            "duct": lambda: W.velocity_channel((14, 12, 11), u_in=0.04),
+            "step": lambda: W.step_cavity((16, 13, 15)),
+            "interpolated": lambda: W.velocity_channel((13, 12, 14), inlet="interp_velocity", outlet="interp_pressure"),
+            "forced": lambda: W.kolmogorov_flow((12, 13, 11), walls=True),
+            "periodic": lambda: W.random_periodic((12, 9, 70), seed=8)}[name]()
+    L = abi.load()
+    out = []
+    for tables in (True, False):
+        with SuperLattice(case, "f32", blocks) as sup:
+            sup.ini_equilibrium(case.rho_u)
+            sup.initialize()
+            for steps in (1, 4, 3):
+                if tables:
+                    sup.collide_and_stream(steps)
+                    continue
+                for _ in range(steps):
+                    for lat in sup.blocks.values():
+                        abi.check(L.lbmh_collide(lat.handle, None))
+                    if sup.halos:
+                        abi.check(L.lbmh_halo_copy_many(sup._halo_table, len(sup.halos), None))
+                    for lat in sup.blocks.values():
+                        abi.check(L.lbmh_stream(lat.handle, None))
+            assert all(lat.step_count() == 8 for lat in sup.blocks.values())
+            out.append([lat.checkpoint("f32") for lat in sup.blocks.values()])
+    assert out[0] == out[1]
