@@ -26,6 +26,7 @@
 #include "lbm_split.hpp"
 #include "lbmh.h"
 #include "lbmh_common.hpp"
+#include "result_copy.hpp"
 
 using namespace lbmh;
 
@@ -954,6 +955,7 @@ int lbmh_lattice_create(const lbmh_lattice_desc* desc, lbmh_lattice** out)
     return fail(LBMH_E_INVALID, "a population column must stay below 2 GiB (padded cells x bytes per population)");
   auto* L = new (std::nothrow) lbmh_lattice();
   if (!L) return fail(LBMH_E_MEMORY, "host allocation failed");
+  ResultPool::get().retain();
   L->device = desc->device;
   L->q = desc->q;
   L->n[0] = desc->nx;
@@ -1032,6 +1034,7 @@ int lbmh_lattice_destroy(lbmh_lattice* L)
   if (L->d_corner_recs) (void)hipFree(L->d_corner_recs);
   if (L->d_plane_recs) (void)hipFree(L->d_plane_recs);
   delete L;
+  ResultPool::get().release();
   return LBMH_OK;
 }
 
@@ -1352,8 +1355,9 @@ int lbmh_populations_download(lbmh_lattice* L, void* host, int host_dtype)
   if (host_dtype < LBMH_F64 || host_dtype > LBMH_F16) return fail(LBMH_E_INVALID, "unknown host dtype");
   DeviceGuard guard(L->device);
   const size_t bytes = size_t(L->q) * L->ncore * storage_size(host_dtype);
-  DeviceBuffer staging;
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  ResultBuffer staging;
+  const int ra = staging.allocate(L->device, bytes);
+  if (ra != LBMH_OK) return ra;
   const CoreGeom g = core_geom(L);
   const uint32_t grid = grid_for(L->ncore, 256);
   LBMH_HIP(hipDeviceSynchronize());
@@ -1372,8 +1376,7 @@ int lbmh_populations_download(lbmh_lattice* L, void* host, int host_dtype)
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(host, staging.p, bytes, hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return staging.to_host(host, bytes);
 }
 
 // One population column of a host block in OpenLB's storage order, with the
@@ -1888,8 +1891,10 @@ int lbmh_field_export(lbmh_lattice* L, int field, int overlap, const double conv
   if (points > 0xffffffffull || !field_export_grid_fits(field_export_blocks(L->n[0], L->n[1], L->n[2], overlap)))
     return fail(LBMH_E_INVALID, "block too large for one export (its 32z x 8x tiles exceed 2^32 work-items)");
   DeviceGuard guard(L->device);
-  DeviceBuffer out;
-  LBMH_HIP(hipMalloc(&out.p, want * sizeof(float)));
+  ResultBuffer out;
+  const int ra = out.allocate(L->device, want * sizeof(float));
+  if (ra != LBMH_OK) return ra;
+  LBMH_HIP(hipDeviceSynchronize());
   FieldConversion conv{0.0, 0.0, 0.0};
   if (conversion) conv = FieldConversion{conversion[0], conversion[1], conversion[2]};
   const int forced = (L->kind == LBMH_FORCED_BGK || L->kind == LBMH_FORCED_TRT) ? 1 : 0;
@@ -1905,8 +1910,7 @@ int lbmh_field_export(lbmh_lattice* L, int field, int overlap, const double conv
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(host, out.p, want * sizeof(float), hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return out.to_host(host, want * sizeof(float));
 }
 
 int lbmh_reduce_field(lbmh_lattice* L, int field, int op, const uint8_t* materials, const double conversion[3],
@@ -1954,8 +1958,9 @@ int lbmh_moments(lbmh_lattice* L, double* rho_u)
   if (!L || !rho_u) return fail(LBMH_E_INVALID, "null argument");
   DeviceGuard guard(L->device);
   const size_t bytes = size_t(4) * L->ncore * sizeof(double);
-  DeviceBuffer out;
-  LBMH_HIP(hipMalloc(&out.p, bytes));
+  ResultBuffer out;
+  const int ra = out.allocate(L->device, bytes);
+  if (ra != LBMH_OK) return ra;
   const CoreGeom g = core_geom(L);
   const uint32_t grid = grid_for(L->ncore, 256);
   const int forced = (L->kind == LBMH_FORCED_BGK || L->kind == LBMH_FORCED_TRT) ? 1 : 0;
@@ -1971,8 +1976,7 @@ int lbmh_moments(lbmh_lattice* L, double* rho_u)
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(rho_u, out.p, bytes, hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return out.to_host(rho_u, bytes);
 }
 
 int lbmh_reduce_moments(lbmh_lattice* L, double out[4])

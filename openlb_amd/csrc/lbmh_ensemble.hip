@@ -21,6 +21,7 @@
 #include "lbm_ensemble.hpp"
 #include "lbmh.h"
 #include "lbmh_common.hpp"
+#include "result_copy.hpp"
 
 using namespace lbmh;
 
@@ -193,6 +194,15 @@ int pull_state(lbmh_ensemble* E)
 {
   LBMH_HIP(hipDeviceSynchronize());
   LBMH_HIP(hipMemcpy(E->h_state.data(), device_state(E, 0), E->h_state.size(), hipMemcpyDeviceToHost));
+  return LBMH_OK;
+}
+
+// The state of member m alone.
+int pull_state(lbmh_ensemble* E, int m)
+{
+  LBMH_HIP(hipDeviceSynchronize());
+  LBMH_HIP(hipMemcpy(E->h_state.data() + size_t(m) * E->state_bytes, device_state(E, 0, m), E->state_bytes,
+                     hipMemcpyDeviceToHost));
   return LBMH_OK;
 }
 
@@ -454,6 +464,7 @@ int lbmh_ensemble_create(const lbmh_ensemble_desc* d, lbmh_ensemble** out)
   if (d->population_bytes < kAlign || d->cell_capacity < 1) return fail(LBMH_E_INVALID, "arena sizes must be positive");
   auto* E = new (std::nothrow) lbmh_ensemble();
   if (!E) return fail(LBMH_E_MEMORY, "host allocation failed");
+  ResultPool::get().retain();
   E->device = d->device;
   E->q = d->q;
   E->storage = d->storage;
@@ -513,6 +524,7 @@ int lbmh_ensemble_destroy(lbmh_ensemble* E)
   if (E->d_pplanes) (void)hipFree(E->d_pplanes);
   if (E->d_plane_scratch) (void)hipFree(E->d_plane_scratch);
   delete E;
+  ResultPool::get().release();
   return LBMH_OK;
 }
 
@@ -794,7 +806,7 @@ int lbmh_ensemble_status(lbmh_ensemble* E, int m, int64_t* done, int64_t* left)
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   return with_q(E, [&](auto qc) -> int {
     constexpr int Q = decltype(qc)::value;
@@ -829,7 +841,7 @@ int lbmh_ensemble_ini_equilibrium(lbmh_ensemble* E, int m, const double* rho_u)
   if (rc != LBMH_OK) return rc;
   if (!rho_u) return fail(LBMH_E_INVALID, "null moments");
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer staging;
@@ -861,7 +873,7 @@ int lbmh_ensemble_upload(lbmh_ensemble* E, int m, const void* host, int dtype)
   if (rc != LBMH_OK) return rc;
   if (!host || dtype < LBMH_F64 || dtype > LBMH_F16) return fail(LBMH_E_INVALID, "bad host buffer or dtype");
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
   DeviceBuffer staging;
@@ -895,12 +907,13 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
   if (rc != LBMH_OK) return rc;
   if (!host || dtype < LBMH_F64 || dtype > LBMH_F16) return fail(LBMH_E_INVALID, "bad host buffer or dtype");
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
-  DeviceBuffer staging;
+  ResultBuffer staging;
   const size_t bytes = size_t(E->q) * mem.ncore * storage_size(dtype);
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  rc = staging.allocate(E->device, bytes);
+  if (rc != LBMH_OK) return rc;
   rc = with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
@@ -918,8 +931,7 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(host, staging.p, bytes, hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return staging.to_host(host, bytes);
 }
 
 namespace {
@@ -983,7 +995,7 @@ int lbmh_ensemble_checkpoint_save(lbmh_ensemble* E, int m, int real, void* buffe
   int rc = check_member(E, m);
   if (rc != LBMH_OK) return rc;
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   CheckpointBlock b;
   std::vector<double> walls;
@@ -1036,10 +1048,11 @@ int lbmh_ensemble_field_export(lbmh_ensemble* E, int m, int field, int overlap, 
   if (points > 0xffffffffull || !field_export_grid_fits(field_export_blocks(mem.n[0], mem.n[1], mem.n[2], overlap)))
     return fail(LBMH_E_INVALID, "member too large for one export (its 32z x 8x tiles exceed 2^32 work-items)");
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
-  DeviceBuffer out;
-  LBMH_HIP(hipMalloc(&out.p, want * sizeof(float)));
+  ResultBuffer out;
+  rc = out.allocate(E->device, want * sizeof(float));
+  if (rc != LBMH_OK) return rc;
   FieldConversion conv{0.0, 0.0, 0.0};
   if (conversion) conv = FieldConversion{conversion[0], conversion[1], conversion[2]};
   const int forced = (E->kind == LBMH_FORCED_BGK || E->kind == LBMH_FORCED_TRT) ? 1 : 0;
@@ -1079,8 +1092,7 @@ int lbmh_ensemble_field_export(lbmh_ensemble* E, int m, int field, int overlap, 
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(host, out.p, want * sizeof(float), hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return out.to_host(host, want * sizeof(float));
 }
 
 int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
@@ -1089,12 +1101,13 @@ int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
   if (rc != LBMH_OK) return rc;
   if (!rho_u) return fail(LBMH_E_INVALID, "null output");
   DeviceGuard guard(E->device);
-  rc = pull_state(E);
+  rc = pull_state(E, m);
   if (rc != LBMH_OK) return rc;
   const Member& mem = E->members[m];
-  DeviceBuffer out;
+  ResultBuffer out;
   const size_t bytes = size_t(4) * mem.ncore * sizeof(double);
-  LBMH_HIP(hipMalloc(&out.p, bytes));
+  rc = out.allocate(E->device, bytes);
+  if (rc != LBMH_OK) return rc;
   const int forced = (E->kind == LBMH_FORCED_BGK || E->kind == LBMH_FORCED_TRT) ? 1 : 0;
   rc = with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
@@ -1109,8 +1122,7 @@ int lbmh_ensemble_moments(lbmh_ensemble* E, int m, double* rho_u)
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
-  LBMH_HIP(hipMemcpy(rho_u, out.p, bytes, hipMemcpyDeviceToHost));
-  return LBMH_OK;
+  return out.to_host(rho_u, bytes);
 }
 
 int lbmh_ensemble_step(lbmh_ensemble* E, int64_t n, void* stream)
