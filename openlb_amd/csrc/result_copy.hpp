@@ -3,22 +3,28 @@
 // An export evaluates a field into device memory and copies it to the caller's
 // pageable buffer.  Handed that buffer, hipMemcpy moved 10 GB/s (275 MB of
 // density and velocity of a 256^3 block: 27.6 ms): one thread copies out of the
-// runtime's staging memory and takes the page faults of a fresh array, 13 GB/s
-// where the link gives 52 GB/s.  Here several threads each copy one chunk to
-// their slot of a pinned buffer and on to the caller's, so that transfers and
-// host copies overlap.  Small exports (the 96 members of a study, 1 MB each)
-// cost a hipMalloc and a hipFree more than the copy: 230 us each.
+// runtime's staging memory and takes the page faults of a fresh array, 8-13 GB/s
+// where the link gives 52 GB/s.  Here helper threads copy chunks through a
+// pinned buffer (9.1 ms), so that transfers, host copies and page faults
+// overlap.  A small export (the 96 members of a study, 1 MB each) paid for a
+// hipMalloc and a hipFree and then for 256 page faults in a row, 230 us each:
+// it now takes one transfer, during which the helpers touch the caller's pages,
+// and 125 us.
 //
-// One pinned buffer (12 MB) and one device workspace (up to 64 MB) per process
-// serve whoever holds the lease; a second thread exporting at the same time
-// allocates for itself.  They are freed with the last lattice or ensemble.
+// One pinned buffer (12 MB), one device workspace (up to 64 MB) and five idle
+// helper threads per process serve whoever holds the lease; a second thread
+// exporting at the same time allocates and copies for itself.  They go with
+// the last lattice or ensemble.
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <system_error>
 #include <thread>
@@ -29,9 +35,81 @@
 namespace lbmh {
 
 constexpr size_t kCopyChunk = size_t(2) << 20;     // bytes of one transfer
-constexpr int kCopyThreads = 6;                    // slots, and threads of a large copy
+constexpr int kCopyThreads = 6;                    // slots; the caller and its helpers
 constexpr size_t kCopyDirect = size_t(64) << 10;   // up to here hipMemcpy's own path is as fast
+constexpr size_t kCopyHelped = size_t(256) << 10;  // from here on the helpers pay for their wake-up
 constexpr size_t kWorkspaceLimit = size_t(64) << 20;
+
+// Threads that run one job together with the caller.  Used under the lease.
+class CopyHelpers {
+ public:
+  // job(slot) for slot 0 on this thread and the others on the helpers that
+  // could be started; returns when all are done.
+  void run(const std::function<void(int)>& job)
+  {
+    if (threads_.empty()) pid_ = getpid();
+    try {
+      while (int(threads_.size()) < kCopyThreads - 1) {
+        const int slot = int(threads_.size()) + 1;
+        threads_.emplace_back([this, slot, round = round_] { serve(slot, round); });
+      }
+    } catch (const std::exception&) {
+      // fewer helpers
+    }
+    {
+      std::lock_guard<std::mutex> l(mutex_);
+      job_ = &job;
+      pending_ = int(threads_.size());
+      ++round_;
+    }
+    wake_.notify_all();
+    job(0);
+    std::unique_lock<std::mutex> l(mutex_);
+    done_.wait(l, [this] { return pending_ == 0; });
+    job_ = nullptr;
+  }
+
+  void stop()
+  {
+    {
+      std::lock_guard<std::mutex> l(mutex_);
+      quit_ = true;
+    }
+    wake_.notify_all();
+    // in a forked child the helpers do not exist
+    for (std::thread& t : threads_) {
+      if (pid_ == getpid()) t.join();
+      else t.detach();
+    }
+    threads_.clear();
+    quit_ = false;
+  }
+
+ private:
+  void serve(int slot, uint64_t seen)
+  {
+    std::unique_lock<std::mutex> l(mutex_);
+    for (;;) {
+      wake_.wait(l, [&] { return quit_ || round_ != seen; });
+      if (quit_) return;
+      seen = round_;
+      const std::function<void(int)>* job = job_;
+      l.unlock();
+      (*job)(slot);
+      l.lock();
+      if (--pending_ == 0) done_.notify_one();
+    }
+  }
+
+  std::mutex mutex_;
+  std::condition_variable wake_, done_;
+  std::vector<std::thread> threads_;
+  const std::function<void(int)>* job_ = nullptr;
+  uint64_t round_ = 0;
+  int pending_ = 0;
+  bool quit_ = false;
+  pid_t pid_ = 0;
+};
 
 struct ResultPool {
   std::mutex lease;        // held while an export uses the buffers
@@ -41,10 +119,12 @@ struct ResultPool {
   void* device = nullptr;
   size_t device_bytes = 0;
   int ordinal = -1;        // device the workspace lies on
+  CopyHelpers helpers;
 
   static ResultPool& get()
   {
-    static ResultPool pool;
+    // never destroyed: helpers that wait when the process exits are left to it
+    static ResultPool& pool = *new ResultPool;
     return pool;
   }
 
@@ -59,6 +139,7 @@ struct ResultPool {
     std::lock_guard<std::mutex> c(count_mutex);
     if (--users > 0) return;
     std::lock_guard<std::mutex> l(lease);
+    helpers.stop();
     if (pinned) (void)hipHostFree(pinned);
     drop_workspace();
     pinned = nullptr;
@@ -123,39 +204,55 @@ class ResultBuffer {
       LBMH_HIP(hipMemcpy(host, p, bytes, hipMemcpyDeviceToHost));
       return LBMH_OK;
     }
-    std::atomic<size_t> next{0};
+    char* const to = static_cast<char*>(host);
     std::atomic<int> error{hipSuccess};
-    auto work = [&](int slot, bool set_device) {
-      if (set_device) {
-        const hipError_t e = hipSetDevice(ordinal_);
-        if (e != hipSuccess) {
-          error = e;
-          return;
-        }
+    if (bytes <= kCopyChunk * kCopyThreads) {
+      // one transfer; meanwhile the helpers touch their part of the caller's
+      // pages, and copy it when the transfer is done
+      char* const stage = static_cast<char*>(pool.pinned);
+      if (bytes < kCopyHelped) {
+        LBMH_HIP(hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost));
+        std::memcpy(to, stage, bytes);
+        return LBMH_OK;
       }
-      char* stage = static_cast<char*>(pool.pinned) + size_t(slot) * kCopyChunk;
-      while (error == hipSuccess) {
-        const size_t at = next.fetch_add(kCopyChunk);
-        if (at >= bytes) return;
-        const size_t n = std::min(kCopyChunk, bytes - at);
-        const hipError_t e = hipMemcpy(stage, static_cast<const char*>(p) + at, n, hipMemcpyDeviceToHost);
-        if (e != hipSuccess) {
-          error = e;
-          return;
+      constexpr size_t kPage = 4096;
+      const size_t part = (bytes / kCopyThreads + kPage) / kPage * kPage;
+      std::atomic<int> arrived{0};  // 1: the data is there, -1: it will not be
+      std::atomic<size_t> next{0};
+      pool.helpers.run([&](int slot) {
+        if (slot == 0) {
+          const hipError_t e = hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost);
+          if (e != hipSuccess) error = e;
+          arrived = e == hipSuccess ? 1 : -1;
         }
-        std::memcpy(static_cast<char*>(host) + at, stage, n);
-      }
-    };
-    // a thread pays from two chunks each on
-    const int threads = int(std::min<size_t>(kCopyThreads, bytes / (2 * kCopyChunk)));
-    std::vector<std::thread> helpers;
-    try {
-      for (int t = 1; t < threads; ++t) helpers.emplace_back(work, t, true);
-    } catch (const std::exception&) {
-      // fewer helpers: the others, or this thread alone, take all chunks
+        for (;;) {
+          const size_t at = next.fetch_add(part);
+          if (at >= bytes) return;
+          const size_t n = std::min(part, bytes - at);
+          if (arrived == 0) {
+            for (size_t k = 0; k < n; k += kPage) const_cast<volatile char*>(to)[at + k] = 0;
+            while (arrived == 0) std::this_thread::yield();
+          }
+          if (arrived < 0) return;
+          std::memcpy(to + at, stage + at, n);
+        }
+      });
+    } else {
+      std::atomic<size_t> next{0};
+      pool.helpers.run([&](int slot) {
+        const hipError_t d = hipSetDevice(ordinal_);
+        if (d != hipSuccess) error = d;
+        char* const stage = static_cast<char*>(pool.pinned) + size_t(slot) * kCopyChunk;
+        while (error == hipSuccess) {
+          const size_t at = next.fetch_add(kCopyChunk);
+          if (at >= bytes) return;
+          const size_t n = std::min(kCopyChunk, bytes - at);
+          const hipError_t e = hipMemcpy(stage, static_cast<const char*>(p) + at, n, hipMemcpyDeviceToHost);
+          if (e != hipSuccess) error = e;
+          else std::memcpy(to + at, stage, n);
+        }
+      });
     }
-    work(0, false);
-    for (std::thread& t : helpers) t.join();
     if (error != hipSuccess) return hip_fail(static_cast<hipError_t>(error.load()), "hipMemcpy(device to host)");
     return LBMH_OK;
   }

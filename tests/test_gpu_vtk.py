@@ -142,3 +142,44 @@ def test_export_argument_errors(gpu_available):
         with pytest.raises(abi.LbmhError, match="conversion"):
             abi.check(L.lbmh_field_export(lat.handle, 3, 1, None, ptr, out.size))
         abi.check(L.lbmh_field_export(lat.handle, 0, 1, None, ptr, out.size))
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (16, 32, 32), (30, 30, 25), (64, 64, 63), (96, 120, 130)])
+def test_exports_of_every_size_reach_the_host_whole(gpu_available, shape):
+    """The way to the host depends on the size: hipMemcpy up to 64 KB, one
+    pinned transfer, a transfer shared by helper threads from 256 KB, chunks of
+    2 MB from 12 MB; FP64 moments, float32 fields and populations of a lattice
+    and of an ensemble member of the same state agree at every size, also
+    from two threads at once."""
+    import threading
+
+    case = W.taylor_green(shape)
+    pop, ids = Ensemble.bytes_for(19, "f32", shape)
+    with BlockLattice.from_case(case, "f32") as lat, Ensemble(19, "f32", "bgk", 1, pop + 512, ids + 512) as ens:
+        m = ens.add(case)
+        ens.ini_equilibrium(m, case.rho_u)
+        lat.ini_equilibrium(case.rho_u)
+        want = {}
+        for threads in (1, 2):
+            got = [None, None]
+
+            def work(k):
+                for _ in range(3):
+                    src, arg = (lat, ()) if k == 0 else (ens, (m,))
+                    f = V.SuperLatticeVelocity3D(src, member=m if k else None)
+                    got[k] = (src.moments(*arg), f.evaluate(0), (src.download(m, "f32") if k else
+                                                                 src.download_populations("f32")))
+            ts = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+            for t in ts:
+                t.start()
+                if threads == 1:
+                    t.join()
+            for t in ts:
+                t.join()
+            for a, b in zip(*got):
+                np.testing.assert_array_equal(a, b)
+            u = got[0][0][1:].transpose(3, 2, 1, 0).astype(np.float32).reshape(-1)
+            # the two sum 19 populations' momenta, of size up to 0.05, in different orders
+            assert np.abs(got[0][1] - u).max() <= 19 * 2.0 ** -24 * 0.05
+            for k, a in enumerate(got[0]):
+                np.testing.assert_array_equal(a, want.setdefault(k, a))
