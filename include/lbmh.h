@@ -250,6 +250,13 @@ int lbmh_moments(lbmh_lattice* lattice, double* rho_u);
 int lbmh_field_export(lbmh_lattice* lattice, int field, int overlap, const double conversion[3], float* host,
                       size_t floats);
 
+/* The same for one block of a split lattice: an overlap point (overlap 1) to
+ * which the halos into the block copy a bulk cell of another block reports
+ * that cell's field, as OpenLB's writer communicates the overlap before it
+ * evaluates the functor (src/io/superVtmWriter3D.hh:71-75). */
+int lbmh_split_field_export(lbmh_lattice* lattice, int field, int overlap, const double conversion[3], float* host,
+                            size_t floats);
+
 /* Reduction of a cell field over the core cells whose dynamics id is
  * selected: the sum, minimum or maximum of each component, in FP64, and the
  * number of cells visited.  Fields: the four of lbmh_field_export, each cell

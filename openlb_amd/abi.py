@@ -27,7 +27,7 @@ EXPORTS = (
     "lbmh_reduce_moments_noalloc", "lbmh_statistics",
     "lbmh_set_local_boundary", "lbmh_classify_boundary", "lbmh_initialize",
     "lbmh_classify_boundary_overlap", "lbmh_set_overlap_ids", "lbmh_halo_copy_many",
-    "lbmh_split_step",
+    "lbmh_split_step", "lbmh_split_field_export",
     "lbmh_collide", "lbmh_stream", "lbmh_halo_create", "lbmh_halo_destroy", "lbmh_halo_copy",
     "lbmh_synchronize", "lbmh_device_synchronize", "lbmh_lattice_footprint", "lbmh_abi_version", "lbmh_device_count",
     "lbmh_device_arch", "lbmh_last_error", "lbmh_set_launch_config", "lbmh_get_launch_config",
@@ -111,6 +111,7 @@ def load() -> ctypes.CDLL:
     L.lbmh_get_step_count.argtypes = [vp, ctypes.POINTER(i64)]
     L.lbmh_get_shifts.argtypes = [vp, vp]
     L.lbmh_field_export.argtypes = [vp, i32, i32, vp, vp, ctypes.c_size_t]
+    L.lbmh_split_field_export.argtypes = [vp, i32, i32, vp, vp, ctypes.c_size_t]
     L.lbmh_ensemble_field_export.argtypes = [vp, i32, i32, i32, vp, vp, ctypes.c_size_t]
     L.lbmh_checkpoint_size.argtypes = [vp, i32, ctypes.POINTER(ctypes.c_size_t)]
     L.lbmh_checkpoint_save.argtypes = [vp, i32, vp, ctypes.c_size_t]

@@ -907,6 +907,56 @@ int with_types(const lbmh_lattice* L, F&& f)
 }
 
 
+// lbmh_field_export; `joined`: overlap points take the bulk cells of other blocks that the halos copy there
+int export_field(lbmh_lattice* L, int field, int overlap, const double conversion[3], float* host, size_t floats, bool joined)
+{
+  if (!L || !host) return fail(LBMH_E_INVALID, "null argument");
+  if (field < LBMH_FIELD_DENSITY || field > LBMH_FIELD_PHYS_PRESSURE) return fail(LBMH_E_INVALID, "unknown field");
+  if (overlap < 0 || overlap > 1) return fail(LBMH_E_INVALID, "overlap must be 0 or 1 (the block's padding)");
+  if ((field == LBMH_FIELD_PHYS_VELOCITY || field == LBMH_FIELD_PHYS_PRESSURE) && !conversion)
+    return fail(LBMH_E_INVALID, "physical fields need the unit conversion factors");
+  const uint64_t points = uint64_t(L->n[0] + 2 * overlap) * (L->n[1] + 2 * overlap) * (L->n[2] + 2 * overlap);
+  const size_t want = size_t(points) * field_components(field);
+  if (floats != want)
+    return fail(LBMH_E_INVALID, "field buffer holds " + std::to_string(floats) + " floats, the export " +
+                                    std::to_string(want));
+  if (points > 0xffffffffull || !field_export_grid_fits(field_export_blocks(L->n[0], L->n[1], L->n[2], overlap)))
+    return fail(LBMH_E_INVALID, "block too large for one export (its 32z x 8x tiles exceed 2^32 work-items)");
+  DeviceGuard guard(L->device);
+  ResultBuffer out;
+  const int ra = out.allocate(L->device, want * sizeof(float));
+  if (ra != LBMH_OK) return ra;
+  LBMH_HIP(hipDeviceSynchronize());
+  FieldConversion conv{0.0, 0.0, 0.0};
+  if (conversion) conv = FieldConversion{conversion[0], conversion[1], conversion[2]};
+  const int forced = (L->kind == LBMH_FORCED_BGK || L->kind == LBMH_FORCED_TRT) ? 1 : 0;
+  const double* F = L->params.force;
+  const int rc = with_types(L, [&](auto qc, auto s) -> int {
+    constexpr int Q = decltype(qc)::value;
+    using S = decltype(s);
+    hipLaunchKernelGGL((field_export_kernel<Q, S>),
+                       dim3(uint32_t(field_export_blocks(L->n[0], L->n[1], L->n[2], overlap))),
+                       dim3(kExportTileZ * kExportTileX), 0, 0, post_args<Q>(L), overlap, field, conv, forced, F[0] * 0.5, F[1] * 0.5, F[2] * 0.5,
+                       force_field<S>(L), static_cast<float*>(out.p), uint32_t(points));
+    LBMH_HIP(hipGetLastError());
+    if (!joined || overlap != 1) return LBMH_OK;
+    for (const lbmh_halo* H : L->halos_in) {
+      if (!H->src) return fail(LBMH_E_INVALID, "a block of this halo was destroyed");
+      if (!H->count) continue;
+      const double* G = H->src->params.force;
+      const int src_forced = (H->src->kind == LBMH_FORCED_BGK || H->src->kind == LBMH_FORCED_TRT) ? 1 : 0;
+      hipLaunchKernelGGL((field_overlap_kernel<Q, S>), dim3(grid_for(H->count, 256)), dim3(256), 0, 0,
+                         post_args<Q>(H->src), H->d_pairs, H->count, L->size[1] * L->size[2], L->size[2],
+                         uint32_t(L->n[0] + 2), uint32_t(L->n[1] + 2), field, conv, src_forced, G[0] * 0.5, G[1] * 0.5,
+                         G[2] * 0.5, force_field<S>(H->src), static_cast<float*>(out.p));
+      LBMH_HIP(hipGetLastError());
+    }
+    return LBMH_OK;
+  });
+  if (rc != LBMH_OK) return rc;
+  return out.to_host(host, want * sizeof(float));
+}
+
 }  // namespace
 
 extern "C" {
@@ -1878,39 +1928,13 @@ int lbmh_checkpoint_load(lbmh_lattice* L, int real, const void* buffer, size_t b
 
 int lbmh_field_export(lbmh_lattice* L, int field, int overlap, const double conversion[3], float* host, size_t floats)
 {
-  if (!L || !host) return fail(LBMH_E_INVALID, "null argument");
-  if (field < LBMH_FIELD_DENSITY || field > LBMH_FIELD_PHYS_PRESSURE) return fail(LBMH_E_INVALID, "unknown field");
-  if (overlap < 0 || overlap > 1) return fail(LBMH_E_INVALID, "overlap must be 0 or 1 (the block's padding)");
-  if ((field == LBMH_FIELD_PHYS_VELOCITY || field == LBMH_FIELD_PHYS_PRESSURE) && !conversion)
-    return fail(LBMH_E_INVALID, "physical fields need the unit conversion factors");
-  const uint64_t points = uint64_t(L->n[0] + 2 * overlap) * (L->n[1] + 2 * overlap) * (L->n[2] + 2 * overlap);
-  const size_t want = size_t(points) * field_components(field);
-  if (floats != want)
-    return fail(LBMH_E_INVALID, "field buffer holds " + std::to_string(floats) + " floats, the export " +
-                                    std::to_string(want));
-  if (points > 0xffffffffull || !field_export_grid_fits(field_export_blocks(L->n[0], L->n[1], L->n[2], overlap)))
-    return fail(LBMH_E_INVALID, "block too large for one export (its 32z x 8x tiles exceed 2^32 work-items)");
-  DeviceGuard guard(L->device);
-  ResultBuffer out;
-  const int ra = out.allocate(L->device, want * sizeof(float));
-  if (ra != LBMH_OK) return ra;
-  LBMH_HIP(hipDeviceSynchronize());
-  FieldConversion conv{0.0, 0.0, 0.0};
-  if (conversion) conv = FieldConversion{conversion[0], conversion[1], conversion[2]};
-  const int forced = (L->kind == LBMH_FORCED_BGK || L->kind == LBMH_FORCED_TRT) ? 1 : 0;
-  const double* F = L->params.force;
-  const int rc = with_types(L, [&](auto qc, auto s) -> int {
-    constexpr int Q = decltype(qc)::value;
-    using S = decltype(s);
-    hipLaunchKernelGGL((field_export_kernel<Q, S>),
-                       dim3(uint32_t(field_export_blocks(L->n[0], L->n[1], L->n[2], overlap))),
-                       dim3(kExportTileZ * kExportTileX), 0, 0, post_args<Q>(L), overlap, field, conv, forced, F[0] * 0.5, F[1] * 0.5, F[2] * 0.5,
-                       force_field<S>(L), static_cast<float*>(out.p), uint32_t(points));
-    LBMH_HIP(hipGetLastError());
-    return LBMH_OK;
-  });
-  if (rc != LBMH_OK) return rc;
-  return out.to_host(host, want * sizeof(float));
+  return export_field(L, field, overlap, conversion, host, floats, false);
+}
+
+int lbmh_split_field_export(lbmh_lattice* L, int field, int overlap, const double conversion[3], float* host,
+                            size_t floats)
+{
+  return export_field(L, field, overlap, conversion, host, floats, true);
 }
 
 int lbmh_reduce_field(lbmh_lattice* L, int field, int op, const uint8_t* materials, const double conversion[3],
