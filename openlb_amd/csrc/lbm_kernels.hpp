@@ -517,13 +517,45 @@ __device__ __forceinline__ double wave_max(double v)
   return v;
 }
 
+// A workgroup's {sum, sum, sum, max} of its threads' values, in a fixed order.
+__device__ __forceinline__ void combine_statistics(const double (&acc)[4], double* out)
+{
+  __shared__ double lds[4][kBlock / 64];
+  __syncthreads();  // a previous combination has been read
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const double s = wave_sum(acc[k]);
+    if (lane == 0) lds[k][wave] = s;
+  }
+  {
+    const double m = wave_max(acc[3]);
+    if (lane == 0) lds[3][wave] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 0; k < 4; ++k) {
+      double s = 0.0;
+      for (int w = 0; w < kBlock / 64; ++w) s = k == 3 ? fmax(s, lds[3][w]) : s + lds[k][w];
+      out[k] = s;
+    }
+  }
+}
+
 // Lattice statistics of OpenLB (LatticeStatistics::Aggregatable, src/core/
 // latticeStatistics.h:49-71): over the cells whose collision reports a
 // statistic -- bulk cells {rho, |u|^2} (u with the F/2 shift when forced) and
 // moving walls {rho_w, |u_w|^2} (collision.h:343); BounceBack reports none.
-// Partial per workgroup: {count, sum rho, sum |u|^2, max |u|^2}.
-template <int Q, typename S>
-__global__ __launch_bounds__(kBlock) void statistics_kernel(double* partial, const uint8_t* ids, const S* pop,
+// Partial per workgroup: {count, sum rho, sum |u|^2, max |u|^2}; the workgroup
+// that finishes last combines them in a fixed order into `out`, in pinned host
+// memory, and stores this reading's `number` in `flag` behind it (or into device
+// memory, flag null).  A reading of a small lattice is all latency: a second
+// launch for the partials and a copy of the result took 16 of its 33 us (24^3
+// cavity).  LOCAL: some cell has a local boundary; without, the kernel is a
+// third of the code.
+template <int Q, typename S, bool LOCAL>
+__global__ __launch_bounds__(kBlock) void statistics_kernel(double* out, uint64_t* flag, uint64_t number,
+                                                            double* partial, uint32_t* finished, const uint8_t* ids, const S* pop,
                                                             CoreGeom g, Shifts<Q> sh, const double* walls,
                                                             const uint32_t* info, double omega,
                                                             double hfx, double hfy, double hfz, int forced,
@@ -535,9 +567,10 @@ __global__ __launch_bounds__(kBlock) void statistics_kernel(double* partial, con
     const int id = ids ? ids[c] : 1;
     if (id == 0 || id == 2) continue;
     double rho, usq;
-    const LocalInfo li = info ? unpack_local_info(info[id < 3 ? 0 : id]) : LocalInfo{kMovingWall, 0, 0, 0};
+    LocalInfo li{kMovingWall, 0, 0, 0};
+    if constexpr (LOCAL) li = unpack_local_info(info[id < 3 ? 0 : id]);
     if (id >= 3 && li.kind == kDeadWall) continue;
-    if (id >= 3 && li.kind != kMovingWall) {
+    if (LOCAL && id >= 3 && li.kind != kMovingWall) {
       // the statistic the local boundary's collision reports
       const uint32_t n = padded_of_core(g, c);
       V f[Q];
@@ -573,51 +606,28 @@ __global__ __launch_bounds__(kBlock) void statistics_kernel(double* partial, con
     acc[2] += usq;
     acc[3] = fmax(acc[3], usq);
   }
-  __shared__ double lds[4][kBlock / 64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double s = wave_sum(acc[k]);
-    if (lane == 0) lds[k][wave] = s;
-  }
-  {
-    const double m = wave_max(acc[3]);
-    if (lane == 0) lds[3][wave] = m;
+  combine_statistics(acc, partial + blockIdx.x * 4);
+  // the other workgroups' partials may lie in another XCD's L2: written back
+  // before the count, read after it
+  __shared__ bool last;
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = __hip_atomic_fetch_add(finished, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x;
   }
   __syncthreads();
-  if (threadIdx.x < 4) {
-    double s = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w)
-      s = threadIdx.x == 3 ? fmax(s, lds[3][w]) : s + lds[threadIdx.x][w];
-    partial[blockIdx.x * 4 + threadIdx.x] = s;
+  if (!last) return;
+  __threadfence();
+  double all[4] = {0, 0, 0, 0};
+  for (uint32_t p = threadIdx.x; p < gridDim.x; p += kBlock) {
+    for (int k = 0; k < 3; ++k)
+      all[k] += __hip_atomic_load(partial + p * 4 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    all[3] = fmax(all[3], __hip_atomic_load(partial + p * 4 + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
   }
-}
-
-static __global__ __launch_bounds__(kBlock) void statistics_partials_kernel(double* out, const double* partial,
-                                                                            uint32_t nparts)
-{
-  __shared__ double lds[4][kBlock / 64];
-  double acc[4] = {0, 0, 0, 0};
-  for (uint32_t p = threadIdx.x; p < nparts; p += kBlock) {
-    for (int k = 0; k < 3; ++k) acc[k] += partial[p * 4 + k];
-    acc[3] = fmax(acc[3], partial[p * 4 + 3]);
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double s = wave_sum(acc[k]);
-    if (lane == 0) lds[k][wave] = s;
-  }
-  {
-    const double m = wave_max(acc[3]);
-    if (lane == 0) lds[3][wave] = m;
-  }
-  __syncthreads();
-  if (threadIdx.x < 4) {
-    double s = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w)
-      s = threadIdx.x == 3 ? fmax(s, lds[3][w]) : s + lds[threadIdx.x][w];
-    out[threadIdx.x] = s;
+  combine_statistics(all, out);
+  if (threadIdx.x == 0) {
+    *finished = 0;  // for the next reading
+    // after the result (written by this thread), for a host that waits on it
+    if (flag) __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 

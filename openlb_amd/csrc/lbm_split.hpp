@@ -11,8 +11,9 @@
 //
 // With one launch per block and phase, and the descriptor tables of the halos
 // and of each post-processor stage sent from the host in every step, the 101^3
-// LocalVelocity cavity on 2x2x2 blocks took 440 us per step, of which the
-// kernels' work is about 60 us.
+// LocalVelocity cavity on 2x2x2 blocks took 440 us per step; it takes 87 us, of
+// which the collision is 42 us, the halos 17 us, and the edge and corner
+// processors with their remote neighbours 28 us.
 #pragma once
 
 #include "lbm_ensemble.hpp"

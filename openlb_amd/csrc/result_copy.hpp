@@ -119,6 +119,7 @@ struct ResultPool {
   void* device = nullptr;
   size_t device_bytes = 0;
   int ordinal = -1;        // device the workspace lies on
+  uint64_t number = 0;     // under the lease: readings that wait on the pinned buffer
   CopyHelpers helpers;
 
   static ResultPool& get()
@@ -190,17 +191,26 @@ class ResultBuffer {
     return LBMH_OK;
   }
 
+  // The pinned buffer, which kernels can write to, or null without the lease.
+  void* pinned()
+  {
+    ResultPool& pool = ResultPool::get();
+    if (!lock_.owns_lock()) return nullptr;
+    if (!pool.pinned && hipHostMalloc(&pool.pinned, kCopyChunk * kCopyThreads, hipHostMallocPortable) != hipSuccess) {
+      pool.pinned = nullptr;
+      (void)hipGetLastError();
+    }
+    return pool.pinned;
+  }
+
+  // A number no earlier holder of the lease was given.
+  uint64_t next_number() { return lock_.owns_lock() ? ++ResultPool::get().number : 0; }
+
   // The first `bytes` to pageable host memory, after the null stream's work.
   int to_host(void* host, size_t bytes)
   {
     ResultPool& pool = ResultPool::get();
-    if (bytes > kCopyDirect && lock_.owns_lock() && !pool.pinned) {
-      if (hipHostMalloc(&pool.pinned, kCopyChunk * kCopyThreads, hipHostMallocPortable) != hipSuccess) {
-        pool.pinned = nullptr;
-        (void)hipGetLastError();
-      }
-    }
-    if (bytes <= kCopyDirect || !lock_.owns_lock() || !pool.pinned) {
+    if (bytes <= kCopyDirect || !pinned()) {
       LBMH_HIP(hipMemcpy(host, p, bytes, hipMemcpyDeviceToHost));
       return LBMH_OK;
     }

@@ -127,3 +127,26 @@ def test_empty_selection_and_errors(gpu_available):
             abi.check(L.lbmh_reduce_field(lat.handle, 0, 7, None, None, ptr, None))
         with pytest.raises(abi.LbmhError, match="conversion"):
             abi.check(L.lbmh_reduce_field(lat.handle, 3, 0, None, None, ptr, None))
+
+
+@pytest.mark.parametrize("storage", ["f64", "f32"])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (16, 16, 1), (257, 1, 1), (9, 8, 64), (70, 64, 65)])
+def test_statistics_combine_every_workgroup_once(gpu_available, shape, storage):
+    """The workgroup that finishes last combines the others' partials: one
+    workgroup, one full, one and a rest, eighteen, and more cells than the 1024
+    workgroups hold at once; readings repeated without a step between agree bit
+    for bit.  Against numpy over the FP64 moments: sums of n terms of size one
+    to n times the rounding of the storage's arithmetic."""
+    case = W.random_periodic(shape, seed=9)
+    eps = 2.0 ** -52 if storage == "f64" else 2.0 ** -23
+    with BlockLattice.from_case(case, storage) as lat:
+        lat.ini_equilibrium(case.rho_u)
+        lat.collide_and_stream(3)
+        first, m = lat.statistics(), lat.moments()
+        for _ in range(3):
+            assert lat.statistics() == first
+    usq = (m[1:] ** 2).sum(axis=0)
+    assert first["cells"] == m[0].size
+    assert abs(first["average_rho"] - m[0].mean()) <= 64 * eps
+    assert abs(first["average_energy"] - 0.5 * usq.mean()) <= 64 * eps * max(usq.max(), 1e-3)
+    assert abs(first["max_u"] - np.sqrt(usq.max())) <= 64 * eps
