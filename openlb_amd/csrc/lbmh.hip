@@ -102,7 +102,7 @@ struct lbmh_lattice {
   bool id_defined[kMaxWalls] = {};   // ids given a wall or boundary entry
   uint8_t material_of[kMaxWalls] = {};  // the material (id of lbmh_set_dynamics_ids) each dynamics id stands for
   uint32_t info[kMaxWalls] = {};     // packed LocalInfo per id
-  uint32_t* d_info = nullptr;
+  uint32_t* d_info = nullptr;          // info[], then the count of finished workgroups of a statistics pass
   bool has_local = false;
   // per-cell FORCE of the forced kinds: [3][ncore] on the device in the
   // arithmetic type (double for FP64 storage, float otherwise) and in FP64 on
@@ -1065,11 +1065,11 @@ int lbmh_lattice_create(const lbmh_lattice_desc* desc, lbmh_lattice** out)
   hipError_t e = hipMalloc(&L->d_pop, pop_bytes);
   if (e == hipSuccess) e = hipMalloc((void**)&L->d_ids, L->ncore);
   if (e == hipSuccess) e = hipMalloc((void**)&L->d_walls, sizeof(double) * 4 * kMaxWalls);
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_partials, sizeof(double) * (4 * (L->n_partials + 1) + 1));
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_info, sizeof(uint32_t) * kMaxWalls);
-  if (e == hipSuccess) e = hipMemcpy(L->d_info, L->info, sizeof(L->info), hipMemcpyHostToDevice);
-  // the count of finished workgroups behind the partials
-  if (e == hipSuccess) e = hipMemset(L->d_partials + 4 * (L->n_partials + 1), 0, sizeof(double));
+  if (e == hipSuccess) e = hipMalloc((void**)&L->d_partials, sizeof(double) * 4 * (L->n_partials + 1));
+  if (e == hipSuccess) e = hipMalloc((void**)&L->d_info, sizeof(uint32_t) * (kMaxWalls + 1));
+  // the info table, and the count of finished workgroups of a statistics pass
+  const std::vector<uint32_t> info_and_count(kMaxWalls + 1, 0u);
+  if (e == hipSuccess) e = hipMemcpy(L->d_info, info_and_count.data(), sizeof(uint32_t) * (kMaxWalls + 1), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(L->d_pop, 0, pop_bytes);
   if (e == hipSuccess) e = hipMemset(L->d_ids, 0, L->ncore);
   if (e == hipSuccess) e = hipMemcpy(L->d_walls, L->walls, sizeof(L->walls), hipMemcpyHostToDevice);
@@ -2107,7 +2107,7 @@ int lbmh_statistics(lbmh_lattice* L, double out[4])
   uint64_t* const flag = pinned ? reinterpret_cast<uint64_t*>(pinned + 8) : nullptr;
   const uint64_t number = buffer.next_number();
   if (flag) __atomic_store_n(flag, uint64_t(0), __ATOMIC_RELEASE);  // exports leave data there
-  uint32_t* const finished = reinterpret_cast<uint32_t*>(L->d_partials + 4 * (L->n_partials + 1));
+  uint32_t* const finished = L->d_info + kMaxWalls;
   const int rs = settle(L);
   if (rs != LBMH_OK) return rs;
   const int rc = with_types(L, [&](auto qc, auto s) -> int {

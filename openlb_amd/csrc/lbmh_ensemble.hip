@@ -111,9 +111,10 @@ struct lbmh_ensemble {
   std::vector<Member> members;
   std::vector<unsigned char> h_table;   // host mirror of the member table
   // steps left and done and PS shifts of every member: two copies of
-  // max_members records on the device, the first current between calls (each
-  // step reads one and writes the other), and a host mirror of it
-  void* d_state = nullptr;
+  // max_members records on the device behind the table, the first current
+  // between calls (each step reads one and writes the other), and a host
+  // mirror of it
+  char* d_state = nullptr;
   size_t state_bytes = 0;               // one record
   std::vector<unsigned char> h_state;
   lbmh_launch_config launch{0, 4};  // used once launch_chosen, else step_launch()
@@ -155,7 +156,7 @@ MemberState<Q>& state(lbmh_ensemble* E, int m)
 // The device's copy k of member m's state.
 char* device_state(lbmh_ensemble* E, uint32_t k, int m = 0)
 {
-  return static_cast<char*>(E->d_state) + (size_t(k) * size_t(E->max_members) + size_t(m)) * E->state_bytes;
+  return E->d_state + (size_t(k) * size_t(E->max_members) + size_t(m)) * E->state_bytes;
 }
 
 EnsembleLimits limits_of(const lbmh_ensemble* E)
@@ -229,10 +230,12 @@ int push_table(lbmh_ensemble* E)
   if (rc != LBMH_OK) return rc;
   if (map.size() > E->chunk_capacity) return fail(LBMH_E_MEMORY, "chunk map capacity exceeded");
   E->total_chunks = uint32_t(map.size());
-  LBMH_HIP(hipMemcpy(E->d_table, E->h_table.data(), E->h_table.size(), hipMemcpyHostToDevice));
-  // both copies: a slot without a member has no workgroup to carry its state over
-  for (uint32_t k = 0; k < 2; ++k)
-    LBMH_HIP(hipMemcpy(device_state(E, k), E->h_state.data(), E->h_state.size(), hipMemcpyHostToDevice));
+  // table and both copies of the states (a slot without a member has no
+  // workgroup to carry its state over) in one copy
+  std::vector<unsigned char> all = E->h_table;
+  all.resize(size_t(E->d_state - static_cast<char*>(E->d_table)));
+  for (int k = 0; k < 2; ++k) all.insert(all.end(), E->h_state.begin(), E->h_state.end());
+  LBMH_HIP(hipMemcpy(E->d_table, all.data(), all.size(), hipMemcpyHostToDevice));
   if (!map.empty()) LBMH_HIP(hipMemcpy(E->d_chunk, map.data(), map.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
   E->version += 1;
   return LBMH_OK;
@@ -483,16 +486,16 @@ int lbmh_ensemble_create(const lbmh_ensemble_desc* d, lbmh_ensemble** out)
   hipError_t e = hipMalloc(&E->d_pop, E->pop_arena.capacity());
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_ids, E->id_arena.capacity());
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_walls, sizeof(double) * 4 * kEnsembleWalls * E->max_members);
-  if (e == hipSuccess) e = hipMalloc(&E->d_table, E->h_table.size());
-  if (e == hipSuccess) e = hipMalloc(&E->d_state, 2 * E->h_state.size());
-  if (e == hipSuccess) e = hipMemset(E->d_state, 0, 2 * E->h_state.size());
+  const size_t state_at = align_up(E->h_table.size()), table_bytes = state_at + 2 * E->h_state.size();
+  if (e == hipSuccess) e = hipMalloc(&E->d_table, table_bytes);
+  E->d_state = static_cast<char*>(E->d_table) + state_at;
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_chunk, sizeof(uint32_t) * E->chunk_capacity);
   E->boundary_capacity = d->boundary_capacity ? d->boundary_capacity : d->cell_capacity / 4 + 64;
   if (e == hipSuccess) e = hipMalloc((void**)&E->d_info, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
   if (e == hipSuccess) e = hipMemset(E->d_info, 0, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
   for (uint2** list : {&E->d_local, &E->d_edges, &E->d_corners, &E->d_planes, &E->d_pplanes})
     if (e == hipSuccess) e = hipMalloc((void**)list, sizeof(uint2) * E->boundary_capacity);
-  if (e == hipSuccess) e = hipMemcpy(E->d_table, E->h_table.data(), E->h_table.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemset(E->d_table, 0, table_bytes);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&E->capture_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
     const int rc = hip_fail(e, "lbmh_ensemble_create");
@@ -514,7 +517,6 @@ int lbmh_ensemble_destroy(lbmh_ensemble* E)
   if (E->d_ids) (void)hipFree(E->d_ids);
   if (E->d_walls) (void)hipFree(E->d_walls);
   if (E->d_table) (void)hipFree(E->d_table);
-  if (E->d_state) (void)hipFree(E->d_state);
   if (E->d_chunk) (void)hipFree(E->d_chunk);
   if (E->d_info) (void)hipFree(E->d_info);
   if (E->d_local) (void)hipFree(E->d_local);
