@@ -261,6 +261,46 @@ class SuperLattice:
         self.close()
 
 
+def piece_sources(case, ranges, key):
+    """The overlap points of cuboid `key`'s VTK piece (overlap 1) that hold a
+    copy of a bulk cell of a cuboid on another axis split, after OpenLB's
+    writer communicates the overlap (src/io/superVtmWriter3D.hh,
+    SuperLatticeF functors on communicated blocks): {source key: (point
+    indices in this piece, point indices in the source cuboid's core export)},
+    both in VTK point order (x fastest).  Overlap cells across a face the
+    block spans periodically by itself are its own images and not listed."""
+    shape = case.shape
+    lo = [ranges[d][key[d]][0] for d in range(3)]
+    n = [ranges[d][key[d]][1] - lo[d] for d in range(3)]
+    self_periodic = [bool(case.periodic[d] and len(ranges[d]) == 1) for d in range(3)]
+    ex, ey = n[0] + 2, n[1] + 2
+    out: dict = {}
+    for x in range(-1, n[0] + 1):
+        for y in range(-1, n[1] + 1):
+            for z in range(-1, n[2] + 1):
+                r = (x, y, z)
+                away = [d for d in range(3) if r[d] < 0 or r[d] >= n[d]]
+                if not away or all(self_periodic[d] for d in away):
+                    continue
+                g = [lo[d] + r[d] for d in range(3)]
+                ok = True
+                for d in range(3):
+                    if not 0 <= g[d] < shape[d]:
+                        if not case.periodic[d]:
+                            ok = False
+                            break
+                        g[d] %= shape[d]
+                if not ok or case.ids[tuple(g)] != 1:
+                    continue
+                src_key = tuple(next(k for k, (a, b) in enumerate(ranges[d]) if a <= g[d] < b) for d in range(3))
+                s = [g[d] - ranges[d][src_key[d]][0] for d in range(3)]
+                sn = [ranges[d][src_key[d]][1] - ranges[d][src_key[d]][0] for d in range(3)]
+                lists = out.setdefault(src_key, ([], []))
+                lists[0].append(((z + 1) * ey + (y + 1)) * ex + (x + 1))
+                lists[1].append((s[2] * sn[1] + s[1]) * sn[0] + s[0])
+    return {k: (np.asarray(a, dtype=np.int64), np.asarray(b, dtype=np.int64)) for k, (a, b) in out.items()}
+
+
 def overlap_ids(case, lo, hi) -> np.ndarray:
     """Materials around the block [lo, hi) of a case: the padded map of the
     block's first overlap layer, read from the whole domain (periodic axes
