@@ -5,6 +5,7 @@ parameters, so a member must be bit-identical to the same lattice advanced
 on its own by lbmh_step. The single-lattice path is pinned to the oracle and
 to OpenLB by test_gpu_parity.py, so bit-identity extends that pin to every
 member."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -339,3 +340,46 @@ def test_step_state_over_odd_and_even_calls(gpu_available, calls):
                 lat.ini_equilibrium(c.rho_u)
                 lat.collide_and_stream(ran)
                 np.testing.assert_array_equal(ens.download(m, "f32"), lat.download_populations("f32"))
+
+
+@pytest.mark.parametrize("steps", [1, 3, 4])
+def test_a_captured_call_can_be_replayed(gpu_available, steps):
+    """A program may capture an ensemble call into a graph of its own: every
+    replay advances the members by the captured number of steps, odd ones too
+    (the call ends on the copy of the states it started from), with reads and
+    plain steps of the program between the replays."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def call(name, *args):
+        assert getattr(hip, name)(*args) == 0, name
+
+    case = W.lid_driven_cavity((9, 8, 33), tau=0.7, lid_u=0.05)
+    stream, graph, replay = ctypes.c_void_p(), ctypes.c_void_p(), ctypes.c_void_p()
+    with Ensemble(19, "f32", "bgk", max_members=2, population_bytes=1 << 21, cell_capacity=1 << 13) as ens:
+        m = ens.add(case)
+        ens.ini_equilibrium(m, case.rho_u)
+        call("hipStreamCreateWithFlags", ctypes.byref(stream), 1)
+        call("hipStreamBeginCapture", stream, 1)
+        ens.step(steps, stream=stream.value)
+        call("hipStreamEndCapture", stream, ctypes.byref(graph))
+        call("hipGraphInstantiate", ctypes.byref(replay), graph, None, None, ctypes.c_size_t(0))
+        done = 0
+        for extra in (0, 1, 2):
+            call("hipGraphLaunch", replay, stream)
+            call("hipStreamSynchronize", stream)
+            done += steps
+            if extra:
+                ens.step(extra)
+                done += extra
+            assert ens.status(m) == (done, -1)
+            np.testing.assert_array_equal(ens.download(m, "f32"), _after(case, done))
+        call("hipGraphExecDestroy", replay)
+        call("hipGraphDestroy", graph)
+        call("hipStreamDestroy", stream)
+
+
+def _after(case, steps):
+    with BlockLattice.from_case(case, "f32") as lat:
+        lat.ini_equilibrium(case.rho_u)
+        lat.collide_and_stream(steps)
+        return lat.download_populations("f32")
