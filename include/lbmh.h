@@ -435,7 +435,9 @@ int lbmh_get_launch_config(const lbmh_lattice* lattice, lbmh_launch_config* conf
 
 /* Time candidate launch shapes on a scratch lattice of the same extent,
  * dynamics ids and parameters (the lattice's own populations are untouched),
- * keep the fastest on the lattice and return it in *chosen (may be NULL).
+ * keep the fastest on the lattice and return it in *chosen (may be NULL).  The
+ * shape in use and the default are among the candidates, and the shape in use
+ * stays unless another is faster in a second timing too.
  * trial_steps >= 1 timed steps per candidate.  Needs device memory for one
  * more copy of the lattice. */
 int lbmh_autotune(lbmh_lattice* lattice, int trial_steps, lbmh_launch_config* chosen);
@@ -543,7 +545,8 @@ int lbmh_ensemble_step_graph(lbmh_ensemble* ensemble, int64_t n_steps, void* str
  * flat faces are collided in the step kernel).  A shape set here is kept. */
 int lbmh_ensemble_set_launch_config(lbmh_ensemble* ensemble, const lbmh_launch_config* config);
 
-/* Time the candidate launch shapes (LDS reservation x XCD group) on the
+/* Time the candidate launch shapes (LDS reservation x XCD group, the shape in
+ * use and the default, as in lbmh_autotune) on the
  * ensemble's own members, trial_steps timed steps each, keep the fastest and
  * return it in *chosen (may be NULL).  No OpenLB counterpart.  The members'
  * populations and step state are copied aside and restored after every

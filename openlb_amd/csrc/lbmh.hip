@@ -22,6 +22,7 @@
 
 #include "boundary_classify.hpp"
 #include "checkpoint.hpp"
+#include "launch_shape.hpp"
 #include "lbm_fields.hpp"
 #include "lbm_kernels.hpp"
 #include "lbm_split.hpp"
@@ -2208,30 +2209,23 @@ int lbmh_autotune(lbmh_lattice* L, int trial_steps, lbmh_launch_config* chosen)
   }
   LBMH_HIP(hipEventCreate(&cleanup.e0));
   LBMH_HIP(hipEventCreate(&cleanup.e1));
-  static const int kLds[] = {0, 24576, 32768, 40960, 49152, 65536};
-  static const int kGroup[] = {0, 2, 4, 8, 16};
-  float best_ms = 0.f;
+  const std::vector<lbmh_launch_config> shapes =
+      tuning_shapes(L->launch, default_launch(L, L->has_local), {0, 2, 4, 8, 16, 32}, {0, 24576, 32768, 40960, 49152, 65536},
+                    grid_for(L->ncore, kBlock));
   lbmh_launch_config best = L->launch;
-  bool have = false;
-  for (int group : kGroup) {
-    for (int lds : kLds) {
-      T->launch = lbmh_launch_config{lds, group};
-      rc = lbmh_step(T, 2, nullptr);
-      if (rc != LBMH_OK) return rc;
-      LBMH_HIP(hipEventRecord(cleanup.e0, nullptr));
-      rc = lbmh_step(T, trial_steps, nullptr);
-      if (rc != LBMH_OK) return rc;
-      LBMH_HIP(hipEventRecord(cleanup.e1, nullptr));
-      LBMH_HIP(hipEventSynchronize(cleanup.e1));
-      float ms = 0.f;
-      LBMH_HIP(hipEventElapsedTime(&ms, cleanup.e0, cleanup.e1));
-      if (!have || ms < best_ms) {
-        best_ms = ms;
-        best = T->launch;
-        have = true;
-      }
-    }
-  }
+  rc = fastest_shape(shapes, [&](const lbmh_launch_config& shape, float* ms) -> int {
+    T->launch = shape;
+    const int rw = lbmh_step(T, 2, nullptr);
+    if (rw != LBMH_OK) return rw;
+    LBMH_HIP(hipEventRecord(cleanup.e0, nullptr));
+    const int rt = lbmh_step(T, trial_steps, nullptr);
+    if (rt != LBMH_OK) return rt;
+    LBMH_HIP(hipEventRecord(cleanup.e1, nullptr));
+    LBMH_HIP(hipEventSynchronize(cleanup.e1));
+    LBMH_HIP(hipEventElapsedTime(ms, cleanup.e0, cleanup.e1));
+    return LBMH_OK;
+  }, best);
+  if (rc != LBMH_OK) return rc;
   L->launch = best;
   L->launch_chosen = true;
   if (chosen) *chosen = best;

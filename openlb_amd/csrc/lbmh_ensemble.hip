@@ -17,6 +17,7 @@
 
 #include "boundary_classify.hpp"
 #include "checkpoint.hpp"
+#include "launch_shape.hpp"
 #include "lbm_fields.hpp"
 #include "lbm_ensemble.hpp"
 #include "lbmh.h"
@@ -1221,39 +1222,36 @@ int lbmh_ensemble_autotune(lbmh_ensemble* E, int trial_steps, lbmh_launch_config
     LBMH_HIP(hipMemcpy(E->d_state, sc.state, state_bytes, hipMemcpyDeviceToDevice));
     return LBMH_OK;
   };
-  static const int kLds[] = {0, 16384, 24576, 32768, 40960, 49152};
-  static const int kGroup[] = {4, 8};
   const lbmh_launch_config before = E->launch;
   const bool before_chosen = E->launch_chosen;
+  E->launch_chosen = false;
+  const lbmh_launch_config standard = step_launch(E);
+  E->launch_chosen = before_chosen;
+  const std::vector<lbmh_launch_config> shapes =
+      tuning_shapes(step_launch(E), standard, {4, 8, 16, 32}, {0, 16384, 24576, 32768, 40960, 49152}, E->total_chunks);
   lbmh_launch_config best = before;
-  float best_ms = 0.f;
-  bool have = false;
-  int rc = LBMH_OK;
-  for (int group : kGroup) {
-    for (int lds : kLds) {
-      E->launch = lbmh_launch_config{lds, group};
-      E->launch_chosen = true;  // time exactly this shape
-      rc = launch_steps(E, 1, nullptr);
-      if (rc == LBMH_OK && hipEventRecord(sc.e0, nullptr) != hipSuccess) rc = fail(LBMH_E_DEVICE, "hipEventRecord");
-      if (rc == LBMH_OK) rc = launch_steps(E, trial_steps, nullptr);
-      if (rc == LBMH_OK && hipEventRecord(sc.e1, nullptr) != hipSuccess) rc = fail(LBMH_E_DEVICE, "hipEventRecord");
-      if (rc == LBMH_OK && hipEventSynchronize(sc.e1) != hipSuccess) rc = fail(LBMH_E_DEVICE, "hipEventSynchronize");
-      float ms = 0.f;
-      if (rc == LBMH_OK && hipEventElapsedTime(&ms, sc.e0, sc.e1) != hipSuccess) rc = fail(LBMH_E_DEVICE, "hipEventElapsedTime");
-      const int rr = restore();
-      if (rc == LBMH_OK) rc = rr;
-      if (rc != LBMH_OK) {
-        E->launch = before;
-        E->launch_chosen = before_chosen;
-        E->version += 1;
-        return rc;
-      }
-      if (!have || ms < best_ms) {
-        best_ms = ms;
-        best = E->launch;
-        have = true;
-      }
-    }
+  const int rc = fastest_shape(shapes, [&](const lbmh_launch_config& shape, float* ms) -> int {
+    E->launch = shape;
+    E->launch_chosen = true;  // time exactly this shape
+    auto timed = [&]() -> int {
+      const int rw = launch_steps(E, 1, nullptr);
+      if (rw != LBMH_OK) return rw;
+      LBMH_HIP(hipEventRecord(sc.e0, nullptr));
+      const int rt = launch_steps(E, trial_steps, nullptr);
+      if (rt != LBMH_OK) return rt;
+      LBMH_HIP(hipEventRecord(sc.e1, nullptr));
+      LBMH_HIP(hipEventSynchronize(sc.e1));
+      LBMH_HIP(hipEventElapsedTime(ms, sc.e0, sc.e1));
+      return LBMH_OK;
+    };
+    const int rt = timed(), rr = restore();
+    return rt != LBMH_OK ? rt : rr;
+  }, best);
+  if (rc != LBMH_OK) {
+    E->launch = before;
+    E->launch_chosen = before_chosen;
+    E->version += 1;
+    return rc;
   }
   E->launch = best;
   E->launch_chosen = true;
