@@ -408,6 +408,13 @@ int lbmh_synchronize(lbmh_lattice* lattice);
  * (src/core/superLattice.hh:666-671). */
 int lbmh_device_synchronize(int device);
 
+/* Results reach the host through one pinned buffer (up to 12 MB) and idle
+ * helper threads that the process keeps from its first large result on, also
+ * past its last lattice or ensemble, and a device workspace (up to 64 MB) that
+ * goes with the last of them.  Give all of it back; the next result sets up
+ * what it needs.  No OpenLB counterpart. */
+int lbmh_release_buffers(void);
+
 /* Launch shape of the time-step kernel.  No OpenLB counterpart: the CUDA
  * platform launches every kernel with 32-thread blocks (src/core/platform/gpu/
  * cuda/operator.hh:422-429).  lds_bytes reserves dynamic LDS per 256-thread

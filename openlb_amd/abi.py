@@ -27,7 +27,7 @@ EXPORTS = (
     "lbmh_reduce_moments_noalloc", "lbmh_statistics",
     "lbmh_set_local_boundary", "lbmh_classify_boundary", "lbmh_initialize",
     "lbmh_classify_boundary_overlap", "lbmh_set_overlap_ids", "lbmh_halo_copy_many",
-    "lbmh_split_step", "lbmh_split_field_export",
+    "lbmh_split_step", "lbmh_split_field_export", "lbmh_release_buffers",
     "lbmh_collide", "lbmh_stream", "lbmh_halo_create", "lbmh_halo_destroy", "lbmh_halo_copy",
     "lbmh_synchronize", "lbmh_device_synchronize", "lbmh_lattice_footprint", "lbmh_abi_version", "lbmh_device_count",
     "lbmh_device_arch", "lbmh_last_error", "lbmh_set_launch_config", "lbmh_get_launch_config",
@@ -137,6 +137,7 @@ def load() -> ctypes.CDLL:
     L.lbmh_halo_copy.argtypes = [vp, vp]
     L.lbmh_synchronize.argtypes = [vp]
     L.lbmh_device_synchronize.argtypes = [i32]
+    L.lbmh_release_buffers.argtypes = []
     L.lbmh_lattice_footprint.argtypes = [vp, ctypes.POINTER(ctypes.c_size_t)]
     L.lbmh_device_count.argtypes = [ctypes.POINTER(i32)]
     L.lbmh_device_arch.argtypes = [i32, ctypes.c_char_p, ctypes.c_size_t]

@@ -1577,6 +1577,12 @@ int lbmh_device_synchronize(int device)
   return LBMH_OK;
 }
 
+int lbmh_release_buffers(void)
+{
+  ResultPool::get().give_back();
+  return LBMH_OK;
+}
+
 int lbmh_ini_equilibrium(lbmh_lattice* L, const double* rho_u)
 {
   if (!L || !rho_u) return fail(LBMH_E_INVALID, "null argument");

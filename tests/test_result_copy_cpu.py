@@ -1,0 +1,180 @@
+"""The buffers and helper threads that bring results to the host
+(openlb_amd/csrc/result_copy.hpp), compiled with g++ against stand-ins for the
+HIP calls they make: device memory is host memory of a set size, and the first
+call that waits for the null stream waits out its backlog."""
+import os
+import subprocess
+
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+HEAD = r"""
+#include <sys/resource.h>
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <map>
+#include <thread>
+#include <vector>
+#include "result_copy.hpp"
+
+namespace lbmh { thread_local std::string g_error; }
+using namespace lbmh;
+
+static int bad = 0;
+#define CHECK(c) do { if (!(c)) { std::printf("line %d: %s\n", __LINE__, #c); ++bad; } } while (0)
+
+// the stand-in device
+static std::mutex fake;
+static std::map<void*, size_t> device_blocks, host_blocks;
+static size_t device_limit = size_t(1) << 40, device_used = 0;
+static std::vector<unsigned> host_flags;             // of every hipHostMalloc
+static std::vector<std::pair<void*, size_t>> copies;  // destination and size of every transfer
+static std::atomic<int> backlog_ms{0};
+static std::map<void*, size_t> registered;            // host memory the runtime knows
+static int device_mallocs = 0;
+
+static void drain()
+{
+  const int ms = backlog_ms.exchange(0);
+  if (ms) std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+}
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n)
+{
+  std::lock_guard<std::mutex> l(fake);
+  ++device_mallocs;
+  if (device_used + n > device_limit) return hipErrorOutOfMemory;
+  *p = std::malloc(n);
+  device_blocks[*p] = n;
+  device_used += n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p)
+{
+  std::lock_guard<std::mutex> l(fake);
+  device_used -= device_blocks.at(p);
+  device_blocks.erase(p);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned flags)
+{
+  std::lock_guard<std::mutex> l(fake);
+  *p = std::malloc(n);
+  host_blocks[*p] = n;
+  host_flags.push_back(flags);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p)
+{
+  std::lock_guard<std::mutex> l(fake);
+  host_blocks.erase(p);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind)
+{
+  drain();
+  std::memcpy(to, from, n);
+  std::lock_guard<std::mutex> l(fake);
+  copies.push_back({to, n});
+  return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+  drain();
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
+{
+  std::memset(a, 0, sizeof(*a));
+  a->type = hipMemoryTypeUnregistered;
+  for (auto& r : registered)
+    if (p >= r.first && p < static_cast<char*>(r.first) + r.second) a->type = hipMemoryTypeHost;
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "stand-in"; }
+}
+
+// One result of `n` bytes into `host`, as an export brings it there.
+static int bring(std::vector<unsigned char>& host, size_t n)
+{
+  host.assign(n, 0xee);
+  ResultBuffer out;
+  const int rc = out.allocate(0, n);
+  if (rc != LBMH_OK) return rc;
+  for (size_t k = 0; k < n; k += 1009) static_cast<unsigned char*>(out.p)[k] = static_cast<unsigned char>(k >> 8);
+  const int rt = out.to_host(host.data(), n);
+  for (size_t k = 0; k < n; k += 1009) CHECK(host[k] == static_cast<unsigned char>(k >> 8));
+  return rt;
+}
+
+static size_t threads()
+{
+  FILE* f = std::fopen("/proc/self/status", "r");
+  char line[256];
+  size_t n = 0;
+  while (std::fgets(line, sizeof line, f)) std::sscanf(line, "Threads: %zu", &n);
+  std::fclose(f);
+  return n;
+}
+"""
+
+# one lattice after another, each read a few times: nothing is set up again
+LIFETIME = r"""
+int main() {
+  ResultPool& pool = ResultPool::get();
+  std::vector<unsigned char> host;
+  size_t made = 0, alive = 0;
+  for (int k = 0; k < 8; ++k) {
+    pool.retain();
+    for (size_t n : {size_t(100) << 10, size_t(3) << 20, size_t(30) << 20}) {
+      CHECK(bring(host, n) == LBMH_OK);
+      CHECK(device_used >= n && device_used < 2 * n);  // a small result keeps a small workspace
+    }
+    pool.release();
+    CHECK(device_used == 0);  // the workspace goes with the last lattice
+    if (k == 0) { made = host_flags.size(); alive = threads(); }
+    CHECK(host_flags.size() == made && threads() == alive);
+  }
+  size_t held = 0;
+  for (auto& b : host_blocks) held += b.second;
+  CHECK(held <= (size_t(12) << 20) + 4096 && alive <= 6);  // bounded
+  pool.give_back();
+  CHECK(host_blocks.empty() && device_used == 0 && threads() == 1);
+  pool.retain();
+  CHECK(bring(host, size_t(3) << 20) == LBMH_OK);  // and set up again when needed
+  pool.give_back();  // a lattice is still alive
+  CHECK(host_blocks.empty() && device_used == 0);
+  CHECK(bring(host, size_t(3) << 20) == LBMH_OK);
+  pool.release();
+"""
+
+TAIL = r"""
+  std::printf("bad %d\n", bad);
+  std::fflush(stdout);
+  std::_Exit(bad != 0);
+}
+"""
+
+
+def run(body, tmp_path):
+    src, exe = tmp_path / "check.cpp", tmp_path / "check"
+    src.write_text(HEAD + body + TAIL)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include",
+                    f"-I{os.path.join(ROOT, 'include')}", f"-I{os.path.join(ROOT, 'openlb_amd', 'csrc')}",
+                    str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
+def test_buffers_outlive_the_last_lattice(tmp_path):
+    """A program with one lattice at a time sets the pinned buffer and the
+    helper threads up once; the device workspace goes with the last lattice, and
+    lbmh_release_buffers gives everything back."""
+    run(LIFETIME, tmp_path)
