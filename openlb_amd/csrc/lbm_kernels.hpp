@@ -547,7 +547,7 @@ __device__ __forceinline__ void combine_statistics(const double (&acc)[4], doubl
 // statistic -- bulk cells {rho, |u|^2} (u with the F/2 shift when forced) and
 // moving walls {rho_w, |u_w|^2} (collision.h:343); BounceBack reports none.
 // Partial per workgroup: {count, sum rho, sum |u|^2, max |u|^2}; the workgroup
-// that finishes last combines them in a fixed order into `out`, in pinned host
+// that finishes last combines them in a fixed order into `out`, in coherent host
 // memory, and stores this reading's `number` in `flag` behind it (or into device
 // memory, flag null).  A reading of a small lattice is all latency: a second
 // launch for the partials and a copy of the result took 16 of its 33 us (24^3

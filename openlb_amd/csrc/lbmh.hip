@@ -2108,12 +2108,11 @@ int lbmh_statistics(lbmh_lattice* L, double out[4])
   const int forced = (L->kind == LBMH_FORCED_BGK || L->kind == LBMH_FORCED_TRT) ? 1 : 0;
   const double* hf = L->params.force;
   ResultBuffer buffer;
-  double* const pinned = static_cast<double*>(buffer.pinned());
+  double* const pinned = static_cast<double*>(buffer.reading());
   double* const result = pinned ? pinned : L->d_partials + 4 * L->n_partials;
-  // behind the result in pinned memory: this reading's number, once it is there
+  // behind the result: this reading's number, once it is there
   uint64_t* const flag = pinned ? reinterpret_cast<uint64_t*>(pinned + 8) : nullptr;
   const uint64_t number = buffer.next_number();
-  if (flag) __atomic_store_n(flag, uint64_t(0), __ATOMIC_RELEASE);  // exports leave data there
   uint32_t* const finished = L->d_info + kMaxWalls;
   const int rs = settle(L);
   if (rs != LBMH_OK) return rs;

@@ -11,6 +11,9 @@
 // it now takes one transfer, during which the helpers touch the caller's pages,
 // and 125 us.
 //
+// A reading of a few words (lbmh_statistics) has pinned memory of its own, which
+// a running kernel writes and the host polls.
+//
 // One pinned buffer (12 MB), one device workspace (up to 64 MB) and five idle
 // helper threads per process serve whoever holds the lease; a second thread
 // exporting at the same time allocates and copies for itself.  The workspace
@@ -44,6 +47,7 @@ constexpr int kCopyThreads = 6;                    // slots; the caller and its 
 constexpr size_t kCopyDirect = size_t(64) << 10;   // up to here hipMemcpy's own path is as fast
 constexpr size_t kCopyHelped = size_t(256) << 10;  // from here on the helpers pay for their wake-up
 constexpr size_t kWorkspaceLimit = size_t(64) << 20;
+constexpr size_t kReadingBytes = 128;  // the values, and from byte 64 on the reading's number
 
 // Threads that run one job together with the caller.  Used under the lease.
 class CopyHelpers {
@@ -124,7 +128,8 @@ struct ResultPool {
   void* device = nullptr;
   size_t device_bytes = 0;
   int ordinal = -1;        // device the workspace lies on
-  uint64_t number = 0;     // under the lease: readings that wait on the pinned buffer
+  void* reading = nullptr; // pinned and coherent, kReadingBytes
+  uint64_t number = 0;     // under the lease: readings so far
   CopyHelpers helpers;
 
   static ResultPool& get()
@@ -155,6 +160,8 @@ struct ResultPool {
     helpers.stop();
     if (pinned) (void)hipHostFree(pinned);
     pinned = nullptr;
+    if (reading) (void)hipHostFree(reading);
+    reading = nullptr;
     drop_workspace();
   }
 
@@ -204,7 +211,25 @@ class ResultBuffer {
     return LBMH_OK;
   }
 
-  // The pinned buffer, which kernels can write to, or null without the lease.
+  // Memory for a reading that the host takes while the kernel runs, or null
+  // without the lease.  Such a poll needs coherent memory: without the flag an
+  // allocation follows the environment (HIP_HOST_COHERENT).
+  void* reading()
+  {
+    ResultPool& pool = ResultPool::get();
+    if (!lock_.owns_lock()) return nullptr;
+    if (!pool.reading) {
+      if (hipHostMalloc(&pool.reading, kReadingBytes, hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+        pool.reading = nullptr;
+        (void)hipGetLastError();
+        return nullptr;
+      }
+      std::memset(pool.reading, 0, kReadingBytes);
+    }
+    return pool.reading;
+  }
+
+  // The pinned buffer, or null without the lease.
   void* pinned()
   {
     ResultPool& pool = ResultPool::get();

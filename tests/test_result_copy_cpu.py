@@ -155,6 +155,30 @@ int main() {
   pool.release();
 """
 
+# what a kernel writes while the host polls lies in coherent memory of its own
+READING = r"""
+int main() {
+  ResultPool& pool = ResultPool::get();
+  pool.retain();
+  uint64_t last = 0;
+  void* at = nullptr;
+  {
+    ResultBuffer b;
+    at = b.reading();
+    CHECK(at && host_flags.size() == 1 && (host_flags[0] & hipHostMallocCoherent) && host_blocks[at] <= 4096);
+    for (size_t k = 0; k < kReadingBytes; ++k) CHECK(static_cast<char*>(at)[k] == 0);
+    last = b.next_number();
+    CHECK(last > 0);
+    ResultBuffer other;  // no lease: no memory and no number to wait for
+    CHECK(!other.reading() && other.next_number() == 0);
+  }
+  std::vector<unsigned char> host;
+  CHECK(bring(host, size_t(20) << 20) == LBMH_OK);
+  ResultBuffer b;
+  CHECK(b.reading() == at && b.next_number() > last);
+  for (size_t k = 0; k < kReadingBytes; ++k) CHECK(static_cast<char*>(at)[k] == 0);  // untouched by exports
+"""
+
 TAIL = r"""
   std::printf("bad %d\n", bad);
   std::fflush(stdout);
@@ -178,3 +202,8 @@ def test_buffers_outlive_the_last_lattice(tmp_path):
     helper threads up once; the device workspace goes with the last lattice, and
     lbmh_release_buffers gives everything back."""
     run(LIFETIME, tmp_path)
+
+
+def test_readings_are_polled_in_coherent_memory(tmp_path):
+    """lbmh_statistics' result and number: a small coherent allocation, no part of the export buffer."""
+    run(READING, tmp_path)
