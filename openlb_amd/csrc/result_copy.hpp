@@ -30,6 +30,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <condition_variable>
 #include <cstring>
 #include <functional>
@@ -263,7 +264,12 @@ class ResultBuffer {
         std::memcpy(to, stage, bytes);
         return LBMH_OK;
       }
+      // The transfer waits for the steps queued before it: the helpers spin for
+      // it only as long as a short one takes, then sleep until it is there.
       constexpr size_t kPage = 4096;
+      constexpr auto kSpin = std::chrono::microseconds(200);
+      std::mutex mutex;
+      std::condition_variable there;
       const size_t part = (bytes / kCopyThreads + kPage) / kPage * kPage;
       std::atomic<int> arrived{0};  // 1: the data is there, -1: it will not be
       std::atomic<size_t> next{0};
@@ -271,7 +277,11 @@ class ResultBuffer {
         if (slot == 0) {
           const hipError_t e = hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost);
           if (e != hipSuccess) error = e;
-          arrived = e == hipSuccess ? 1 : -1;
+          {
+            std::lock_guard<std::mutex> l(mutex);
+            arrived = e == hipSuccess ? 1 : -1;
+          }
+          there.notify_all();
         }
         for (;;) {
           const size_t at = next.fetch_add(part);
@@ -279,13 +289,20 @@ class ResultBuffer {
           const size_t n = std::min(part, bytes - at);
           if (arrived == 0) {
             for (size_t k = 0; k < n; k += kPage) const_cast<volatile char*>(to)[at + k] = 0;
-            while (arrived == 0) std::this_thread::yield();
+            const auto until = std::chrono::steady_clock::now() + kSpin;
+            while (arrived == 0 && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+            if (arrived == 0) {
+              std::unique_lock<std::mutex> l(mutex);
+              there.wait(l, [&] { return arrived != 0; });
+            }
           }
           if (arrived < 0) return;
           std::memcpy(to + at, stage + at, n);
         }
       });
     } else {
+      // every transfer waits for the steps queued before it, in a busy wait: one thread does
+      LBMH_HIP(hipStreamSynchronize(nullptr));
       std::atomic<size_t> next{0};
       pool.helpers.run([&](int slot) {
         const hipError_t d = hipSetDevice(ordinal_);

@@ -1,7 +1,7 @@
 """The buffers and helper threads that bring results to the host
 (openlb_amd/csrc/result_copy.hpp), compiled with g++ against stand-ins for the
-HIP calls they make: device memory is host memory of a set size, and the first
-call that waits for the null stream waits out its backlog."""
+HIP calls they make: device memory is host memory of a set size, and a call that
+waits for the null stream waits out its backlog, busily, as the runtime does."""
 import os
 import subprocess
 
@@ -30,14 +30,16 @@ static std::map<void*, size_t> device_blocks, host_blocks;
 static size_t device_limit = size_t(1) << 40, device_used = 0;
 static std::vector<unsigned> host_flags;             // of every hipHostMalloc
 static std::vector<std::pair<void*, size_t>> copies;  // destination and size of every transfer
-static std::atomic<int> backlog_ms{0};
+static std::atomic<int64_t> drained_at{0};            // ns of the steady clock
 static std::map<void*, size_t> registered;            // host memory the runtime knows
 static int device_mallocs = 0;
 
+static int64_t now() { return std::chrono::steady_clock::now().time_since_epoch().count(); }
+
 static void drain()
 {
-  const int ms = backlog_ms.exchange(0);
-  if (ms) std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+  while (now() < drained_at) {
+  }
 }
 
 extern "C" {
@@ -179,6 +181,33 @@ int main() {
   for (size_t k = 0; k < kReadingBytes; ++k) CHECK(static_cast<char*>(at)[k] == 0);  // untouched by exports
 """
 
+# one thread waits for the work queued before a result, whatever the size
+BACKLOG = r"""
+static double cpu_ms()
+{
+  rusage u;
+  getrusage(RUSAGE_SELF, &u);
+  return (u.ru_utime.tv_sec + u.ru_stime.tv_sec) * 1e3 + (u.ru_utime.tv_usec + u.ru_stime.tv_usec) * 1e-3;
+}
+int main() {
+  ResultPool::get().retain();
+  for (size_t n : {size_t(100) << 10, size_t(3) << 20, size_t(12) << 20, size_t(30) << 20}) {
+    std::vector<unsigned char> host;
+    CHECK(bring(host, n) == LBMH_OK);  // sets up
+    const double idle = cpu_ms();
+    CHECK(bring(host, n) == LBMH_OK);
+    const double alone = cpu_ms() - idle;
+    constexpr int kWait = 400;
+    drained_at = now() + int64_t(kWait) * 1000000;
+    const double before = cpu_ms();
+    CHECK(bring(host, n) == LBMH_OK);
+    const double used = cpu_ms() - before;
+    std::printf("%zu bytes: %.0f ms of CPU time behind %d ms, %.0f ms alone\n", n, used, kWait, alone);
+    // the caller's wait, the copy itself, and half a wait to spare
+    CHECK(used < 1.5 * kWait + alone);
+  }
+"""
+
 TAIL = r"""
   std::printf("bad %d\n", bad);
   std::fflush(stdout);
@@ -207,3 +236,8 @@ def test_buffers_outlive_the_last_lattice(tmp_path):
 def test_readings_are_polled_in_coherent_memory(tmp_path):
     """lbmh_statistics' result and number: a small coherent allocation, no part of the export buffer."""
     run(READING, tmp_path)
+
+
+def test_one_thread_waits_for_the_queued_steps(tmp_path):
+    """A result behind a long backlog takes one thread's CPU time, not every helper's."""
+    run(BACKLOG, tmp_path)
