@@ -208,6 +208,16 @@ int main() {
   }
 """
 
+# below kCopyHelped no helper is started or woken
+SMALL = r"""
+int main() {
+  ResultPool::get().retain();
+  std::vector<unsigned char> host;
+  for (size_t n : {size_t(2000), kCopyDirect, kCopyDirect + 1, size_t(432) << 10, kCopyHelped - 1}) CHECK(bring(host, n) == LBMH_OK);
+  CHECK(threads() == 1);
+  CHECK(bring(host, kCopyHelped) == LBMH_OK && threads() == 6);
+"""
+
 TAIL = r"""
   std::printf("bad %d\n", bad);
   std::fflush(stdout);
@@ -241,3 +251,7 @@ def test_readings_are_polled_in_coherent_memory(tmp_path):
 def test_one_thread_waits_for_the_queued_steps(tmp_path):
     """A result behind a long backlog takes one thread's CPU time, not every helper's."""
     run(BACKLOG, tmp_path)
+
+
+def test_small_results_wake_no_helpers(tmp_path):
+    run(SMALL, tmp_path)
