@@ -147,7 +147,7 @@ def test_export_argument_errors(gpu_available):
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 32, 32), (30, 30, 25), (64, 64, 63), (96, 120, 130)])
 def test_exports_of_every_size_reach_the_host_whole(gpu_available, shape):
     """The way to the host depends on the size: hipMemcpy up to 64 KB, one
-    pinned transfer, a transfer shared by helper threads from 256 KB, chunks of
+    pinned transfer, a transfer shared by helper threads from 640 KB, chunks of
     2 MB from 12 MB; FP64 moments, float32 fields and populations of a lattice
     and of an ensemble member of the same state agree at every size, also
     from two threads at once."""
@@ -183,3 +183,26 @@ def test_exports_of_every_size_reach_the_host_whole(gpu_available, shape):
             assert np.abs(got[0][1] - u).max() <= 19 * 2.0 ** -24 * 0.05
             for k, a in enumerate(got[0]):
                 np.testing.assert_array_equal(a, want.setdefault(k, a))
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (30, 30, 30), (64, 64, 63)])
+def test_exports_into_pinned_memory(gpu_available, shape):
+    """A destination the runtime has pinned takes its result in one transfer:
+    the same bytes as a pageable one, between untouched neighbours."""
+    ctypes = abi.ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+    case = W.taylor_green(shape)
+    n = int(np.prod(shape))
+    at = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(at), ctypes.c_size_t(8 * (4 * n + 20)), ctypes.c_uint(0)) == 0
+    out = np.ctypeslib.as_array(ctypes.cast(at, ctypes.POINTER(ctypes.c_double)), (4 * n + 20,))
+    out[:] = -7.0
+    with BlockLattice.from_case(case, "f32") as lat:
+        lat.ini_equilibrium(case.rho_u)
+        lat.collide_and_stream(3)
+        want = lat.moments().reshape(-1)
+        abi.check(abi.load().lbmh_moments(lat.handle, ctypes.c_void_p(at.value + 80)))
+    got = out.copy()
+    assert hip.hipHostFree(at) == 0
+    np.testing.assert_array_equal(got[10:-10], want)
+    assert (got[:10] == -7.0).all() and (got[-10:] == -7.0).all()

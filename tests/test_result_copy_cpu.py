@@ -218,6 +218,21 @@ int main() {
   CHECK(bring(host, kCopyHelped) == LBMH_OK && threads() == 6);
 """
 
+# a destination the runtime knows takes one transfer, straight into it
+PINNED = r"""
+int main() {
+  ResultPool::get().retain();
+  for (size_t n : {size_t(100) << 10, size_t(3) << 20, size_t(30) << 20}) {
+    std::vector<unsigned char> host(n);
+    registered[host.data()] = n;
+    copies.clear();
+    CHECK(bring(host, n) == LBMH_OK);  // assign() keeps the allocation
+    CHECK(copies.size() == 1 && copies[0].first == host.data() && copies[0].second == n);
+    registered.clear();
+  }
+  CHECK(host_flags.empty() && threads() == 1);
+"""
+
 TAIL = r"""
   std::printf("bad %d\n", bad);
   std::fflush(stdout);
@@ -255,3 +270,7 @@ def test_one_thread_waits_for_the_queued_steps(tmp_path):
 
 def test_small_results_wake_no_helpers(tmp_path):
     run(SMALL, tmp_path)
+
+
+def test_pinned_destinations_take_one_transfer(tmp_path):
+    run(PINNED, tmp_path)
