@@ -41,6 +41,7 @@
 #include "lbm_local.hpp"
 #include "lbm_storage.hpp"
 #include "lbmh_common.hpp"
+#include "result_copy.hpp"
 
 namespace lbmh {
 
@@ -284,7 +285,7 @@ int checkpoint_save_typed(const CheckpointBlock& b, uint8_t* out)
   const uint32_t n = b.n_padded;
   uint8_t* p = out;
   DeviceBuffer staging;
-  if (!std::is_same_v<S, T>) LBMH_HIP(hipMalloc(&staging.p, size_t(n) * sizeof(T)));
+  if (!std::is_same_v<S, T>) LBMH_HIP(device_alloc(&staging.p, size_t(n) * sizeof(T)));
   LBMH_HIP(hipDeviceSynchronize());
   for (int i = 0; i < b.q; ++i) {
     put<int64_t>(p, openlb_shift(b.shift[i], b.dist[i], n));
@@ -359,7 +360,7 @@ int checkpoint_load_typed(const CheckpointBlock& b, const uint8_t* in, int64_t* 
     }
   }
   DeviceBuffer staging;
-  if (!std::is_same_v<S, T>) LBMH_HIP(hipMalloc(&staging.p, size_t(n) * sizeof(T)));
+  if (!std::is_same_v<S, T>) LBMH_HIP(device_alloc(&staging.p, size_t(n) * sizeof(T)));
   LBMH_HIP(hipDeviceSynchronize());
   for (int i = 0; i < b.q; ++i) {
     S* col = static_cast<S*>(b.d_pop) + uint64_t(i) * b.stride;

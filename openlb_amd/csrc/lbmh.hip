@@ -401,14 +401,14 @@ int resolve_remote(lbmh_lattice* L)
         std::memcpy(init.data() + k * 4 * es, v, sizeof(v));
       }
     }
-    LBMH_HIP(hipMalloc(&L->d_remote, init.size()));
+    LBMH_HIP(device_alloc(&L->d_remote, init.size()));
     LBMH_HIP(hipMemcpy(L->d_remote, init.data(), init.size(), hipMemcpyHostToDevice));
   }
   for (lbmh_halo* H : L->halos_in) {
     for (int st = 0; st < kPostStages; ++st) {
       const auto& v = H->remote[st];
       if (v.empty()) continue;
-      LBMH_HIP(hipMalloc((void**)&H->d_remote[st], sizeof(RemotePair) * v.size()));
+      LBMH_HIP(device_alloc((void**)&H->d_remote[st], sizeof(RemotePair) * v.size()));
       LBMH_HIP(hipMemcpy(H->d_remote[st], v.data(), sizeof(RemotePair) * v.size(), hipMemcpyHostToDevice));
     }
   }
@@ -468,7 +468,7 @@ int launch_remote_stage(lbmh_lattice* runner, const std::vector<lbmh_lattice*>& 
     if (runner->d_remote_batch) LBMH_HIP(hipFree(runner->d_remote_batch));
     runner->d_remote_batch = nullptr;
     runner->remote_batch_bytes = 0;
-    LBMH_HIP(hipMalloc(&runner->d_remote_batch, bytes));
+    LBMH_HIP(device_alloc(&runner->d_remote_batch, bytes));
     runner->remote_batch_bytes = bytes;
   }
   LBMH_HIP(hipMemcpyAsync(runner->d_remote_batch, descs.data(), bytes, hipMemcpyHostToDevice, stream));
@@ -844,7 +844,7 @@ int split_steps(const std::vector<lbmh_lattice*>& blocks, const std::vector<lbmh
     if (lead->d_split) LBMH_HIP(hipFree(lead->d_split));
     lead->d_split = nullptr;
     lead->split_bytes = 0;
-    LBMH_HIP(hipMalloc(&lead->d_split, bytes));
+    LBMH_HIP(device_alloc(&lead->d_split, bytes));
     lead->split_bytes = bytes;
   }
   LBMH_HIP(hipMemcpyAsync(lead->d_split, t.bytes().data(), bytes, hipMemcpyHostToDevice, stream));
@@ -1063,11 +1063,11 @@ int lbmh_lattice_create(const lbmh_lattice_desc* desc, lbmh_lattice** out)
   DeviceGuard guard(L->device);
   const size_t pop_bytes = size_t(L->stride) * L->q * storage_size(L->storage);
   L->n_partials = 1024;
-  hipError_t e = hipMalloc(&L->d_pop, pop_bytes);
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_ids, L->ncore);
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_walls, sizeof(double) * 4 * kMaxWalls);
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_partials, sizeof(double) * 4 * (L->n_partials + 1));
-  if (e == hipSuccess) e = hipMalloc((void**)&L->d_info, sizeof(uint32_t) * (kMaxWalls + 1));
+  hipError_t e = device_alloc(&L->d_pop, pop_bytes);
+  if (e == hipSuccess) e = device_alloc((void**)&L->d_ids, L->ncore);
+  if (e == hipSuccess) e = device_alloc((void**)&L->d_walls, sizeof(double) * 4 * kMaxWalls);
+  if (e == hipSuccess) e = device_alloc((void**)&L->d_partials, sizeof(double) * 4 * (L->n_partials + 1));
+  if (e == hipSuccess) e = device_alloc((void**)&L->d_info, sizeof(uint32_t) * (kMaxWalls + 1));
   // the info table, and the count of finished workgroups of a statistics pass
   const std::vector<uint32_t> info_and_count(kMaxWalls + 1, 0u);
   if (e == hipSuccess) e = hipMemcpy(L->d_info, info_and_count.data(), sizeof(uint32_t) * (kMaxWalls + 1), hipMemcpyHostToDevice);
@@ -1179,7 +1179,7 @@ int lbmh_set_force_field(lbmh_lattice* L, const double* force)
   for (size_t k = 0; k < n; ++k)
     if (!std::isfinite(force[k])) return fail(LBMH_E_INVALID, "FORCE field holds a non-finite value");
   if (!L->d_force) {
-    LBMH_HIP(hipMalloc(&L->d_force, n * es));
+    LBMH_HIP(device_alloc(&L->d_force, n * es));
     L->footprint += n * es;
   }
   if (L->storage == LBMH_F64) {
@@ -1339,7 +1339,7 @@ int lbmh_set_local_boundary(lbmh_lattice* L, int id, int kind, double rho, const
       d = nullptr;
     }
     if (h.empty()) return LBMH_OK;
-    LBMH_HIP(hipMalloc((void**)&d, sizeof(uint32_t) * h.size()));
+    LBMH_HIP(device_alloc((void**)&d, sizeof(uint32_t) * h.size()));
     LBMH_HIP(hipMemcpy(d, h.data(), sizeof(uint32_t) * h.size(), hipMemcpyHostToDevice));
     return LBMH_OK;
   };
@@ -1356,7 +1356,7 @@ int lbmh_set_local_boundary(lbmh_lattice* L, int id, int kind, double rho, const
     }
     if (h.empty()) return LBMH_OK;
     const std::vector<PostCell> recs = post_records(L, h, kind);
-    LBMH_HIP(hipMalloc((void**)&d, sizeof(PostCell) * recs.size()));
+    LBMH_HIP(device_alloc((void**)&d, sizeof(PostCell) * recs.size()));
     LBMH_HIP(hipMemcpy(d, recs.data(), sizeof(PostCell) * recs.size(), hipMemcpyHostToDevice));
     return LBMH_OK;
   };
@@ -1373,7 +1373,7 @@ int lbmh_set_local_boundary(lbmh_lattice* L, int id, int kind, double rho, const
       L->d_scratch = nullptr;
     }
     const size_t elem = L->storage == LBMH_F64 ? sizeof(double) : sizeof(float);
-    LBMH_HIP(hipMalloc(&L->d_scratch, elem * L->q * L->h_planes.size()));
+    LBMH_HIP(device_alloc(&L->d_scratch, elem * L->q * L->h_planes.size()));
   }
   if (rc != LBMH_OK) return rc;
   L->has_local = true;
@@ -1404,7 +1404,7 @@ int lbmh_populations_upload(lbmh_lattice* L, const void* host, int host_dtype)
   DeviceGuard guard(L->device);
   const size_t bytes = size_t(L->q) * L->ncore * storage_size(host_dtype);
   DeviceBuffer staging;
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  LBMH_HIP(device_alloc(&staging.p, bytes));
   LBMH_HIP(hipMemcpy(staging.p, host, bytes, hipMemcpyHostToDevice));
   const CoreGeom g = core_geom(L);
   const uint32_t grid = grid_for(L->ncore, 256);
@@ -1518,7 +1518,7 @@ int lbmh_column_upload(lbmh_lattice* L, int i, const void* host, int64_t shift, 
         LBMH_HIP(hipMemcpy(col, dev.data(), size_t(n) * sizeof(T), hipMemcpyHostToDevice));
       } else {
         DeviceBuffer staging;
-        LBMH_HIP(hipMalloc(&staging.p, size_t(n) * sizeof(T)));
+        LBMH_HIP(device_alloc(&staging.p, size_t(n) * sizeof(T)));
         LBMH_HIP(hipMemcpy(staging.p, dev.data(), size_t(n) * sizeof(T), hipMemcpyHostToDevice));
         hipLaunchKernelGGL((column_import_kernel<S, T>), dim3(grid_for(uint32_t(n), 256)), dim3(256), 0, 0, col,
                            static_cast<const T*>(staging.p), uint32_t(n));
@@ -1553,7 +1553,7 @@ int lbmh_column_download(lbmh_lattice* L, int i, void* host, int64_t shift, int 
         LBMH_HIP(hipMemcpy(dev.data(), col, size_t(n) * sizeof(T), hipMemcpyDeviceToHost));
       } else {
         DeviceBuffer staging;
-        LBMH_HIP(hipMalloc(&staging.p, size_t(n) * sizeof(T)));
+        LBMH_HIP(device_alloc(&staging.p, size_t(n) * sizeof(T)));
         hipLaunchKernelGGL((column_export_kernel<S, T>), dim3(grid_for(uint32_t(n), 256)), dim3(256), 0, 0,
                            static_cast<T*>(staging.p), col, uint32_t(n));
         LBMH_HIP(hipGetLastError());
@@ -1589,7 +1589,7 @@ int lbmh_ini_equilibrium(lbmh_lattice* L, const double* rho_u)
   DeviceGuard guard(L->device);
   const size_t bytes = size_t(4) * L->ncore * sizeof(double);
   DeviceBuffer staging;
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  LBMH_HIP(device_alloc(&staging.p, bytes));
   LBMH_HIP(hipMemcpy(staging.p, rho_u, bytes, hipMemcpyHostToDevice));
   const CoreGeom g = core_geom(L);
   const uint32_t grid = grid_for(L->ncore, 256);
@@ -1689,7 +1689,7 @@ int lbmh_halo_create(lbmh_lattice* dst, const lbmh_lattice* src, const uint32_t*
   const_cast<lbmh_lattice*>(src)->halos_out.push_back(H);
   DeviceGuard guard(dst->device);
   if (n) {
-    hipError_t e = hipMalloc((void**)&H->d_pairs, sizeof(uint2) * n);
+    hipError_t e = device_alloc((void**)&H->d_pairs, sizeof(uint2) * n);
     if (e == hipSuccess) e = hipMemcpy(H->d_pairs, pairs.data(), sizeof(uint2) * n, hipMemcpyHostToDevice);
     if (e != hipSuccess) {
       const int rc = hip_fail(e, "lbmh_halo_create");
@@ -1802,7 +1802,7 @@ int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream)
       if (owner->d_halo_batch) LBMH_HIP(hipFree(owner->d_halo_batch));
       owner->d_halo_batch = nullptr;
       owner->halo_batch_bytes = 0;
-      LBMH_HIP(hipMalloc(&owner->d_halo_batch, bytes));
+      LBMH_HIP(device_alloc(&owner->d_halo_batch, bytes));
       owner->halo_batch_bytes = bytes;
     }
     LBMH_HIP(hipMemcpyAsync(owner->d_halo_batch, descs.data(), bytes, hipMemcpyHostToDevice, s));

@@ -484,18 +484,18 @@ int lbmh_ensemble_create(const lbmh_ensemble_desc* d, lbmh_ensemble** out)
   E->id_arena = Arena(align_up(d->cell_capacity) + kAlign * size_t(E->max_members));
   E->chunk_capacity = uint32_t(d->cell_capacity / kBlock + size_t(E->max_members) + 1);
   DeviceGuard guard(E->device);
-  hipError_t e = hipMalloc(&E->d_pop, E->pop_arena.capacity());
-  if (e == hipSuccess) e = hipMalloc((void**)&E->d_ids, E->id_arena.capacity());
-  if (e == hipSuccess) e = hipMalloc((void**)&E->d_walls, sizeof(double) * 4 * kEnsembleWalls * E->max_members);
+  hipError_t e = device_alloc(&E->d_pop, E->pop_arena.capacity());
+  if (e == hipSuccess) e = device_alloc((void**)&E->d_ids, E->id_arena.capacity());
+  if (e == hipSuccess) e = device_alloc((void**)&E->d_walls, sizeof(double) * 4 * kEnsembleWalls * E->max_members);
   const size_t state_at = align_up(E->h_table.size()), table_bytes = state_at + 2 * E->h_state.size();
-  if (e == hipSuccess) e = hipMalloc(&E->d_table, table_bytes);
+  if (e == hipSuccess) e = device_alloc(&E->d_table, table_bytes);
   E->d_state = static_cast<char*>(E->d_table) + state_at;
-  if (e == hipSuccess) e = hipMalloc((void**)&E->d_chunk, sizeof(uint32_t) * E->chunk_capacity);
+  if (e == hipSuccess) e = device_alloc((void**)&E->d_chunk, sizeof(uint32_t) * E->chunk_capacity);
   E->boundary_capacity = d->boundary_capacity ? d->boundary_capacity : d->cell_capacity / 4 + 64;
-  if (e == hipSuccess) e = hipMalloc((void**)&E->d_info, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
+  if (e == hipSuccess) e = device_alloc((void**)&E->d_info, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
   if (e == hipSuccess) e = hipMemset(E->d_info, 0, sizeof(uint32_t) * kEnsembleWalls * E->max_members);
   for (uint2** list : {&E->d_local, &E->d_edges, &E->d_corners, &E->d_planes, &E->d_pplanes})
-    if (e == hipSuccess) e = hipMalloc((void**)list, sizeof(uint2) * E->boundary_capacity);
+    if (e == hipSuccess) e = device_alloc((void**)list, sizeof(uint2) * E->boundary_capacity);
   if (e == hipSuccess) e = hipMemset(E->d_table, 0, table_bytes);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&E->capture_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -748,7 +748,7 @@ int lbmh_ensemble_set_local_boundary(lbmh_ensemble* E, int m, int id, int kind, 
   LBMH_HIP(hipDeviceSynchronize());
   if (kind == LBMH_INTERP_PRESSURE && !planes.empty() && !E->d_plane_scratch) {
     const size_t elem = E->storage == LBMH_F64 ? sizeof(double) : sizeof(float);
-    LBMH_HIP(hipMalloc(&E->d_plane_scratch, elem * size_t(E->q) * E->boundary_capacity));
+    LBMH_HIP(device_alloc(&E->d_plane_scratch, elem * size_t(E->q) * E->boundary_capacity));
   }
   if (kind == LBMH_INTERP_PRESSURE && !planes.empty()) mem.pressure_planes = true;
   for (const auto& kv : entry_ids) {
@@ -849,7 +849,7 @@ int lbmh_ensemble_ini_equilibrium(lbmh_ensemble* E, int m, const double* rho_u)
   const Member& mem = E->members[m];
   DeviceBuffer staging;
   const size_t bytes = size_t(4) * mem.ncore * sizeof(double);
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  LBMH_HIP(device_alloc(&staging.p, bytes));
   LBMH_HIP(hipMemcpy(staging.p, rho_u, bytes, hipMemcpyHostToDevice));
   const int forced = (E->kind == LBMH_FORCED_BGK || E->kind == LBMH_FORCED_TRT) ? 1 : 0;
   rc = with_types(E, [&](auto qc, auto s) -> int {
@@ -881,7 +881,7 @@ int lbmh_ensemble_upload(lbmh_ensemble* E, int m, const void* host, int dtype)
   const Member& mem = E->members[m];
   DeviceBuffer staging;
   const size_t bytes = size_t(E->q) * mem.ncore * storage_size(dtype);
-  LBMH_HIP(hipMalloc(&staging.p, bytes));
+  LBMH_HIP(device_alloc(&staging.p, bytes));
   LBMH_HIP(hipMemcpy(staging.p, host, bytes, hipMemcpyHostToDevice));
   rc = with_types(E, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
@@ -1208,11 +1208,11 @@ int lbmh_ensemble_autotune(lbmh_ensemble* E, int trial_steps, lbmh_launch_config
   const size_t state_bytes = E->h_state.size();
   LBMH_HIP(hipDeviceSynchronize());
   if (end) {
-    const hipError_t e = hipMalloc(&sc.pop, end);
+    const hipError_t e = device_alloc(&sc.pop, end);
     if (e != hipSuccess) return fail(LBMH_E_MEMORY, "autotune needs device memory for a copy of the members' populations");
     LBMH_HIP(hipMemcpy(sc.pop, E->d_pop, end, hipMemcpyDeviceToDevice));
   }
-  LBMH_HIP(hipMalloc(&sc.state, state_bytes));
+  LBMH_HIP(device_alloc(&sc.state, state_bytes));
   LBMH_HIP(hipMemcpy(sc.state, E->d_state, state_bytes, hipMemcpyDeviceToDevice));
   LBMH_HIP(hipEventCreate(&sc.e0));
   LBMH_HIP(hipEventCreate(&sc.e1));

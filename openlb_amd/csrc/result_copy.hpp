@@ -180,6 +180,20 @@ struct ResultPool {
   }
 };
 
+// hipMalloc that gives the idle workspace back where the card has no room
+// otherwise: what an export leaves allocated refuses no later call.
+inline hipError_t device_alloc(void** p, size_t bytes)
+{
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  ResultPool& pool = ResultPool::get();
+  std::unique_lock<std::mutex> l(pool.lease, std::try_to_lock);
+  if (!l.owns_lock() || !pool.device) return e;
+  (void)hipGetLastError();
+  pool.drop_workspace();
+  return hipMalloc(p, bytes);
+}
+
 // Device memory for one export, and its way to the host.
 class ResultBuffer {
  public:
@@ -202,7 +216,13 @@ class ResultBuffer {
         size_t size = kCopyDirect;  // doubled up to what is needed
         while (size < bytes) size *= 2;
         void* fresh = nullptr;
-        LBMH_HIP(hipMalloc(&fresh, size));
+        hipError_t e = hipMalloc(&fresh, size);
+        if (e == hipErrorOutOfMemory && size > bytes) {  // a full card: no more than needed
+          (void)hipGetLastError();
+          size = bytes;
+          e = hipMalloc(&fresh, size);
+        }
+        if (e != hipSuccess) return hip_fail(e, "hipMalloc");
         pool.device = fresh;
         pool.device_bytes = size;
         pool.ordinal = ordinal;
@@ -210,7 +230,13 @@ class ResultBuffer {
       p = pool.device;
       return LBMH_OK;
     }
-    LBMH_HIP(hipMalloc(&own_, bytes));
+    hipError_t e = hipMalloc(&own_, bytes);
+    if (e == hipErrorOutOfMemory && lock_.owns_lock() && pool.device) {
+      (void)hipGetLastError();
+      pool.drop_workspace();
+      e = hipMalloc(&own_, bytes);
+    }
+    if (e != hipSuccess) return hip_fail(e, "hipMalloc");
     p = own_;
     return LBMH_OK;
   }

@@ -233,6 +233,35 @@ int main() {
   CHECK(host_flags.empty() && threads() == 1);
 """
 
+# a card with little room left refuses nothing for what earlier results left allocated
+FULL = r"""
+int main() {
+  constexpr size_t MB = size_t(1) << 20;
+  ResultPool::get().retain();
+  std::vector<unsigned char> host;
+  void* a = nullptr;
+  void* b = nullptr;
+  device_limit = 100 * MB;
+  CHECK(device_alloc(&a, 97 * MB) == hipSuccess);
+  CHECK(bring(host, 5 * MB / 2) == LBMH_OK);  // 4 MB would not fit
+  CHECK(hipFree(a) == hipSuccess);
+  CHECK(bring(host, 60 * MB) == LBMH_OK);
+  CHECK(device_used == 64 * MB);
+  CHECK(bring(host, 80 * MB) == LBMH_OK);     // needs the workspace's room
+  CHECK(bring(host, 60 * MB) == LBMH_OK);
+  CHECK(device_alloc(&a, 90 * MB) == hipSuccess && device_used == 90 * MB);
+  CHECK(bring(host, 30 * MB) != LBMH_OK && device_alloc(&b, 30 * MB) == hipErrorOutOfMemory);
+  CHECK(bring(host, 10 * MB) == LBMH_OK);
+  {
+    // another thread's export holds the lease: its workspace stays
+    ResultBuffer out;
+    CHECK(out.allocate(0, 8 * MB) == LBMH_OK);
+    std::thread other([&] { CHECK(device_alloc(&b, 30 * MB) == hipErrorOutOfMemory); });
+    other.join();
+    CHECK(device_blocks.count(out.p));
+  }
+"""
+
 TAIL = r"""
   std::printf("bad %d\n", bad);
   std::fflush(stdout);
@@ -274,3 +303,7 @@ def test_small_results_wake_no_helpers(tmp_path):
 
 def test_pinned_destinations_take_one_transfer(tmp_path):
     run(PINNED, tmp_path)
+
+
+def test_kept_workspace_refuses_no_later_call(tmp_path):
+    run(FULL, tmp_path)
