@@ -176,7 +176,9 @@ int lbmh_halo_copy(lbmh_halo* halo, void* stream);
  * src/communication/superCommunicator.hh:189-218).  The halos must share
  * device, q and storage; the batch's descriptor table is kept by the first
  * halo's destination block, so batches led by one block must run on one
- * stream. */
+ * stream.  The table is sent from the host in each call: a stream that is being
+ * captured is refused (LBMH_E_STATE), as for the steps of joined blocks with
+ * post-processors that read each other's cells. */
 int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream);
 
 /* n_steps time steps of all blocks of a split lattice: per step the collision
@@ -185,9 +187,13 @@ int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream);
  * collideAndStream, src/core/superLattice.hh:601-663): lbmh_collide of every
  * block, lbmh_halo_copy_many and lbmh_stream of every block, bit for bit.
  * Blocks that share device, q, storage, bulk kind and step count, listed
- * together with every block their halos join them to, run each phase in one
- * launch; others one launch per block.  The tables of the call are kept by
- * the first block, so calls led by one block must run on one stream. */
+ * together with every block their halos join them to, run the collision, the
+ * copies and the edge and corner processors in one launch each; cells that
+ * collide from a list (inner edges and corners) and plane processors take a
+ * launch per block, and so does everything for other blocks.  The tables of the
+ * call are built in it, sent from the host and kept by the first block: calls
+ * led by one block must run on one stream, and a stream that is being captured
+ * is refused (LBMH_E_STATE). */
 int lbmh_split_step(lbmh_lattice* const* lattices, size_t n_lattices, lbmh_halo* const* halos, size_t n_halos,
                     int64_t n_steps, void* stream);
 

@@ -204,6 +204,18 @@ int settle(const lbmh_lattice* L)
   return LBMH_OK;
 }
 
+// Calls that send tables of theirs to the device refuse a stream that is being
+// captured: the graph would keep the address of host memory that is gone when
+// the call returns, and shifts that have moved on by its replay.
+int refuse_capture(hipStream_t stream, const char* call)
+{
+  if (!stream || stream == hipStreamLegacy) return LBMH_OK;  // cannot be captured
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  LBMH_HIP(hipStreamIsCapturing(stream, &status));
+  if (status == hipStreamCaptureStatusNone) return LBMH_OK;
+  return fail(LBMH_E_STATE, std::string(call) + " cannot be captured: it sends tables from the host");
+}
+
 CoreGeom core_geom(const lbmh_lattice* L)
 {
   CoreGeom g;
@@ -463,6 +475,8 @@ int launch_remote_stage(lbmh_lattice* runner, const std::vector<lbmh_lattice*>& 
     }
   }
   if (descs.empty()) return LBMH_OK;
+  const int rc = refuse_capture(stream, "a step of joined blocks with post-processors");
+  if (rc != LBMH_OK) return rc;
   const size_t bytes = sizeof(RemoteBatchDesc<Q>) * descs.size();
   if (runner->remote_batch_bytes < bytes) {
     if (runner->d_remote_batch) LBMH_HIP(hipFree(runner->d_remote_batch));
@@ -1764,6 +1778,8 @@ int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream)
   lbmh_lattice* owner = halos[0]->dst;
   DeviceGuard guard(owner->device);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int rc = refuse_capture(s, "lbmh_halo_copy_many");
+  if (rc != LBMH_OK) return rc;
   for (size_t h = 0; h < n; ++h) {
     on_stream(halos[h]->dst, s);
     on_stream(halos[h]->src, s);
@@ -1846,8 +1862,10 @@ int lbmh_split_step(lbmh_lattice* const* lattices, size_t n_lattices, lbmh_halo*
     for (const lbmh_halo* H : X->halos_in) tables = tables && known(H->src);
     for (const lbmh_halo* H : X->halos_out) tables = tables && (!H->dst || !has_post(H->dst) || known(H->dst));
   }
+  if (n_steps == 0) return LBMH_OK;
+  const int captured = refuse_capture(static_cast<hipStream_t>(stream), "lbmh_split_step");
+  if (captured != LBMH_OK) return captured;
   if (tables) {
-    if (n_steps == 0) return LBMH_OK;
     DeviceGuard guard(blocks[0]->device);
     return with_types(blocks[0], [&](auto qc, auto t) -> int {
       return split_steps<decltype(qc)::value, decltype(t)>(blocks, joins, n_steps, static_cast<hipStream_t>(stream));

@@ -10,6 +10,7 @@ itself computes on the same cuboids (tests/golden/multiblock/, OpenLB run with
 CuboidDecomposition::splitRegular: the overlap exchange of
 src/communication/superCommunicator.hh:189-218 with periodic images resolved
 through src/geometry/cuboidDecomposition.hh:155-177)."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -383,3 +384,49 @@ def test_split_step_matches_the_single_phases(gpu_available, name, blocks):
             assert all(lat.step_count() == 8 for lat in sup.blocks.values())
             out.append([lat.checkpoint("f32") for lat in sup.blocks.values()])
     assert out[0] == out[1]
+
+
+def test_calls_that_send_tables_refuse_a_capture(gpu_available):
+    """lbmh_split_step, lbmh_halo_copy_many and the steps of joined blocks with
+    post-processors send tables from host memory that is gone when they return:
+    a stream that is being captured is refused, and nothing has changed where
+    nothing had been launched."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def call(name, *args):
+        assert getattr(hip, name)(*args) == 0, name
+
+    def refused(rc):
+        assert rc == abi.E_STATE and "capture" in L.lbmh_last_error().decode()
+
+    L = abi.load()
+    case = W.local_velocity_cavity((12, 13, 14), tau=0.7, lid_u=0.06)
+    stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+    call("hipStreamCreateWithFlags", ctypes.byref(stream), 1)
+    out = []
+    for capture in (True, False):
+        with SuperLattice(case, "f32", (2, 1, 2)) as sup:
+            sup.ini_equilibrium(case.rho_u)
+            sup.initialize()
+            sup.collide_and_stream(2)
+            sup.synchronize()  # the calls that this block leads move to another stream
+            handles = (ctypes.c_void_p * len(sup.blocks))(*[lat.handle.value for lat in sup.blocks.values()])
+            if capture:
+                call("hipStreamBeginCapture", stream, 1)
+                refused(L.lbmh_split_step(handles, len(handles), sup._halo_table, len(sup.halos), 3, stream))
+                refused(L.lbmh_halo_copy_many(sup._halo_table, len(sup.halos), stream))
+                call("hipStreamEndCapture", stream, ctypes.byref(graph))
+                call("hipGraphDestroy", graph)
+            abi.check(L.lbmh_split_step(handles, len(handles), sup._halo_table, len(sup.halos), 3, stream))
+            out.append(sup.download_populations("f32"))
+            if capture:
+                # the phases: the collisions are captured, the last block's streaming is refused
+                call("hipStreamSynchronize", stream)
+                call("hipStreamBeginCapture", stream, 1)
+                for lat in sup.blocks.values():
+                    abi.check(L.lbmh_collide(lat.handle, stream))
+                refused([L.lbmh_stream(lat.handle, stream) for lat in sup.blocks.values()][-1])
+                call("hipStreamEndCapture", stream, ctypes.byref(graph))
+                call("hipGraphDestroy", graph)
+    call("hipStreamDestroy", stream)
+    np.testing.assert_array_equal(out[0], out[1])
