@@ -10,6 +10,23 @@
 
 namespace lbmh {
 
+// The collision of a split lattice, all blocks in one launch: by what the blocks
+// hold together, and without a cap on the resident workgroups if any block has
+// local boundaries, as flat faces are then collided in the same pass.  FP32,
+// uncapped against a 40 KB reservation, us per step: 128^3 in 8 blocks (159 MB)
+// 85.0 and 86.3, 184^3 in 8 (473 MB) 258.8 and 254.9, 256^3 in 64 (1275 MB) 935
+// and 918; FP64, against 48 KB: 128^3 in 8 (319 MB) 149.2 and 145.6, 184^3 in 32
+// (947 MB) 687 and 674; FP16 128^3 (80 MB) 59.3 and 66.7; LocalVelocity cavity
+// 161^3 in 8, FP32, 208 and 239.  The line is the Infinity Cache's size.  XCD
+// groups as in an ensemble.
+inline lbmh_launch_config split_launch(int storage, bool local, uint64_t bytes)
+{
+  lbmh_launch_config c{0, 32};
+  if (storage == LBMH_F16 || local || bytes < 256000000u) return c;
+  c.lds_bytes = storage == LBMH_F64 ? 49152 : 40960;
+  return c;
+}
+
 // The XCD group a pass of `chunks` chunks runs with (chunk_of_block): a window
 // of 8 x group chunks that the pass does not fill leaves every chunk in
 // dispatch order, whatever the group.

@@ -873,9 +873,9 @@ int split_steps(const std::vector<lbmh_lattice*>& blocks, const std::vector<lbmh
   step.chunk_block = reinterpret_cast<const uint32_t*>(base + at_chunks);
   step.chunks = uint32_t(chunk_block.size());
   step.blocks = uint32_t(blocks.size());
-  // XCD groups as in an ensemble, unless a shape was chosen for the lead block
-  step.launch = lead->launch;
-  if (!lead->launch_chosen) step.launch.xcd_group = 32;
+  uint64_t held = 0;
+  for (const lbmh_lattice* X : blocks) held += X->stride * uint64_t(Q) * sizeof(S);
+  step.launch = lead->launch_chosen ? lead->launch : split_launch(lead->storage, local, held);
 
   for (int64_t k = 0; k < n_steps; ++k) {
     const uint32_t cur = uint32_t(k & 1);

@@ -56,6 +56,25 @@ int main() {
 }
 """
 
+SPLIT = HEAD + r"""
+int main() {
+  const uint64_t MB = 1000000;
+  // eight FP32 blocks of 60 MB fill 480 MB together, as one of 480 MB does
+  CHECK(split_launch(LBMH_F32, false, 8 * 60 * MB).lds_bytes == 40960);
+  CHECK(split_launch(LBMH_F64, false, 8 * 40 * MB).lds_bytes == 49152);
+  CHECK(split_launch(LBMH_F32, false, 2 * 80 * MB).lds_bytes == 0);
+  for (uint64_t mb : {1, 159, 255, 256, 317, 2000})
+    for (int storage : {LBMH_F64, LBMH_F32, LBMH_F16})
+      for (bool local : {false, true}) {
+        const lbmh_launch_config c = split_launch(storage, local, mb * MB);
+        CHECK(c.xcd_group == 32);
+        CHECK((c.lds_bytes == 0) == (local || storage == LBMH_F16 || mb < 256));
+      }
+  std::printf("bad %d\n", bad);
+  return bad != 0;
+}
+"""
+
 
 def run(program, tmp_path):
     src, exe = tmp_path / "check.cpp", tmp_path / "check"
@@ -70,3 +89,9 @@ def test_autotuners_time_the_shape_in_use_and_the_default(tmp_path):
     """Each autotuner times the shape in use and the default beside its grid, no
     mapping twice, and leaves the shape in use unless another is faster twice."""
     run(TUNING, tmp_path)
+
+
+def test_split_launch_follows_what_all_blocks_hold(tmp_path):
+    """Not the first block's size and boundaries: a reservation once the blocks
+    together outgrow the Infinity Cache, none if any has local boundaries."""
+    run(SPLIT, tmp_path)
