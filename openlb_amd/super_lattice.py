@@ -81,7 +81,6 @@ class SuperLattice:
             self.blocks[key] = BlockLattice.from_case(sub, storage, device, overlap_ids=ring)
             self.origin[key] = lo
         self._build_halos(self_periodic)
-        self._block_table = (ctypes.c_void_p * len(self.blocks))(*[lat.handle.value for lat in self.blocks.values()])
         self._halo_table = (ctypes.c_void_p * max(1, len(self.halos)))(*[h.value for h in self.halos])
 
     # -- decomposition ---------------------------------------------------------
@@ -145,8 +144,9 @@ class SuperLattice:
     def collide_and_stream(self, steps: int = 1):
         if steps < 1 or not self.blocks:
             return
-        abi.check(abi.load().lbmh_split_step(self._block_table, len(self.blocks), self._halo_table, len(self.halos),
-                                             int(steps), None))
+        # the handles as they are now: a block that was closed is refused as null
+        table = (ctypes.c_void_p * len(self.blocks))(*[lat.handle for lat in self.blocks.values()])
+        abi.check(abi.load().lbmh_split_step(table, len(table), self._halo_table, len(self.halos), int(steps), None))
 
     def initialize(self):
         """SuperLattice::initialize(): every block's post-processors once on the

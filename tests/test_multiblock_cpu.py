@@ -15,6 +15,9 @@ single-block pin (tests/test_oracle_golden.py): 1e-12 of max |f_i| for FP64,
 The division itself is checked against Cuboid::divide's rule (the sizes of the
 split, src/geometry/cuboid.hh:184-211), which SuperLattice in
 openlb_amd/super_lattice.py restates."""
+import ctypes
+import itertools
+
 import numpy as np
 import pytest
 
@@ -204,3 +207,88 @@ def test_openlb_resumes_from_library_split_checkpoint(name):
     err = G.rel_error(got, arrays[f"f_{m}"].astype(np.float64), case.q, flow)
     print(f"OpenLB resumed from the library's step-{start} split checkpoint of {name}: rel {err:.2e}", flush=True)
     assert err <= TOL[real], err
+
+
+class FakeLibrary:
+    """Records lbmh_halo_create's lists and lbmh_split_step's handles."""
+
+    def __init__(self):
+        self.halos, self.stepped = [], []
+
+    def lbmh_halo_create(self, dst, src, dst_cells, src_cells, n, out):
+        lists = [np.ctypeslib.as_array((ctypes.c_uint32 * n).from_address(p.value)).copy() for p in (dst_cells, src_cells)]
+        self.halos.append((dst.value, src.value, *lists))
+        out._obj.value = 1000 + len(self.halos)
+        return 0
+
+    def lbmh_halo_destroy(self, halo):
+        return 0
+
+    def lbmh_split_step(self, lattices, n, halos, m, steps, stream):
+        self.stepped.append((list(lattices), m, steps))
+        return 0 if all(lattices) else -1
+
+    def lbmh_last_error(self):
+        return b"null lattice"
+
+
+class FakeBlock:
+    def __init__(self, case, number):
+        self.shape, self.handle = tuple(case.shape), ctypes.c_void_p(number)
+
+    def close(self):
+        self.handle = None
+
+
+def fake_super_lattice(monkeypatch, case, blocks):
+    from openlb_amd import super_lattice as SL
+    library, count = FakeLibrary(), itertools.count(1)
+    monkeypatch.setattr(SL.abi, "load", lambda: library)
+    monkeypatch.setattr(SL.abi, "_lib", library)
+    monkeypatch.setattr(SL.BlockLattice, "from_case", lambda sub, *a, **k: FakeBlock(sub, next(count)))
+    return SL.SuperLattice(case, "f32", blocks), library
+
+
+def test_a_closed_block_is_refused(monkeypatch):
+    """collide_and_stream hands over the blocks' handles as they are: a block
+    that was closed in the meantime goes in as null, which the library refuses."""
+    from openlb_amd import abi
+    from openlb_amd import workloads as W
+    sup, library = fake_super_lattice(monkeypatch, W.taylor_green((6, 5, 4)), (2, 1, 1))
+    sup.collide_and_stream(3)
+    assert library.stepped == [([1, 2], len(sup.halos), 3)]
+    sup.blocks[(1, 0, 0)].close()
+    with pytest.raises(abi.LbmhError):
+        sup.collide_and_stream()
+    assert library.stepped[-1][0] == [1, None]
+
+
+@pytest.mark.parametrize("case,blocks", [("periodic", (2, 2, 2)), ("periodic", (3, 1, 2)), ("channel", (2, 2, 1)),
+                                         ("cavity", (2, 2, 2))])
+def test_halo_lists_hold_the_pieces_overlap_rule(monkeypatch, case, blocks):
+    """lbmh_split_field_export fills a piece's overlap points from the halos'
+    lists, bulk sources only: the points and sources of piece_sources, which
+    OpenLB's files pin above."""
+    from openlb_amd import workloads as W
+    from openlb_amd.super_lattice import piece_sources
+    case = {"periodic": lambda: W.taylor_green((7, 6, 5)), "cavity": lambda: W.lid_driven_cavity((7, 8, 6), tau=0.6),
+            "channel": lambda: W.velocity_channel((8, 7, 6), u_in=0.04)}[case]()
+    sup, library = fake_super_lattice(monkeypatch, case, blocks)
+    keys = {lat.handle.value: key for key, lat in sup.blocks.items()}
+    for key in sup.blocks:
+        want, got = {}, {}
+        for src, (points, sources) in piece_sources(case, sup.ranges, key).items():
+            want[src] = set(zip(points.tolist(), sources.tolist()))
+        n = sup.blocks[key].shape
+        for dst, src, dst_cells, src_cells in library.halos:
+            if keys[dst] != key:
+                continue
+            sk = keys[src]
+            sn, lo = sup.blocks[sk].shape, sup.origin[sk]
+            for d, s in zip(dst_cells.tolist(), src_cells.tolist()):
+                x, y, z = np.unravel_index(d, [k + 2 for k in n])
+                cx, cy, cz = (int(v) - 1 for v in np.unravel_index(s, [k + 2 for k in sn]))
+                if case.ids[lo[0] + cx, lo[1] + cy, lo[2] + cz] == 1:
+                    point = (int(z) * (n[1] + 2) + int(y)) * (n[0] + 2) + int(x)
+                    got.setdefault(sk, set()).add((point, (cz * sn[1] + cy) * sn[0] + cx))
+        assert got == want
