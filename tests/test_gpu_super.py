@@ -430,3 +430,140 @@ def test_calls_that_send_tables_refuse_a_capture(gpu_available):
                 call("hipGraphDestroy", graph)
     call("hipStreamDestroy", stream)
     np.testing.assert_array_equal(out[0], out[1])
+
+
+def _phases(sup, steps, stream=None):
+    L = abi.load()
+    for _ in range(steps):
+        for lat in sup.blocks.values():
+            abi.check(L.lbmh_collide(lat.handle, stream))
+        if sup.halos:
+            abi.check(L.lbmh_halo_copy_many(sup._halo_table, len(sup.halos), stream))
+        for lat in sup.blocks.values():
+            abi.check(L.lbmh_stream(lat.handle, stream))
+
+
+def _split(sup, steps, stream=None):
+    handles = (ctypes.c_void_p * len(sup.blocks))(*[lat.handle.value for lat in sup.blocks.values()])
+    abi.check(abi.load().lbmh_split_step(handles, len(handles), sup._halo_table, len(sup.halos), steps, stream))
+
+
+@pytest.mark.parametrize("case,blocks", [("periodic", (2, 1, 1)), ("cavity_local", (2, 2, 1))])
+def test_split_step_over_whole_windows_and_a_rest(gpu_available, case, blocks):
+    """With XCD groups of 1 a window is 8 chunks: the blocks' launch holds whole
+    windows, which odd steps run backwards, and a rest in dispatch order."""
+    case = {"periodic": lambda: W.random_periodic((20, 19, 18), seed=5),
+            "cavity_local": lambda: W.local_velocity_cavity((21, 19, 18), tau=0.7, lid_u=0.06)}[case]()
+    out = []
+    for run in (_split, _phases):
+        with SuperLattice(case, "f32", blocks) as sup:
+            chunks = sum(-(-lat.ncore // 256) for lat in sup.blocks.values())
+            assert chunks > 16 and chunks % 8
+            sup.ini_equilibrium(case.rho_u)
+            sup.initialize()
+            next(iter(sup.blocks.values())).set_launch_config(0, 1)
+            for steps in (1, 2, 3):
+                run(sup, steps)
+            out.append([lat.checkpoint("f32") for lat in sup.blocks.values()])
+    assert out[0] == out[1]
+
+
+def test_split_step_of_blocks_that_share_no_tables(gpu_available):
+    """Blocks of another bulk kind, of another step count, or joined to a block
+    that is not listed take the single phases instead."""
+    L = abi.load()
+
+    def make(kind, seed):
+        case = W.random_periodic((9, 8, 13), seed=seed)
+        case.kind = kind
+        lat = BlockLattice.from_case(case, "f32")
+        lat.ini_equilibrium(case.rho_u)
+        return lat
+
+    def split(lats, steps):
+        t = (ctypes.c_void_p * len(lats))(*[lat.handle.value for lat in lats])
+        abi.check(L.lbmh_split_step(t, len(t), None, 0, steps, None))
+
+    for kinds, ahead in ((("bgk", "trt"), 0), (("bgk", "bgk"), 3)):
+        got, want = ([make(k, i) for i, k in enumerate(kinds)] for _ in range(2))
+        got[0].collide_and_stream(ahead)
+        want[0].collide_and_stream(ahead)
+        split(got, 5)
+        for a, b in zip(got, want):
+            b.collide_and_stream(5)
+            assert a.step_count() == b.step_count()
+            np.testing.assert_array_equal(a.download_populations("f32"), b.download_populations("f32"))
+            a.close()
+            b.close()
+
+    case = W.random_periodic((12, 9, 10), seed=8)
+    out = []
+    for tables in (True, False):
+        with SuperLattice(case, "f32", (2, 1, 1)) as sup:
+            sup.ini_equilibrium(case.rho_u)
+            a, b = sup.blocks.values()
+            halos = (ctypes.c_void_p * 1)(sup.halos[0].value)  # into the first block, from the second
+            for _ in range(3):
+                if tables:
+                    one = (ctypes.c_void_p * 1)(a.handle.value)
+                    abi.check(L.lbmh_split_step(one, 1, halos, 1, 1, None))
+                else:
+                    abi.check(L.lbmh_collide(a.handle, None))
+                    abi.check(L.lbmh_halo_copy_many(halos, 1, None))
+                    abi.check(L.lbmh_stream(a.handle, None))
+                b.collide_and_stream()
+            out.append([a.checkpoint("f32"), b.checkpoint("f32")])
+    assert out[0] == out[1]
+
+
+@pytest.mark.parametrize("route", ["step", "halo", "phases", "split"])
+def test_evaluations_wait_for_work_on_another_stream(gpu_available, route):
+    """Evaluations run on the null stream: behind a backlog on a stream that
+    does not wait for it they give what the same steps on the null stream give,
+    for every way to step and every evaluation, bit for bit."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    case = W.local_velocity_cavity((60, 40, 50), tau=0.7, lid_u=0.06) if route != "halo" else W.taylor_green((60, 40, 50))
+    blocks = (1, 1, 1) if route == "step" else (2, 1, 1)
+    stream = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(stream), 1) == 0
+    results = []
+    for on in (None, stream):
+        with SuperLattice(case, "f32", blocks) as sup:
+            sup.ini_equilibrium(case.rho_u)
+            sup.initialize()
+            sup.synchronize()
+            lats = list(sup.blocks.values())
+
+            def advance(steps):
+                if route == "step":
+                    lats[0].collide_and_stream(steps, stream=on.value if on else None)
+                elif route == "phases":
+                    _phases(sup, steps, on)
+                elif route == "split":
+                    _split(sup, steps, on)
+                else:
+                    L = abi.load()
+                    for _ in range(steps):
+                        for lat in lats:
+                            abi.check(L.lbmh_collide(lat.handle, on))
+                        for h in sup.halos:
+                            abi.check(L.lbmh_halo_copy(h, on))
+                        for lat in lats:
+                            abi.check(L.lbmh_stream(lat.handle, on))
+
+            got = []
+            for read in (lambda lat, key: list(lat.statistics().values()),
+                         lambda lat, key: lat.moments(),
+                         lambda lat, key: sup.field_export(key, 1, 1),
+                         lambda lat, key: sup.field_export(key, 0, 0),
+                         lambda lat, key: lat.download_populations("f32"),
+                         lambda lat, key: lat.reduce_moments(),
+                         lambda lat, key: lat.reduce_field("density", "sum")[0],
+                         lambda lat, key: np.frombuffer(lat.checkpoint("f32"), dtype=np.uint8)):
+                advance(150)
+                # the last block first: it has only been touched by the calls above
+                got += [np.asarray(read(lat, key)) for key, lat in reversed(sup.blocks.items())]
+            results.append(got)
+    assert hip.hipStreamDestroy(stream) == 0
+    for a, b in zip(*results):
+        np.testing.assert_array_equal(a, b)
