@@ -133,8 +133,8 @@ static __global__ __launch_bounds__(kBlock) void ensemble_settle_kernel(uint32_t
   if (k < words) to[k] = from[k];
 }
 
-// LOCAL = kLocalSkip when some member has local boundaries: their cells are
-// left to ensemble_local_kernel.
+// LOCAL = kLocalFlat when some member has local boundaries: their inner edges
+// and corners are left to ensemble_local_kernel.
 template <int Q, typename S, int KIND, int LOCAL = kLocalNone>
 __global__ __launch_bounds__(kBlock) void ensemble_step_kernel(const EnsembleEntry<Q>* __restrict__ table,
                                                                const MemberState<Q>* __restrict__ state,
@@ -186,8 +186,7 @@ template <int Q, typename S, int KIND, bool SCRATCH = false>
 __global__ __launch_bounds__(64) void ensemble_post_kernel(const EnsembleEntry<Q>* __restrict__ table,
                                                            const MemberState<Q>* __restrict__ state,
                                                            const uint2* __restrict__ cells, uint32_t count,
-                                                            EnsembleLimits limits,
-                                                           int only, int forced,
+                                                           EnsembleLimits limits, int only, int forced,
                                                            typename StorageTraits<S>::V* scratch = nullptr)
 {
   using V = typename StorageTraits<S>::V;

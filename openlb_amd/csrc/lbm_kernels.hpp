@@ -136,10 +136,11 @@ __device__ __forceinline__ void push_periodic_halo(const StepArgs<Q, V>& a, S* p
   }
 }
 
-// How a pass treats the ids >= 3 that carry local-boundary dynamics: the
-// whole-lattice pass leaves them to a second pass over the list of those
-// cells, so the bulk kernel keeps its register budget (and occupancy).
-enum LocalMode : int { kLocalNone = 0, kLocalSkip = 1, kLocalCollide = 2, kLocalFlat = 3 };
+// How a pass treats the ids >= 3 that carry local-boundary dynamics.  The
+// whole-lattice pass (kLocalFlat) collides flat faces and outer edges and
+// corners, and leaves inner edges and corners to a second pass over the list of
+// those cells (kLocalCollide), so it keeps its register budget (and occupancy).
+enum LocalMode : int { kLocalNone = 0, kLocalCollide = 1, kLocalFlat = 2 };
 
 // Time step of core cell c of one block: collide in place, refresh the
 // periodic overlap.  The caller advances the shifts afterwards.
@@ -162,9 +163,6 @@ __device__ __forceinline__ void collide_stream_cell(const StepArgs<Q, typename S
     // NoDynamics cells are not collided, but on a periodic face their
     // populations still cross into the overlap like every other core cell's
     if (id == 0 && !edge) return;
-    if constexpr (LOCAL == kLocalSkip) {
-      if (id >= 3 && (a.info[id] & 0xffu) != kMovingWall) return;
-    }
     if constexpr (LOCAL == kLocalFlat) {
       // flat faces, and the outer edges and corners (BGK at their fixed
       // velocity), stay in this pass; inner edges and corners go to the list pass

@@ -940,7 +940,7 @@ int lbmh_ensemble_download(lbmh_ensemble* E, int m, void* host, int dtype)
 namespace {
 
 // The member as one block for the checkpoint code; its wall table comes from
-// the device into `walls`.  Call after pull_table.
+// the device into `walls`.  Call after pull_state.
 int member_block(lbmh_ensemble* E, int m, CheckpointBlock& b, std::vector<double>& walls)
 {
   const Member& mem = E->members[m];
