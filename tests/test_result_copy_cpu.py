@@ -32,7 +32,7 @@ static std::vector<unsigned> host_flags;             // of every hipHostMalloc
 static std::vector<std::pair<void*, size_t>> copies;  // destination and size of every transfer
 static std::atomic<int64_t> drained_at{0};            // ns of the steady clock
 static std::map<void*, size_t> registered;            // host memory the runtime knows
-static int device_mallocs = 0;
+static int events = 0;
 
 static int64_t now() { return std::chrono::steady_clock::now().time_since_epoch().count(); }
 
@@ -46,7 +46,6 @@ extern "C" {
 hipError_t hipMalloc(void** p, size_t n)
 {
   std::lock_guard<std::mutex> l(fake);
-  ++device_mallocs;
   if (device_used + n > device_limit) return hipErrorOutOfMemory;
   *p = std::malloc(n);
   device_blocks[*p] = n;
@@ -85,6 +84,23 @@ hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind)
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t)
+{
+  drain();
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
+{
+  *e = reinterpret_cast<hipEvent_t>(&events);
+  ++events;
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t)
+{
+  --events;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t)
 {
   drain();
   return hipSuccess;
@@ -148,7 +164,7 @@ int main() {
   for (auto& b : host_blocks) held += b.second;
   CHECK(held <= (size_t(12) << 20) + 4096 && alive <= 6);  // bounded
   pool.give_back();
-  CHECK(host_blocks.empty() && device_used == 0 && threads() == 1);
+  CHECK(host_blocks.empty() && device_used == 0 && threads() == 1 && events == 0);
   pool.retain();
   CHECK(bring(host, size_t(3) << 20) == LBMH_OK);  // and set up again when needed
   pool.give_back();  // a lattice is still alive
