@@ -519,7 +519,6 @@ __device__ __forceinline__ double wave_max(double v)
 __device__ __forceinline__ void combine_statistics(const double (&acc)[4], double* out)
 {
   __shared__ double lds[4][kBlock / 64];
-  __syncthreads();  // a previous combination has been read
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
@@ -544,16 +543,11 @@ __device__ __forceinline__ void combine_statistics(const double (&acc)[4], doubl
 // latticeStatistics.h:49-71): over the cells whose collision reports a
 // statistic -- bulk cells {rho, |u|^2} (u with the F/2 shift when forced) and
 // moving walls {rho_w, |u_w|^2} (collision.h:343); BounceBack reports none.
-// Partial per workgroup: {count, sum rho, sum |u|^2, max |u|^2}; the workgroup
-// that finishes last combines them in a fixed order into `out`, in coherent host
-// memory, and stores this reading's `number` in `flag` behind it (or into device
-// memory, flag null).  A reading of a small lattice is all latency: a second
-// launch for the partials and a copy of the result took 16 of its 33 us (24^3
-// cavity).  LOCAL: some cell has a local boundary; without, the kernel is a
-// third of the code.
+// Partial per workgroup: {count, sum rho, sum |u|^2, max |u|^2}, combined by
+// statistics_partials_kernel.  LOCAL: some cell has a local boundary; without,
+// the kernel is a third of the code.
 template <int Q, typename S, bool LOCAL>
-__global__ __launch_bounds__(kBlock) void statistics_kernel(double* out, uint64_t* flag, uint64_t number,
-                                                            double* partial, uint32_t* finished, const uint8_t* ids, const S* pop,
+__global__ __launch_bounds__(kBlock) void statistics_kernel(double* partial, const uint8_t* ids, const S* pop,
                                                             CoreGeom g, Shifts<Q> sh, const double* walls,
                                                             const uint32_t* info, double omega,
                                                             double hfx, double hfy, double hfz, int forced,
@@ -605,28 +599,24 @@ __global__ __launch_bounds__(kBlock) void statistics_kernel(double* out, uint64_
     acc[3] = fmax(acc[3], usq);
   }
   combine_statistics(acc, partial + blockIdx.x * 4);
-  // the other workgroups' partials may lie in another XCD's L2: written back
-  // before the count, read after it
-  __shared__ bool last;
-  if (threadIdx.x == 0) {
-    __threadfence();
-    last = __hip_atomic_fetch_add(finished, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x;
-  }
-  __syncthreads();
-  if (!last) return;
-  __threadfence();
+}
+
+// The partials in a fixed order into `out`, in coherent host memory, and this
+// reading's `number` into `flag` behind it, for a host that waits on it (or into
+// device memory, flag null).  The launch boundary is what orders the partials:
+// combined instead by the workgroup that finishes last, each workgroup's fence
+// wrote back its XCD's L2 (24^3 cavity 17.2 us per reading, with this launch
+// 15.7; FP32 100^3 69 and 28 us; FP64 128^3 155 and 63 us).
+static __global__ __launch_bounds__(kBlock) void statistics_partials_kernel(double* out, uint64_t* flag, uint64_t number,
+                                                                            const double* partial, uint32_t nparts)
+{
   double all[4] = {0, 0, 0, 0};
-  for (uint32_t p = threadIdx.x; p < gridDim.x; p += kBlock) {
-    for (int k = 0; k < 3; ++k)
-      all[k] += __hip_atomic_load(partial + p * 4 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    all[3] = fmax(all[3], __hip_atomic_load(partial + p * 4 + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  for (uint32_t p = threadIdx.x; p < nparts; p += kBlock) {
+    for (int k = 0; k < 3; ++k) all[k] += partial[p * 4 + k];
+    all[3] = fmax(all[3], partial[p * 4 + 3]);
   }
   combine_statistics(all, out);
-  if (threadIdx.x == 0) {
-    *finished = 0;  // for the next reading
-    // after the result (written by this thread), for a host that waits on it
-    if (flag) __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  if (threadIdx.x == 0 && flag) __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Second level: one workgroup sums the partials in a fixed order.

@@ -103,7 +103,7 @@ struct lbmh_lattice {
   bool id_defined[kMaxWalls] = {};   // ids given a wall or boundary entry
   uint8_t material_of[kMaxWalls] = {};  // the material (id of lbmh_set_dynamics_ids) each dynamics id stands for
   uint32_t info[kMaxWalls] = {};     // packed LocalInfo per id
-  uint32_t* d_info = nullptr;          // info[], then the count of finished workgroups of a statistics pass
+  uint32_t* d_info = nullptr;
   bool has_local = false;
   // per-cell FORCE of the forced kinds: [3][ncore] on the device in the
   // arithmetic type (double for FP64 storage, float otherwise) and in FP64 on
@@ -1081,10 +1081,8 @@ int lbmh_lattice_create(const lbmh_lattice_desc* desc, lbmh_lattice** out)
   if (e == hipSuccess) e = device_alloc((void**)&L->d_ids, L->ncore);
   if (e == hipSuccess) e = device_alloc((void**)&L->d_walls, sizeof(double) * 4 * kMaxWalls);
   if (e == hipSuccess) e = device_alloc((void**)&L->d_partials, sizeof(double) * 4 * (L->n_partials + 1));
-  if (e == hipSuccess) e = device_alloc((void**)&L->d_info, sizeof(uint32_t) * (kMaxWalls + 1));
-  // the info table, and the count of finished workgroups of a statistics pass
-  const std::vector<uint32_t> info_and_count(kMaxWalls + 1, 0u);
-  if (e == hipSuccess) e = hipMemcpy(L->d_info, info_and_count.data(), sizeof(uint32_t) * (kMaxWalls + 1), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = device_alloc((void**)&L->d_info, sizeof(uint32_t) * kMaxWalls);
+  if (e == hipSuccess) e = hipMemcpy(L->d_info, L->info, sizeof(L->info), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemset(L->d_pop, 0, pop_bytes);
   if (e == hipSuccess) e = hipMemset(L->d_ids, 0, L->ncore);
   if (e == hipSuccess) e = hipMemcpy(L->d_walls, L->walls, sizeof(L->walls), hipMemcpyHostToDevice);
@@ -2131,17 +2129,16 @@ int lbmh_statistics(lbmh_lattice* L, double out[4])
   // behind the result: this reading's number, once it is there
   uint64_t* const flag = pinned ? reinterpret_cast<uint64_t*>(pinned + 8) : nullptr;
   const uint64_t number = buffer.next_number();
-  uint32_t* const finished = L->d_info + kMaxWalls;
   const int rs = settle(L);
   if (rs != LBMH_OK) return rs;
   const int rc = with_types(L, [&](auto qc, auto s) -> int {
     constexpr int Q = decltype(qc)::value;
     using S = decltype(s);
 #define LBMH_STATISTICS(LOCAL_)                                                                                  \
-  hipLaunchKernelGGL((statistics_kernel<Q, S, LOCAL_>), dim3(blocks), dim3(kBlock), 0, 0, result, flag, number,  \
-                     L->d_partials, finished, L->uniform_bulk ? nullptr : L->d_ids, static_cast<const S*>(L->d_pop), g,         \
-                     shifts_of<Q>(L), static_cast<const double*>(L->d_walls), L->d_info, L->params.omega,        \
-                     hf[0] * 0.5, hf[1] * 0.5, hf[2] * 0.5, forced, force_field<S>(L))
+  hipLaunchKernelGGL((statistics_kernel<Q, S, LOCAL_>), dim3(blocks), dim3(kBlock), 0, 0, L->d_partials,          \
+                     L->uniform_bulk ? nullptr : L->d_ids, static_cast<const S*>(L->d_pop), g, shifts_of<Q>(L),   \
+                     static_cast<const double*>(L->d_walls), L->d_info, L->params.omega, hf[0] * 0.5, hf[1] * 0.5, \
+                     hf[2] * 0.5, forced, force_field<S>(L))
     if (L->has_local) LBMH_STATISTICS(true);
     else LBMH_STATISTICS(false);
 #undef LBMH_STATISTICS
@@ -2149,6 +2146,8 @@ int lbmh_statistics(lbmh_lattice* L, double out[4])
     return LBMH_OK;
   });
   if (rc != LBMH_OK) return rc;
+  hipLaunchKernelGGL(statistics_partials_kernel, dim3(1), dim3(kBlock), 0, 0, result, flag, number, L->d_partials, blocks);
+  LBMH_HIP(hipGetLastError());
   double acc[4];
   if (pinned) {
     // a short reading is seen sooner in memory than through the stream's signal

@@ -132,7 +132,7 @@ def test_empty_selection_and_errors(gpu_available):
 @pytest.mark.parametrize("storage", ["f64", "f32"])
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 16, 1), (257, 1, 1), (9, 8, 64), (70, 64, 65)])
 def test_statistics_combine_every_workgroup_once(gpu_available, shape, storage):
-    """The workgroup that finishes last combines the others' partials: one
+    """A second launch combines the workgroups' partials: one
     workgroup, one full, one and a rest, eighteen, and more cells than the 1024
     workgroups hold at once; readings repeated without a step between agree bit
     for bit.  Against numpy over the FP64 moments: sums of n terms of size one
