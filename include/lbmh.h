@@ -190,10 +190,10 @@ int lbmh_halo_copy_many(lbmh_halo* const* halos, size_t n, void* stream);
  * together with every block their halos join them to, run the collision, the
  * copies and the edge and corner processors in one launch each; cells that
  * collide from a list (inner edges and corners) and plane processors take a
- * launch per block, and so does everything for other blocks.  The tables of the
- * call are built in it, sent from the host and kept by the first block: calls
- * led by one block must run on one stream, and a stream that is being captured
- * is refused (LBMH_E_STATE). */
+ * launch per block, and so does everything for other blocks.  The first block
+ * keeps the tables, which are sent from the host where something in them has
+ * changed since its last call: calls led by one block must run on one stream,
+ * and a stream that is being captured is refused (LBMH_E_STATE). */
 int lbmh_split_step(lbmh_lattice* const* lattices, size_t n_lattices, lbmh_halo* const* halos, size_t n_halos,
                     int64_t n_steps, void* stream);
 

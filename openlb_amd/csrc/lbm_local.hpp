@@ -461,6 +461,7 @@ struct PostArgs {
   // momenta/elements.h:1473-1488): the per-cell FORCE [3][ncore] in the
   // arithmetic type, or null and the uniform F/2
   uint32_t forced;
+  uint32_t pad_ = 0;        // no unnamed bytes: tables of these are compared whole
   const void* force;
   double half_force[3];
   uint32_t count;
@@ -468,6 +469,7 @@ struct PostArgs {
   uint32_t sx, sy;
   uint32_t periodic;
   FastDiv div_z, div_y;
+  uint32_t pad2_ = 0;
   double omega;
 };
 

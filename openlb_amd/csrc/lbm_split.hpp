@@ -35,6 +35,7 @@ struct SplitHalo {
   uint32_t dst_n, src_n;
   uint32_t dst_block, src_block;
   uint32_t count;
+  uint32_t pad_ = 0;  // here and below: no unnamed bytes, the tables are compared whole
 };
 
 // The copies of halo_copy_kernel before the streaming: `state` is the copy the
@@ -59,6 +60,7 @@ template <int Q>
 struct SplitPost {
   PostArgs<Q> a;
   uint32_t block;
+  uint32_t pad_ = 0;
 };
 
 template <int Q>
@@ -89,6 +91,7 @@ struct SplitRemote {
   const RemotePair* pairs;
   void* out;
   uint32_t count;
+  uint32_t pad_ = 0;
 };
 
 template <int Q, typename S>

@@ -567,3 +567,55 @@ def test_evaluations_wait_for_work_on_another_stream(gpu_available, route):
     assert hip.hipStreamDestroy(stream) == 0
     for a, b in zip(*results):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("case,blocks", [("cavity_local", (2, 2, 2)), ("duct", (3, 1, 1)), ("forced", (2, 1, 2))])
+def test_split_step_follows_changes_between_calls(gpu_available, case, blocks):
+    """Tables and states that the device has from the last call are not sent
+    again: whatever a program changes between calls must reach the next one.
+    Odd and even calls with, between them, nothing, new parameters, wall values,
+    FORCE, single phases, new populations, a checkpoint and a new boundary."""
+    case = {"cavity_local": lambda: W.local_velocity_cavity((12, 13, 14), tau=0.7, lid_u=0.06),
+            "duct": lambda: W.velocity_channel((14, 12, 11), u_in=0.04),
+            "forced": lambda: W.kolmogorov_flow((12, 13, 11), walls=True)}[case]()
+    rng = np.random.Generator(np.random.PCG64(3))
+    field = 1e-5 * rng.standard_normal((3,) + tuple(case.shape))
+    out = []
+    for run in (_split, _phases):
+        with SuperLattice(case, "f32", blocks) as sup:
+            sup.ini_equilibrium(case.rho_u)
+            sup.initialize()
+            lats = list(sup.blocks.values())
+            saved = []
+
+            def parameters():
+                lats[-1].set_parameters(omega=1.3, force=case.force)
+
+            def walls():
+                free = max(case.walls, default=2) if not case.local else None
+                if free in case.walls:
+                    lats[0].set_wall(free, 1.0, (0.01, 0.0, 0.02))
+
+            def force():
+                if case.kind != "bgk":
+                    sup._scatter(field, lambda lat, part: lat.set_force_field(part))
+
+            def boundary():
+                # the ids again, then the case's own boundaries with another velocity
+                for lat, key in zip(lats, sup.blocks):
+                    lo = sup.origin[key]
+                    ids = case.ids[tuple(slice(lo[d], lo[d] + lat.shape[d]) for d in range(3))]
+                    if not case.local:
+                        lat.define_dynamics(ids)
+                        for wid, (rho, u) in case.walls.items():
+                            lat.set_wall(wid, rho, u)
+
+            for change, steps in ((None, 1), (None, 2), (None, 1), (parameters, 3), (walls, 1), (force, 2),
+                                  (lambda: _phases(sup, 1), 1), (lambda: saved.append(sup.checkpoint("f32")), 1),
+                                  (lambda: sup.ini_equilibrium(case.rho_u), 2), (lambda: sup.restore(saved[0], "f32"), 1),
+                                  (boundary, 3), (None, 1)):
+                if change:
+                    change()
+                run(sup, steps)
+            out.append([lat.checkpoint("f32") for lat in lats])
+    assert out[0] == out[1]
