@@ -47,9 +47,9 @@ constexpr size_t kCopyChunk = size_t(2) << 20;     // bytes of one transfer
 constexpr int kCopyThreads = 6;                    // slots; the caller and its helpers
 constexpr size_t kCopyDirect = size_t(64) << 10;   // up to here hipMemcpy's own path is as fast
 // From here on the helpers pay for their wake-up also where the caller's pages
-// are there already: 432 KB take 42 us without and 50 with them, 843 KB 61 and
-// 58.  (Into pages mapped anew 432 KB take 121 and 90 us.)
-constexpr size_t kCopyHelped = size_t(640) << 10;
+// are there already: 432 KB take 42 us without and 50 with them, 750 KB 69 and
+// 76, 1 MB 79 and 70.  (Into pages mapped anew 432 KB take 121 and 90 us.)
+constexpr size_t kCopyHelped = size_t(896) << 10;
 constexpr size_t kWorkspaceLimit = size_t(64) << 20;
 constexpr size_t kReadingBytes = 128;  // the values, and from byte 64 on the reading's number
 
