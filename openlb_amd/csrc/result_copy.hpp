@@ -5,11 +5,11 @@
 // density and velocity of a 256^3 block: 27.6 ms): one thread copies out of the
 // runtime's staging memory and takes the page faults of a fresh array, 8-13 GB/s
 // where the link gives 52 GB/s.  Here helper threads copy chunks through a
-// pinned buffer (9.1 ms), so that transfers, host copies and page faults
-// overlap.  A small export (the 96 members of a study, 1 MB each) paid for a
-// hipMalloc and a hipFree and then for 256 page faults in a row, 230 us each:
-// it now takes one transfer, during which the helpers touch the caller's pages,
-// and 125 us.
+// pinned buffer, so that transfers, host copies and page faults overlap: 9.1 ms
+// into arrays the program has used before, 12 to 16 ms, by the host, where it
+// takes new ones from the system each time.  Smaller results take one transfer,
+// during which the caller's pages are touched, by the helpers or by the caller,
+// and a workspace that stays allocated.
 //
 // A reading of a few words (lbmh_statistics) has pinned memory of its own, which
 // a running kernel writes and the host polls.
@@ -47,8 +47,9 @@ constexpr size_t kCopyChunk = size_t(2) << 20;     // bytes of one transfer
 constexpr int kCopyThreads = 6;                    // slots; the caller and its helpers
 constexpr size_t kCopyDirect = size_t(64) << 10;   // up to here hipMemcpy's own path is as fast
 // From here on the helpers pay for their wake-up also where the caller's pages
-// are there already: 432 KB take 42 us without and 50 with them, 750 KB 69 and
-// 76, 1 MB 79 and 70.  (Into pages mapped anew 432 KB take 121 and 90 us.)
+// are there already: 432 KB take 41 us without and 54 with them, 750 KB 69 and
+// 76, 1 MB 79 and 68.  Below, the caller touches its pages itself while it would
+// only wait for the transfer (432 KB into pages mapped anew: 122 -> 77 us).
 constexpr size_t kCopyHelped = size_t(896) << 10;
 constexpr size_t kWorkspaceLimit = size_t(64) << 20;
 constexpr size_t kReadingBytes = 128;  // the values, and from byte 64 on the reading's number
@@ -125,42 +126,38 @@ class CopyHelpers {
 };
 
 // What the helpers wait for while the steps queued before a result run: they
-// spin for a few ms, and sleep through a longer wait until it is about to end.
-// Sleep costs the caller 15 to 50 us (48^3 D3Q27, 300 steps and FP64 moments
-// 2357 us, with a spin of 500 us 2372; 129 steps of 170x267x97 and the density
-// 16.08 and 16.13 ms), so only waits it does not show in are slept through.
+// spin for a few ms and then sleep.  Waking them takes 25 to 200 us of the
+// caller's time, so only waits it does not show in are slept through (48^3 D3Q27,
+// 300 steps and FP64 moments: 2357 us, with a spin of 200 us 2385).  An event
+// before the result's kernel, to wake them in time, took 5 to 10 us itself.
 class Gate {
  public:
-  enum State : int { kFailed = -1, kQueued, kSoon, kOpen };
-
-  void set(State s)
+  void set(bool good)
   {
     {
       std::lock_guard<std::mutex> l(mutex_);
-      state_ = s;
+      state_ = good ? 1 : -1;
     }
     changed_.notify_all();
   }
 
-  bool decided() const { return state_ == kOpen || state_ == kFailed; }
+  bool decided() const { return state_ != 0; }
 
   bool wait()
   {
-    for (;;) {
-      const auto until = std::chrono::steady_clock::now() + kSpin;
-      int seen = state_;
-      while ((seen = state_, !decided()) && std::chrono::steady_clock::now() < until) std::this_thread::yield();
-      if (decided()) return state_ == kOpen;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(5);
+    while (!decided() && std::chrono::steady_clock::now() < until) std::this_thread::yield();
+    if (!decided()) {
       std::unique_lock<std::mutex> l(mutex_);
-      changed_.wait(l, [&] { return state_ != seen; });
+      changed_.wait(l, [this] { return decided(); });
     }
+    return state_ > 0;
   }
 
  private:
-  static constexpr auto kSpin = std::chrono::milliseconds(3);
   std::mutex mutex_;
   std::condition_variable changed_;
-  std::atomic<int> state_{kQueued};
+  std::atomic<int> state_{0};
 };
 
 // The pages of n bytes of the caller's memory, which the result overwrites.
@@ -178,8 +175,6 @@ struct ResultPool {
   void* device = nullptr;
   size_t device_bytes = 0;
   int ordinal = -1;        // device the workspace lies on
-  hipEvent_t point = nullptr;
-  int point_ordinal = -1;
   void* reading = nullptr; // pinned and coherent, kReadingBytes
   uint64_t number = 0;     // under the lease: readings so far
   CopyHelpers helpers;
@@ -214,29 +209,7 @@ struct ResultPool {
     pinned = nullptr;
     if (reading) (void)hipHostFree(reading);
     reading = nullptr;
-    drop_event();
     drop_workspace();
-  }
-
-  // For the point in the null stream of device `on` where a result's own work
-  // begins, under the lease; null if there is none to be had.
-  hipEvent_t event(int on)
-  {
-    if (point && point_ordinal != on) drop_event();
-    if (!point && hipEventCreateWithFlags(&point, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      point = nullptr;
-    }
-    point_ordinal = on;
-    return point;
-  }
-
-  void drop_event()
-  {
-    if (!point) return;
-    DeviceGuard guard(point_ordinal);
-    (void)hipEventDestroy(point);
-    point = nullptr;
   }
 
   void drop_workspace()
@@ -275,15 +248,10 @@ class ResultBuffer {
   ResultBuffer(const ResultBuffer&) = delete;
   ResultBuffer& operator=(const ResultBuffer&) = delete;
 
-  // `bytes` on the current device `ordinal`, before the work that fills them is
-  // launched on the null stream
+  // `bytes` on the current device `ordinal`
   int allocate(int ordinal, size_t bytes)
   {
     ordinal_ = ordinal;
-    if (lock_.owns_lock() && bytes >= kCopyHelped) {
-      begin_ = ResultPool::get().event(ordinal);
-      if (begin_) LBMH_HIP(hipEventRecord(begin_, nullptr));
-    }
     ResultPool& pool = ResultPool::get();
     if (lock_.owns_lock() && bytes <= kWorkspaceLimit) {
       if (pool.ordinal != ordinal || pool.device_bytes < bytes) {
@@ -366,7 +334,9 @@ class ResultBuffer {
       // pages, and copy it when the transfer is done
       char* const stage = static_cast<char*>(pool.pinned);
       if (bytes < kCopyHelped) {
-        LBMH_HIP(hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost));
+        LBMH_HIP(hipMemcpyAsync(stage, p, bytes, hipMemcpyDeviceToHost, nullptr));
+        touch(to, bytes);
+        LBMH_HIP(hipStreamSynchronize(nullptr));
         std::memcpy(to, stage, bytes);
         return LBMH_OK;
       }
@@ -376,11 +346,9 @@ class ResultBuffer {
       std::atomic<size_t> next{0};
       pool.helpers.run([&](int slot) {
         if (slot == 0) {
-          hipError_t e = wait_for_steps();
-          arrived.set(Gate::kSoon);
-          if (e == hipSuccess) e = hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost);
+          const hipError_t e = hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost);
           if (e != hipSuccess) error = e;
-          arrived.set(e == hipSuccess ? Gate::kOpen : Gate::kFailed);
+          arrived.set(e == hipSuccess);
         }
         for (;;) {
           const size_t at = next.fetch_add(part);
@@ -393,14 +361,14 @@ class ResultBuffer {
       });
     } else {
       // a transfer waits in a busy loop for the work queued before it: one thread
-      // waits for the steps, while the others touch the pages of their first chunk
+      // does, while the others touch the pages of their first chunk
       Gate drained;
       std::atomic<size_t> next{0};
       pool.helpers.run([&](int slot) {
         if (slot == 0) {
-          const hipError_t e = wait_for_steps();
+          const hipError_t e = hipStreamSynchronize(nullptr);
           if (e != hipSuccess) error = e;
-          drained.set(e == hipSuccess ? Gate::kOpen : Gate::kFailed);
+          drained.set(e == hipSuccess);
         }
         const hipError_t d = hipSetDevice(ordinal_);
         if (d != hipSuccess) error = d;
@@ -424,10 +392,6 @@ class ResultBuffer {
   void* p = nullptr;
 
  private:
-  // The helpers sleep through the steps queued before this result and are woken
-  // when its own kernel starts, so that they are awake when the data comes.
-  hipError_t wait_for_steps() { return begin_ ? hipEventSynchronize(begin_) : hipSuccess; }
-
   static bool known_to_runtime(const void* host)
   {
     hipPointerAttribute_t a{};
@@ -438,7 +402,6 @@ class ResultBuffer {
 
   std::unique_lock<std::mutex> lock_;
   void* own_ = nullptr;
-  hipEvent_t begin_ = nullptr;  // the pool's
   int ordinal_ = 0;
 };
 

@@ -32,7 +32,7 @@ static std::vector<unsigned> host_flags;             // of every hipHostMalloc
 static std::vector<std::pair<void*, size_t>> copies;  // destination and size of every transfer
 static std::atomic<int64_t> drained_at{0};            // ns of the steady clock
 static std::map<void*, size_t> registered;            // host memory the runtime knows
-static int events = 0;
+static std::vector<std::function<void()>> queued;     // transfers not waited for yet
 
 static int64_t now() { return std::chrono::steady_clock::now().time_since_epoch().count(); }
 
@@ -86,23 +86,18 @@ hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind)
 hipError_t hipStreamSynchronize(hipStream_t)
 {
   drain();
+  std::lock_guard<std::mutex> l(fake);
+  for (auto& f : queued) f();
+  queued.clear();
   return hipSuccess;
 }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
+hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind, hipStream_t)
 {
-  *e = reinterpret_cast<hipEvent_t>(&events);
-  ++events;
-  return hipSuccess;
-}
-hipError_t hipEventDestroy(hipEvent_t)
-{
-  --events;
-  return hipSuccess;
-}
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t)
-{
-  drain();
+  std::lock_guard<std::mutex> l(fake);
+  queued.push_back([=] {
+    std::memcpy(to, from, n);
+    copies.push_back({to, n});
+  });
   return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
@@ -164,7 +159,7 @@ int main() {
   for (auto& b : host_blocks) held += b.second;
   CHECK(held <= (size_t(12) << 20) + 4096 && alive <= 6);  // bounded
   pool.give_back();
-  CHECK(host_blocks.empty() && device_used == 0 && threads() == 1 && events == 0);
+  CHECK(host_blocks.empty() && device_used == 0 && threads() == 1);
   pool.retain();
   CHECK(bring(host, size_t(3) << 20) == LBMH_OK);  // and set up again when needed
   pool.give_back();  // a lattice is still alive
