@@ -160,9 +160,8 @@ struct lbmh_lattice {
 // FP16 no cap (D3Q27 384x192x192 341 us against 380 us).  Wide XCD groups keep the
 // lines that neighbouring chunks share in one L2 (FP64 D3Q27 384x192x192, group 8
 // -> 16: 1285 -> 1189 us; FP16 the same block, 8 -> 32: 346 -> 341 us; FP32
-// 4 -> 32: 128^3 54.3 -> 52.8 us, D3Q19 192^3 (538 MB) 184.5 -> 180, 320^3 (2.5 GB)
-// 941 -> 926, 64x512x300 267 -> 260, D3Q27 200^3 321 -> 315, porous 256^3 471.4 ->
-// 470.8; two lose: a 230^3 cavity 332 -> 337, turbulent 256x160x160 263 -> 264.8).
+// 128^3, 4 -> 32: 54.3 -> 52.8 us); an FP32 block above 512 MB is faster with
+// groups of 4 (256^3 466 us against 470 us).
 // With local boundaries the whole-lattice pass collides the flat faces too, and
 // its divergent waves need the occupancy: no cap (201^3 cavity, FP32: 298 us
 // against 324 us).
@@ -177,7 +176,7 @@ static lbmh_launch_config default_launch(const lbmh_lattice* L, bool local)
   }
   if (L->storage == LBMH_F16) return lbmh_launch_config{0, 32};
   if (L->storage == LBMH_F64) return lbmh_launch_config{49152, 16};
-  return lbmh_launch_config{40960, 32};
+  return lbmh_launch_config{40960, bytes < 512 * kMB ? 32 : 4};
 }
 
 struct lbmh_halo {
