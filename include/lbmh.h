@@ -432,8 +432,9 @@ int lbmh_release_buffers(void);
  * the chunks in opposite directions, each chunk on the same XCD.  Defaults
  * follow the storage type and the size of the block: blocks up to 64 MB of
  * populations lds_bytes 0 and one eighth of the chunks per XCD (up to 64),
- * larger ones lds_bytes 40960 and xcd_group 32 (4 above 512 MB) in FP32,
- * 49152 and 16 in FP64, 0 and 32 in FP16; lattices with local velocity /
+ * larger ones lds_bytes 40960 and xcd_group 32 in FP32 (above 512 MB 4, unless
+ * every cell is a bulk cell), 49152 and 16 in FP64, 0 and 32 in FP16; lattices
+ * with local velocity /
  * pressure boundaries take lds_bytes 0 and xcd_group 4 (FP16: 8), as their
  * whole-lattice pass also collides the flat faces, whose divergent waves need
  * the occupancy.  A

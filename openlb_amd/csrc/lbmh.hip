@@ -160,8 +160,12 @@ struct lbmh_lattice {
 // FP16 no cap (D3Q27 384x192x192 341 us against 380 us).  Wide XCD groups keep the
 // lines that neighbouring chunks share in one L2 (FP64 D3Q27 384x192x192, group 8
 // -> 16: 1285 -> 1189 us; FP16 the same block, 8 -> 32: 346 -> 341 us; FP32
-// 128^3, 4 -> 32: 54.3 -> 52.8 us); an FP32 block above 512 MB is faster with
-// groups of 4 (256^3 466 us against 470 us).
+// 128^3, 4 -> 32: 54.3 -> 52.8 us).  FP32 above 512 MB, groups of 4 and of 32, each
+// block in turn: boxes of bulk cells alone gain (192^3 184.5 -> 180 us, 240^3 384
+// -> 376, 320^3 941 -> 926, 203x231x157 196 -> 190, 64x512x300 267 -> 260, D3Q27
+// 200^3 321 -> 315); blocks that read ids lose or stay (porous 256^3 482.5 -> 487 in
+// its first 25 steps, later 470 -> 472, 230^3 cavity 332 -> 337, turbulent
+// 256x160x160 263.1 -> 264.8, porous 200^3 214 -> 210.7).
 // With local boundaries the whole-lattice pass collides the flat faces too, and
 // its divergent waves need the occupancy: no cap (201^3 cavity, FP32: 298 us
 // against 324 us).
@@ -176,7 +180,7 @@ static lbmh_launch_config default_launch(const lbmh_lattice* L, bool local)
   }
   if (L->storage == LBMH_F16) return lbmh_launch_config{0, 32};
   if (L->storage == LBMH_F64) return lbmh_launch_config{49152, 16};
-  return lbmh_launch_config{40960, bytes < 512 * kMB ? 32 : 4};
+  return lbmh_launch_config{40960, bytes < 512 * kMB || L->uniform_bulk ? 32 : 4};
 }
 
 struct lbmh_halo {
