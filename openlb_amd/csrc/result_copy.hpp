@@ -5,11 +5,11 @@
 // density and velocity of a 256^3 block: 27.6 ms): one thread copies out of the
 // runtime's staging memory and takes the page faults of a fresh array, 8-13 GB/s
 // where the link gives 52 GB/s.  Here helper threads copy chunks through a
-// pinned buffer, so that transfers, host copies and page faults overlap: 9.1 ms
-// into arrays the program has used before, 12 to 16 ms, by the host, where it
-// takes new ones from the system each time.  Smaller results take one transfer,
-// during which the caller's pages are touched, by the helpers or by the caller,
-// and a workspace that stays allocated.
+// pinned buffer, so that transfers, host copies and page faults overlap: 8.3 ms
+// into memory the program has used before with the HIP runtime that torch
+// brings, 14.9 ms with ROCm 7.2's own (hipMemcpy alone 17.6 and 22.5).  Smaller
+// results take one transfer, during which the caller's pages are touched, by the
+// helpers or by the caller, and a workspace that stays allocated.
 //
 // A reading of a few words (lbmh_statistics) has pinned memory of its own, which
 // a running kernel writes and the host polls.
