@@ -191,31 +191,24 @@ int with_types(const lbmh_ensemble* E, F&& f)
   return with_types(E->q, E->storage, std::forward<F>(f));
 }
 
-// Bytes of a read of the states: copies of up to 16 KB to pageable memory go a
-// slower way (112 bytes 12 us, 7 KB 15, 16 KB 18, and 17 KB 9), so that reads are
-// never smaller.  The device's allocation ends in as many spare bytes.
-constexpr size_t kPullBytes = (size_t(16) << 10) + 256;
-
-int pull(unsigned char* to, const char* from, size_t bytes)
+// The members' states as the device holds them; the table only changes here on
+// the host.  (Copies above 16 KB take another way through the runtime: repeated
+// on their own 9 us against 12 to 18 below, but 80 to 120 us between kernels and
+// other copies, 18 to 28 below, so reads are not made larger than they need be.)
+int pull_state(lbmh_ensemble* E)
 {
   LBMH_HIP(hipDeviceSynchronize());
-  if (bytes >= kPullBytes) {
-    LBMH_HIP(hipMemcpy(to, from, bytes, hipMemcpyDeviceToHost));
-    return LBMH_OK;
-  }
-  unsigned char all[kPullBytes];
-  LBMH_HIP(hipMemcpy(all, from, kPullBytes, hipMemcpyDeviceToHost));
-  std::memcpy(to, all, bytes);
+  LBMH_HIP(hipMemcpy(E->h_state.data(), device_state(E, 0), E->h_state.size(), hipMemcpyDeviceToHost));
   return LBMH_OK;
 }
-
-// The members' states as the device holds them; the table only changes here on the host.
-int pull_state(lbmh_ensemble* E) { return pull(E->h_state.data(), device_state(E, 0), E->h_state.size()); }
 
 // The state of member m alone.
 int pull_state(lbmh_ensemble* E, int m)
 {
-  return pull(E->h_state.data() + size_t(m) * E->state_bytes, device_state(E, 0, m), E->state_bytes);
+  LBMH_HIP(hipDeviceSynchronize());
+  LBMH_HIP(hipMemcpy(E->h_state.data() + size_t(m) * E->state_bytes, device_state(E, 0, m), E->state_bytes,
+                     hipMemcpyDeviceToHost));
+  return LBMH_OK;
 }
 
 // Assign chunk ranges to active members in slot order and upload table + map.
@@ -497,7 +490,7 @@ int lbmh_ensemble_create(const lbmh_ensemble_desc* d, lbmh_ensemble** out)
   hipError_t e = device_alloc(&E->d_pop, E->pop_arena.capacity());
   if (e == hipSuccess) e = device_alloc((void**)&E->d_ids, E->id_arena.capacity());
   if (e == hipSuccess) e = device_alloc((void**)&E->d_walls, sizeof(double) * 4 * kEnsembleWalls * E->max_members);
-  const size_t state_at = align_up(E->h_table.size()), table_bytes = state_at + 2 * E->h_state.size() + kPullBytes;
+  const size_t state_at = align_up(E->h_table.size()), table_bytes = state_at + 2 * E->h_state.size();
   if (e == hipSuccess) e = device_alloc(&E->d_table, table_bytes);
   E->d_state = static_cast<char*>(E->d_table) + state_at;
   if (e == hipSuccess) e = device_alloc((void**)&E->d_chunk, sizeof(uint32_t) * E->chunk_capacity);
