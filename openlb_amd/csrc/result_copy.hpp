@@ -8,8 +8,8 @@
 // pinned buffer, so that transfers, host copies and page faults overlap: 8.3 ms
 // into memory the program has used before with the HIP runtime that torch
 // brings, 14.9 ms with ROCm 7.2's own (hipMemcpy alone 17.6 and 22.5).  Smaller
-// results take one transfer, during which the caller's pages are touched, by the
-// helpers or by the caller, and a workspace that stays allocated.
+// results take one transfer, during which the helpers touch the caller's pages,
+// and a workspace that stays allocated.
 //
 // A reading of a few words (lbmh_statistics) has pinned memory of its own, which
 // a running kernel writes and the host polls.
@@ -46,11 +46,10 @@ namespace lbmh {
 constexpr size_t kCopyChunk = size_t(2) << 20;     // bytes of one transfer
 constexpr int kCopyThreads = 6;                    // slots; the caller and its helpers
 constexpr size_t kCopyDirect = size_t(64) << 10;   // up to here hipMemcpy's own path is as fast
-// From here on the helpers pay for their wake-up also where the caller's pages
-// are there already: 432 KB take 41 us without and 54 with them, 750 KB 69 and
-// 76, 1 MB 79 and 68.  Below, the caller touches its pages itself while it would
-// only wait for the transfer (432 KB into pages mapped anew: 122 -> 77 us).
-constexpr size_t kCopyHelped = size_t(896) << 10;
+// From here on the helpers pay for their wake-up: 432 KB into memory in use take
+// 42 us without and 54 with them, 549 KB 49 and 53, 1 MB 79 and 68; the velocities
+// of a split cavity's eight pieces, 890 KB each, 980 and 870 us.
+constexpr size_t kCopyHelped = size_t(448) << 10;
 constexpr size_t kWorkspaceLimit = size_t(64) << 20;
 constexpr size_t kReadingBytes = 128;  // the values, and from byte 64 on the reading's number
 
@@ -334,9 +333,9 @@ class ResultBuffer {
       // pages, and copy it when the transfer is done
       char* const stage = static_cast<char*>(pool.pinned);
       if (bytes < kCopyHelped) {
-        LBMH_HIP(hipMemcpyAsync(stage, p, bytes, hipMemcpyDeviceToHost, nullptr));
-        touch(to, bytes);
-        LBMH_HIP(hipStreamSynchronize(nullptr));
+        // (hipMemcpyAsync, the pages touched meanwhile and a wait for the stream:
+        // 15 us more for 166 KB with the runtime that torch brings)
+        LBMH_HIP(hipMemcpy(stage, p, bytes, hipMemcpyDeviceToHost));
         std::memcpy(to, stage, bytes);
         return LBMH_OK;
       }

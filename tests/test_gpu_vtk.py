@@ -147,7 +147,7 @@ def test_export_argument_errors(gpu_available):
 @pytest.mark.parametrize("shape", [(1, 1, 1), (16, 32, 32), (30, 30, 25), (64, 64, 63), (96, 120, 130)])
 def test_exports_of_every_size_reach_the_host_whole(gpu_available, shape):
     """The way to the host depends on the size: hipMemcpy up to 64 KB, one
-    pinned transfer, a transfer shared by helper threads from 896 KB, chunks of
+    pinned transfer, a transfer shared by helper threads from 448 KB, chunks of
     2 MB from 12 MB; FP64 moments, float32 fields and populations of a lattice
     and of an ensemble member of the same state agree at every size, also
     from two threads at once."""

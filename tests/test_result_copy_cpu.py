@@ -32,7 +32,6 @@ static std::vector<unsigned> host_flags;             // of every hipHostMalloc
 static std::vector<std::pair<void*, size_t>> copies;  // destination and size of every transfer
 static std::atomic<int64_t> drained_at{0};            // ns of the steady clock
 static std::map<void*, size_t> registered;            // host memory the runtime knows
-static std::vector<std::function<void()>> queued;     // transfers not waited for yet
 
 static int64_t now() { return std::chrono::steady_clock::now().time_since_epoch().count(); }
 
@@ -86,18 +85,6 @@ hipError_t hipMemcpy(void* to, const void* from, size_t n, hipMemcpyKind)
 hipError_t hipStreamSynchronize(hipStream_t)
 {
   drain();
-  std::lock_guard<std::mutex> l(fake);
-  for (auto& f : queued) f();
-  queued.clear();
-  return hipSuccess;
-}
-hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind, hipStream_t)
-{
-  std::lock_guard<std::mutex> l(fake);
-  queued.push_back([=] {
-    std::memcpy(to, from, n);
-    copies.push_back({to, n});
-  });
   return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
@@ -224,7 +211,7 @@ SMALL = r"""
 int main() {
   ResultPool::get().retain();
   std::vector<unsigned char> host;
-  for (size_t n : {size_t(2000), kCopyDirect, kCopyDirect + 1, size_t(432) << 10, kCopyHelped - 1}) CHECK(bring(host, n) == LBMH_OK);
+  for (size_t n : {size_t(2000), kCopyDirect, kCopyDirect + 1, size_t(300) << 10, kCopyHelped - 1}) CHECK(bring(host, n) == LBMH_OK);
   CHECK(threads() == 1);
   CHECK(bring(host, kCopyHelped) == LBMH_OK && threads() == 6);
 """
